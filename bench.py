@@ -422,7 +422,7 @@ def published_walkthroughs():
     ms, st = best(lambda: FVM.solve(plate_fvm, FVM.TRBDF2(), saveat=0.05), stats=True)
     out.append(dict(workload="the plate as an FVMProblem, TRBDF2 (ours: the affine problem's Jacobian from "
                              "coloured fvm_jvp probes, then the whole integration with Newton-GMRES in one "
-                             "workgroup; published: KLU on the sparse Jacobian), saveat 0.05",
+                             "launch; published: KLU on the sparse Jacobian), saveat 0.05",
                     ms=ms, first_solve_ms=first(make_plate, 0.05), published_ms=49.237, stats=st,
                     note="ms: repeated solves of one problem (the extracted Jacobian is kept on it); "
                          "first_solve_ms: a fresh problem, its device set-up and Jacobian extraction included",
@@ -448,7 +448,7 @@ def published_walkthroughs():
                               final_time=500.0)
 
     ms, st = best(lambda: FVM.solve(big_fvm, FVM.TRBDF2(), saveat=100.0), stats=True)
-    out.append(dict(workload="the same as an FVMProblem, stiff (ours: TRBDF2 in one workgroup as above; "
+    out.append(dict(workload="the same as an FVMProblem, stiff (ours: TRBDF2 in one launch as above; "
                              "published: CVODE_BDF with GMRES), saveat 100",
                     ms=ms, first_solve_ms=first(make_big, 100.0), published_ms=94.839, stats=st,
                     source="docs/src/literate_wyos/diffusion_equations.jl:451-455"))
@@ -596,7 +596,7 @@ def published_walkthroughs():
 
     lrd_fvm = make_lrd()
     ms, st = best(lambda: FVM.solve(lrd_fvm, FVM.TRBDF2(), saveat=2.0), stats=True)
-    out.append(dict(workload="the same as an FVMProblem, stiff (ours: TRBDF2 in one workgroup; published: "
+    out.append(dict(workload="the same as an FVMProblem, stiff (ours: TRBDF2 in one launch; published: "
                              "CVODE_BDF with GMRES), saveat 2", ms=ms, first_solve_ms=first(make_lrd, 2.0),
                     published_ms=163.686, stats=st,
                     source="docs/src/literate_wyos/linear_reaction_diffusion_equations.jl:180-186"))

@@ -4,46 +4,238 @@
 // factorisation of the sparse Jacobian (solve.jl:167-183, jacobian_sparsity
 // solve.jl:50-77).  When f(u) = J u + c (linear fluxes, sources affine in u,
 // conditions constant in t), J is constant: the host package extracts it once
-// from fvm_jvp probes over a colouring of jacobian_sparsity's pattern, and this
-// kernel runs the whole integration in one workgroup of 1024 threads: both stages'
-// Newton iterations with restarted GMRES(m) on W = I - d h J (classical
-// Gram-Schmidt applied twice, the Hessenberg least squares by Givens rotations),
-// the W^-1-filtered error estimate, the step controller, the Dirichlet update and
-// the saveat interpolation, with barriers between phases and no host round trip.
-// A problem of a few thousand nodes is bound by kernel launches and host
-// synchronisations otherwise (about a dozen launches and a synchronisation per
-// Krylov iteration).  The algorithm is the host integrator's (solve.py), step for
-// step; reductions here sum in a different order, so results agree with it to the
-// Krylov and Newton tolerances, not bit for bit.
+// from fvm_jvp probes over a colouring of jacobian_sparsity's pattern, and
+// trbdf2_affine_kernel runs the whole integration: both stages' Newton iterations
+// with restarted GMRES(m) on W = I - d h J (the Hessenberg least squares by Givens
+// rotations), the W^-1-filtered error estimate, the step controller, the Dirichlet
+// update and the saveat interpolation, with no host round trip.
+//
+// Layout: one row per thread, one workgroup per CU, the workgroups resident together
+// (cooperative launch).  Every vector of the integration is a register of its row's
+// thread, the matrix row too, and the Krylov basis of a workgroup's rows lies in its
+// LDS; a product publishes one vector to the grid and a Gram-Schmidt pass is one
+// grid-wide sum (fvm_grid.hpp), so a Krylov step costs two exchanges of 1.5 to 2 us
+// and about as much arithmetic, whatever n.  What bounds it is that latency: 6.0 ms for
+// 805 Krylov steps and 139 Newton iterations on 10,000 rows, where the same loop in
+// one workgroup of 1024 threads, its vectors in memory, took 55.5 ms (one CU's rate
+// out of L2).
+// The algorithm is the host integrator's (solve.py), step for step; reductions here
+// sum in a different order, so results agree with it to the Krylov and Newton
+// tolerances, not bit for bit.
 #include <cmath>
 
-#include "fvm_internal.hpp"
+#include "fvm_grid.hpp"
 
 namespace {
 
-constexpr int kT = 1024;       // threads of the one workgroup
-constexpr int kWaves = kT / 64;
+using fvm::Grid;
+using fvm::GridShared;
+
 constexpr int kMaxRestart = 30;
-constexpr int kChunk = 8;      // dot products reduced together
 constexpr int64_t kMaxN = 65536;
+// Rows per workgroup: 256 up to 64 workgroups, then 512 (128 workgroups at most): a
+// grid-wide sum takes 1.8 us on 64 workgroups, 2.1 us on 128 and 3.1 us on 256.
+constexpr int kRowsS = 256, kRowsL = 512;
+constexpr int64_t kSmallN = 64 * kRowsS;
+// One pass of classical Gram-Schmidt multiplies the basis's loss of orthogonality by
+// |w| / |w'| (the vector's length before and after it; Giraud, Langou, Rozloznik & van
+// den Eshof, Numer. Math. 101, 2005), so the loss is tracked and the pass repeated when
+// it would exceed this part of the solve's own tolerance: at rtol 1e-3 and 10,000 rows
+// no step needs the second pass, which taken always costs 15 %.
+constexpr double kLossPart = 1e-3;
 
 constexpr double kG = 0.58578643762690485;  // 2 - sqrt(2)
 
-struct Trb {
+// J in ELL form (fvm_affine_op), column s of row i at [s n + i]
+struct EllJ {
   int64_t n;
   int W;
-  const int32_t* col;  // [W][n] slot-major
+  const int32_t* col;
   const double* val;
   const double* diag;
   const int32_t* orp;
   const int32_t* ocol;
   const double* oval;
+};
+
+template <int T>
+struct Shared {
+  GridShared<T> grid;
+  double V[kMaxRestart + 1][T];  // the basis on this workgroup's rows
+  double H[kMaxRestart + 1][kMaxRestart];
+  double h[kMaxRestart + 1];
+  double g[kMaxRestart + 1], cs[kMaxRestart], sn[kMaxRestart], y[kMaxRestart];
+};
+
+// The thread's row of J: W slots in registers (W > 0), or read from memory four at a
+// time (W == 0: widths beyond the meshes').
+template <int W>
+struct Row {
+  uint32_t c[W > 0 ? W : 1];  // grid_offset of the column
+  double v[W > 0 ? W : 1];
+  double diag;
+  int o0, o1;
+  __device__ __forceinline__ void load(const EllJ& J, int64_t i, bool active) {
+    diag = active ? J.diag[i] : 0.0;
+    o0 = active ? J.orp[i] : 0;
+    o1 = active ? J.orp[i + 1] : 0;
+#pragma unroll
+    for (int s = 0; s < W; ++s) {
+      c[s] = active ? fvm::grid_offset(J.col[s * J.n + i]) : 0;
+      v[s] = active ? J.val[s * J.n + i] : 0.0;
+    }
+  }
+};
+
+// row i of J x for the vector published last, x this thread's entry of it
+template <int W, int T>
+__device__ __forceinline__ double row_J(const EllJ& J, const Row<W>& R, Grid<T>& G, int64_t i, bool active,
+                                        double x) {
+  double acc = 0.0;
+  if constexpr (W > 0) {
+    double xc[W];
+    G.fetch(R.c, xc, active);
+#pragma unroll
+    for (int s = 0; s < W; ++s) acc += R.v[s] * xc[s];
+  } else if (active) {
+    for (int s0 = 0; s0 < J.W; s0 += 4) {
+      uint32_t c[4];
+      double v[4], xc[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bool on = s0 + s < J.W;
+        c[s] = fvm::grid_offset(on ? J.col[(s0 + s) * J.n + i] : (int)i);
+        v[s] = on ? J.val[(s0 + s) * J.n + i] : 0.0;
+      }
+      G.fetch(c, xc, true);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc += v[s] * xc[s];
+    }
+  }
+  for (int k = R.o0; k < R.o1; ++k) acc += J.oval[k] * G.fetch1(J.ocol[k]);
+  return acc + R.diag * x;
+}
+
+template <int W, int T>
+__device__ __forceinline__ double apply_J(const EllJ& J, const Row<W>& R, Grid<T>& G, int64_t i, bool active,
+                                          double x) {
+  G.publish(i, x, active);
+  return row_J<W>(J, R, G, i, active, x);
+}
+
+// x = A^-1 b approximately, A = a I + bj J, restarted GMRES(m) from x = 0 (solve.py's
+// gmres_device: stop when |r| <= rtol |b|), right-preconditioned by diag(scale) with
+// scale this row's entry; returns the Arnoldi steps taken, or -1 when the grid gave up
+template <int W, int T>
+__device__ __forceinline__ int64_t gmres(Shared<T>& S, Grid<T>& G, const EllJ& J, const Row<W>& R, int64_t i,
+                                         bool active, double a, double bj, double scale, double b, double& x,
+                                         double rtol, int m, int64_t maxiter) {
+  const int tid = threadIdx.x;
+  x = 0.0;
+  double bnorm = -1.0;
+  int64_t total = 0;
+  while (total < maxiter) {
+    // r = b - A x (r = b while x is still zero)
+    double r = b;
+    if (bnorm >= 0.0) r = b - (a * x + bj * apply_J<W>(J, R, G, i, active, x));
+    double rr;
+    if (!G.sum1(r * r, &rr)) return -1;
+    const double beta = sqrt(rr);
+    if (bnorm < 0.0) {
+      bnorm = beta;
+      if (bnorm == 0.0) return 0;
+    } else if (beta <= rtol * bnorm) {
+      break;
+    }
+    double vj = r / beta;
+    S.V[0][tid] = vj;
+    if (tid == 0) S.g[0] = beta;
+    int kd = 0;
+    double loss = 0.0;
+    double z = scale * vj;
+    G.publish(i, z, active);
+    for (int j = 0; j < m; ++j) {
+      double w = a * z + bj * row_J<W>(J, R, G, i, active, z);
+      double ww = 0.0;
+#pragma nounroll
+      for (int pass = 0; pass < 2; ++pass) {
+        // w against the basis, and |w|^2 before the pass
+        if (!G.sum(j + 2, [&](int q) { return (q <= j ? S.V[q][tid] : w) * w; })) return -1;
+        double hh = 0.0;
+#pragma unroll 4
+        for (int q = 0; q <= j; ++q) {
+          const double h = S.grid.tot[q];
+          hh += h * h;
+          w = w - h * S.V[q][tid];
+        }
+        const double w0 = S.grid.tot[j + 1];
+        ww = w0 - hh;  // |w|^2 after it (Pythagoras)
+        if (tid <= j) S.h[tid] = pass == 0 ? S.grid.tot[tid] : S.h[tid] + S.grid.tot[tid];
+        __syncthreads();  // tot is free again, h written
+        const double grown = (loss + 0x1p-52) * sqrt(w0 / ww);
+        if (ww > 0.0 && grown <= kLossPart * rtol) {
+          loss = fmax(loss, grown);
+          break;
+        }
+      }
+      const double hn = sqrt(fmax(ww, 0.0));
+      vj = hn > 0.0 ? w / hn : 0.0;
+      S.V[j + 1][tid] = vj;
+      // the next basis vector goes out before the rotations decide whether it is needed:
+      // they take about as long as its way (one that is not needed is not read, so its
+      // half of the buffer may be written again at once)
+      z = scale * vj;
+      G.publish(i, z, active);
+      if (tid == 0) {
+        double hq = S.h[0];
+#pragma nounroll
+        for (int q = 0; q < j; ++q) {  // previous rotations
+          const double o = S.h[q + 1];
+          S.H[q][j] = S.cs[q] * hq + S.sn[q] * o;
+          hq = -S.sn[q] * hq + S.cs[q] * o;
+        }
+        const double dd = sqrt(hq * hq + hn * hn);
+        const double cs = dd == 0.0 ? 1.0 : hq / dd, sn = dd == 0.0 ? 0.0 : hn / dd;
+        S.cs[j] = cs;
+        S.sn[j] = sn;
+        S.H[j][j] = dd;
+        const double g = S.g[j];
+        S.g[j + 1] = -sn * g;
+        S.g[j] = cs * g;
+      }
+      __syncthreads();
+      ++total;
+      kd = j + 1;
+      if (fabs(S.g[j + 1]) <= rtol * bnorm || total >= maxiter) break;
+    }
+    const double res = fabs(S.g[kd]);
+    if (tid == 0) {  // back substitution
+#pragma nounroll
+      for (int q = kd - 1; q >= 0; --q) {
+        double sum = S.g[q];
+#pragma nounroll
+        for (int p = q + 1; p < kd; ++p) sum -= S.H[q][p] * S.y[p];
+        S.y[q] = sum / S.H[q][q];
+      }
+    }
+    __syncthreads();
+    double acc = 0.0;
+#pragma unroll 4
+    for (int q = 0; q < kd; ++q) acc = acc + S.y[q] * S.V[q][tid];
+    x = x + scale * acc;
+    if (res <= rtol * bnorm) break;
+  }
+  return total;
+}
+
+struct Trb {
+  EllJ J;
   const double* c;
   int32_t n_dir;
   const int32_t* dir_idx;
   const double* dir_val;
-  double* v[14];  // u fn z fg u1 f1 r G dz est tmp interp w spare
-  double* basis;  // (restart + 1) n
+  double* u;  // the state in and out
+  uint64_t* grid;
   double t0, tf, dt, abstol, reltol;
   int64_t maxiters;
   double kappa, krtol;
@@ -54,349 +246,118 @@ struct Trb {
   double* stats;
 };
 
-enum { V_U, V_FN, V_Z, V_FG, V_U1, V_F1, V_R, V_G, V_DZ, V_EST, V_TMP, V_INTERP, V_W, V_SPARE };
-
-struct Shared {
-  double red[kWaves][kChunk];
-  double sums[kChunk];                 // block_sums' results
-  double hp[2][kMaxRestart + 1];       // the two Gram-Schmidt passes' projections
-  double H[kMaxRestart + 1][kMaxRestart];
-  double g[kMaxRestart + 1], cs[kMaxRestart], sn[kMaxRestart], y[kMaxRestart];
-};
-
-__device__ __forceinline__ void bar() { __syncthreads(); }
-
-// Elementwise passes take kU elements per thread per round, every load of a round
-// issued before the first store; each element's arithmetic and each thread's
-// accumulation order (ascending i) are those of a plain loop over i.  One element per
-// round measured fastest (plate 17.6 ms against 18.7 ms with four): four per round
-// doubles the kernel's code to 115 KB, past the 64 KB instruction cache its one CU has.
-constexpr int kU = 1;
-constexpr int kUD = 1;  // the dot sweeps: kUD elements x kChunk basis vectors in flight
-
-template <class L, class St>
-__device__ __forceinline__ void vpass(int64_t n, L load, St store) {
-  for (int64_t i0 = threadIdx.x; i0 < n; i0 += kU * kT) {
-    double v[kU];
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int64_t i = i0 + u * kT;
-      v[u] = i < n ? load(i) : 0.0;
+template <int W, int T>
+__global__ __launch_bounds__(T) void trbdf2_affine_kernel(Trb a) {
+  __shared__ Shared<T> S;
+  const int64_t n = a.J.n;
+  const int64_t i = (int64_t)blockIdx.x * T + threadIdx.x;
+  const bool active = i < n;
+  Grid<T> G;
+  G.open(a.grid, n, &S.grid);
+  Row<W> R;
+  R.load(a.J, i, active);
+  const double ci = active ? a.c[i] : 0.0;
+  double u = active ? a.u[i] : 0.0;
+  bool held = false;  // a Dirichlet node (the last entry naming it wins)
+  double held_at = 0.0;
+  for (int k = 0; k < a.n_dir; ++k)
+    if (a.dir_idx[k] == i) {
+      held = true;
+      held_at = a.dir_val[k];
     }
-#pragma unroll
-    for (int u = 0; u < kU; ++u) {
-      const int64_t i = i0 + u * kT;
-      if (i < n) store(i, v[u]);
-    }
-  }
-}
-
-// sums of k <= kChunk per-thread values over the workgroup, in a fixed order (waves
-// by shuffles, then the waves in order), left in dst[0..k) (LDS) for every thread to
-// read after the call
-__device__ __forceinline__ void block_sums(Shared& S, const double* v, int k, double* dst) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int j = 0; j < kChunk; ++j) {
-    if (j < k) {
-      double x = v[j];
-      for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-      if (lane == 0) S.red[wave][j] = x;
-    }
-  }
-  bar();
-  if ((int)threadIdx.x < k) {
-    double x = 0.0;
-    for (int w = 0; w < kWaves; ++w) x += S.red[w][threadIdx.x];
-    dst[threadIdx.x] = x;
-  }
-  bar();
-}
-
-__device__ __forceinline__ double block_sum(Shared& S, double x) {
-  double v[kChunk] = {x};
-  block_sums(S, v, 1, S.sums);
-  return S.sums[0];
-}
-
-// row i of J x (+ c when affine); W > 0 is the ELL width known at compile time,
-// W == 0 reads it from the operator
-template <int W>
-__device__ __forceinline__ double j_row(const Trb& a, const double* x, int64_t i, bool affine) {
-  const int64_t n = a.n;
-  double acc = 0.0;
-  if (W > 0) {
-    int c[W > 0 ? W : 1];
-    double v[W > 0 ? W : 1];
-#pragma unroll
-    for (int s = 0; s < W; ++s) {
-      c[s] = a.col[s * n + i];
-      v[s] = a.val[s * n + i];
-    }
-#pragma unroll
-    for (int s = 0; s < W; ++s) acc += v[s] * x[c[s]];
-  } else {
-    for (int s = 0; s < a.W; ++s) acc += a.val[s * n + i] * x[a.col[s * n + i]];
-  }
-  for (int k = a.orp[i]; k < a.orp[i + 1]; ++k) acc += a.oval[k] * x[a.ocol[k]];
-  acc += a.diag[i] * x[i];
-  return affine ? acc + a.c[i] : acc;
-}
-
-// y = J x (+ c when affine)
-template <int W>
-__device__ __forceinline__ void apply_J(const Trb& a, const double* x, double* y, bool affine) {
-  vpass(a.n, [&](int64_t i) { return j_row<W>(a, x, i, affine); }, [&](int64_t i, double v) { y[i] = v; });
-  bar();
-}
-
-// sqrt(mean((e / (abstol + reltol max(|p|, |q|)))^2)), the integrators' error norm
-__device__ __forceinline__ double err_norm(Shared& S, const Trb& a, const double* e, const double* p, const double* q) {
-  double acc = 0.0;
-  vpass(
-      a.n,
-      [&](int64_t i) {
-        const double r = e[i] / (a.abstol + a.reltol * fmax(fabs(p[i]), fabs(q[i])));
-        return r * r;
-      },
-      [&](int64_t, double v) { acc += v; });
-  return sqrt(block_sum(S, acc) / (double)a.n);
-}
-
-// x = W^-1 b approximately, W = I - dh J, restarted GMRES(m) from x = 0 (solve.py's
-// gmres_device: stop when |r| <= rtol |b|); returns the Arnoldi steps taken
-template <int W>
-__device__ __forceinline__ int gmres(Shared& S, const Trb& a, const double* b, double* x, double dh, int64_t maxiter) {
-  const int64_t n = a.n;
-  const int m = a.restart;
-  double* w = a.v[V_W];
-  double* r = a.v[V_SPARE];
-  double acc = 0.0;
-  vpass(n, [&](int64_t i) { return b[i]; }, [&](int64_t i, double v) {
-    x[i] = 0.0;
-    acc += v * v;
-  });
-  const double bnorm = sqrt(block_sum(S, acc));
-  if (bnorm == 0.0) return 0;
-  int total = 0;
-  bool x_zero = true;
-  while (total < maxiter) {
-    // r = b - W x (r = b while x is still zero)
-    double beta = bnorm;
-    if (!x_zero) {
-      apply_J<W>(a, x, w, false);
-      acc = 0.0;
-      vpass(
-          n,
-          [&](int64_t i) {
-            const double wx = x[i] - dh * w[i];
-            return b[i] - wx;
-          },
-          [&](int64_t i, double v) {
-            r[i] = v;
-            acc += v * v;
-          });
-      beta = sqrt(block_sum(S, acc));
-      if (beta <= a.krtol * bnorm) break;
-    }
-    const double* rr = x_zero ? b : r;
-    vpass(n, [&](int64_t i) { return rr[i] / beta; }, [&](int64_t i, double v) { a.basis[i] = v; });
-    if (threadIdx.x == 0) {
-      for (int j = 0; j <= m; ++j) S.g[j] = 0.0;
-      S.g[0] = beta;
-    }
-    bar();
-    int kd = 0;
-    for (int j = 0; j < m; ++j) {
-      const double* vj = a.basis + j * n;
-      vpass(n, [&](int64_t i) { return vj[i] - dh * j_row<W>(a, vj, i, false); },
-            [&](int64_t i, double v) { w[i] = v; });
-      bar();
-      // classical Gram-Schmidt applied twice: each pass forms every dot product with
-      // the same w (kChunk per sweep, reduced into S.hp[pass]), then subtracts them
-      // all in one sweep
-      for (int pass = 0; pass < 2; ++pass) {
-        double* hp = S.hp[pass];
-        for (int q0 = 0; q0 <= j; q0 += kChunk) {
-          const int k = j + 1 - q0 < kChunk ? j + 1 - q0 : kChunk;
-          double dd[kChunk];
-#pragma unroll
-          for (int q = 0; q < kChunk; ++q) dd[q] = 0.0;
-          for (int64_t i0 = threadIdx.x; i0 < n; i0 += kUD * kT) {
-            double wv[kUD], bv[kUD][kChunk];
-#pragma unroll
-            for (int u = 0; u < kUD; ++u) {
-              const int64_t i = i0 + u * kT;
-              wv[u] = i < n ? w[i] : 0.0;
-#pragma unroll
-              for (int q = 0; q < kChunk; ++q) bv[u][q] = (q < k && i < n) ? a.basis[(q0 + q) * n + i] : 0.0;
-            }
-#pragma unroll
-            for (int u = 0; u < kUD; ++u) {
-              if (i0 + u * kT < n) {
-#pragma unroll
-                for (int q = 0; q < kChunk; ++q)
-                  if (q < k) dd[q] += bv[u][q] * wv[u];
-              }
-            }
-          }
-          block_sums(S, dd, k, hp + q0);
-        }
-        for (int64_t i0 = threadIdx.x; i0 < n; i0 += kU * kT) {
-          double wv[kU];
-#pragma unroll
-          for (int u = 0; u < kU; ++u) {
-            const int64_t i = i0 + u * kT;
-            wv[u] = i < n ? w[i] : 0.0;
-          }
-          for (int q = 0; q <= j; ++q) {
-            const double h = hp[q];
-            const double* bq = a.basis + q * n;
-#pragma unroll
-            for (int u = 0; u < kU; ++u) {
-              const int64_t i = i0 + u * kT;
-              if (i < n) wv[u] = wv[u] - h * bq[i];
-            }
-          }
-#pragma unroll
-          for (int u = 0; u < kU; ++u) {
-            const int64_t i = i0 + u * kT;
-            if (i < n) w[i] = wv[u];
-          }
-        }
-        bar();
-      }
-      acc = 0.0;
-      vpass(n, [&](int64_t i) { return w[i]; }, [&](int64_t, double v) { acc += v * v; });
-      const double hn = sqrt(block_sum(S, acc));
-      if (hn > 0.0)
-        vpass(n, [&](int64_t i) { return w[i] / hn; }, [&](int64_t i, double v) { a.basis[(j + 1) * n + i] = v; });
-      if (threadIdx.x == 0) {
-        for (int q = 0; q <= j; ++q) S.H[q][j] = S.hp[0][q] + S.hp[1][q];
-        S.H[j + 1][j] = hn;
-        for (int q = 0; q < j; ++q) {  // previous rotations
-          const double p = S.H[q][j], o = S.H[q + 1][j];
-          S.H[q][j] = S.cs[q] * p + S.sn[q] * o;
-          S.H[q + 1][j] = -S.sn[q] * p + S.cs[q] * o;
-        }
-        const double dd = hypot(S.H[j][j], S.H[j + 1][j]);
-        S.cs[j] = dd == 0.0 ? 1.0 : S.H[j][j] / dd;
-        S.sn[j] = dd == 0.0 ? 0.0 : S.H[j + 1][j] / dd;
-        S.H[j][j] = dd;
-        S.H[j + 1][j] = 0.0;
-        S.g[j + 1] = -S.sn[j] * S.g[j];
-        S.g[j] = S.cs[j] * S.g[j];
-      }
-      bar();
-      ++total;
-      kd = j + 1;
-      if (fabs(S.g[j + 1]) <= a.krtol * bnorm || total >= maxiter) break;
-    }
-    if (threadIdx.x == 0) {  // back substitution
-      for (int q = kd - 1; q >= 0; --q) {
-        double sum = S.g[q];
-        for (int p = q + 1; p < kd; ++p) sum -= S.H[q][p] * S.y[p];
-        S.y[q] = sum / S.H[q][q];
-      }
-    }
-    bar();
-    for (int64_t i0 = threadIdx.x; i0 < n; i0 += kU * kT) {
-      double xv[kU];
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const int64_t i = i0 + u * kT;
-        xv[u] = i < n ? x[i] : 0.0;
-      }
-      for (int q = 0; q < kd; ++q) {
-        const double yq = S.y[q];
-        const double* bq = a.basis + q * n;
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
-          const int64_t i = i0 + u * kT;
-          if (i < n) xv[u] = xv[u] + yq * bq[i];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const int64_t i = i0 + u * kT;
-        if (i < n) x[i] = xv[u];
-      }
-    }
-    bar();
-    x_zero = false;
-    if (fabs(S.g[kd]) <= a.krtol * bnorm) break;
-  }
-  return total;
-}
-
-__device__ __forceinline__ void lincomb2(const Trb& a, double* out, double p, const double* x, double q,
-                                         const double* y) {
-  vpass(a.n, [&](int64_t i) { return p * x[i] + q * y[i]; }, [&](int64_t i, double v) { out[i] = v; });
-  bar();
-}
-
-template <int W>
-__global__ __launch_bounds__(kT) void trbdf2_affine_kernel(Trb a) {
-  __shared__ Shared S;
-  const int64_t n = a.n;
-  double *u = a.v[V_U], *fn = a.v[V_FN], *z = a.v[V_Z], *fg = a.v[V_FG], *u1 = a.v[V_U1], *f1 = a.v[V_F1];
-  double *r = a.v[V_R], *G = a.v[V_G], *dz = a.v[V_DZ], *est = a.v[V_EST], *tmp = a.v[V_TMP];
   const double d = kG / 2;
   const double TA = 1.0 / (kG * (2.0 - kG)), TB = -(1.0 - kG) * (1.0 - kG) / (kG * (2.0 - kG));
   const double TK = (3 * kG * kG - 4 * kG + 2) / (6 * (2.0 - kG));
   int64_t nf = 0, njvp = 0, naccept = 0, nreject = 0, nnewton = 0, nkrylov = 0, nfail = 0, ks = 0, it = 0;
   int retcode = 0;  // FVM_ODE_SUCCESS
+  bool up = true;   // the grid's exchanges work
   double t = a.t0, dt = a.dt, eta_keep = 1.0;
-  apply_J<W>(a, u, fn, true);
-  ++nf;
-  // Newton on z - d h f(z) = rhs from the predictor in z; fz <- f(z); false on failure
-  auto newton = [&](double* zz, const double* rhs, double h, double* fz) -> bool {
-    const double dh = d * h;
-    double eta = fvm::ctrl_pow(fmax(eta_keep, 1e-16), 0.8), prev = -1.0;
-    bool ok = false;
-    for (int itn = 0; itn < a.max_newton; ++itn) {
-      apply_J<W>(a, zz, fz, true);
-      ++nf;
-      vpass(n, [&](int64_t i) { return -1.0 * zz[i] + dh * fz[i] + rhs[i]; }, [&](int64_t i, double v) { G[i] = v; });
-      bar();
-      const int ki = gmres<W>(S, a, G, dz, dh, 20 * (int64_t)a.restart);
-      nkrylov += ki;
-      njvp += ki + 1;
-      vpass(n, [&](int64_t i) { return zz[i] + dz[i]; }, [&](int64_t i, double v) { zz[i] = v; });
-      bar();
-      ++nnewton;
-      const double ndz = err_norm(S, a, dz, u, zz);
-      if (!isfinite(ndz)) return false;
-      if (prev >= 0.0) {
-        const double theta = ndz / prev;
-        if (theta >= 1.0) return false;
-        eta = theta / (1.0 - theta);
-      }
-      if (eta * ndz <= a.kappa || ndz == 0.0) {
-        ok = true;
-        break;
-      }
-      prev = ndz;
-    }
-    if (!ok) return false;
-    eta_keep = eta;
-    apply_J<W>(a, zz, fz, true);
-    ++nf;
-    return true;
+  // sqrt(mean((e / (abstol + reltol max(|p|, |q|)))^2)), the integrators' error norm
+  auto err_norm = [&](double e, double p, double q) {
+    const double r = e / (a.abstol + a.reltol * fmax(fabs(p), fabs(q)));
+    double s = 0.0;
+    up = up && G.sum1(active ? r * r : 0.0, &s);
+    return sqrt(s / (double)n);
   };
+  double fn = 0.0;
+  bool fresh = false;  // fn = f(u)
   while (t < a.tf && it < a.maxiters) {
     ++it;
-    const double h = fmin(dt, a.tf - t);
-    // TR stage: z - d h f(z) = u + d h f_n, predictor u + gamma h f_n
-    lincomb2(a, r, 1.0, u, d * h, fn);
-    lincomb2(a, z, 1.0, u, kG * h, fn);
-    bool ok = newton(z, r, h, fg);
-    if (ok) {
-      // BDF2 stage: u1 - d h f(u1) = A z + B u, predictor z + (1 - gamma) h f_gamma
-      lincomb2(a, r, TA, z, TB, u);
-      lincomb2(a, u1, 1.0, z, (1.0 - kG) * h, fg);
-      ok = newton(u1, r, h, f1);
+    const double h = fmin(dt, a.tf - t), dh = d * h;
+    // Three solves per step: stage 0, TR: z - d h f(z) = u + d h f_n, predictor
+    // u + gamma h f_n; stage 1, BDF2: u1 - d h f(u1) = A z + B u, predictor
+    // z + (1 - gamma) h f_gamma; each by Newton.  Stage 2: the error estimate through
+    // W^-1.  One loop, so that the product and the Krylov solve are compiled once.
+    double z = u, u1 = 0.0, fg = 0.0, f1 = 0.0, est = 0.0;
+    bool ok = true;
+#pragma nounroll
+    for (int stage = fresh ? 0 : -1; stage < 3 && ok; ++stage) {
+      double x = 0.0, fx = 0.0, rhs = 0.0;
+      if (stage == -1) {
+        x = u;
+      } else if (stage == 0) {
+        rhs = u + dh * fn;
+        x = u + kG * h * fn;
+      } else if (stage == 1) {
+        rhs = TA * z + TB * u;
+        x = z + (1.0 - kG) * h * fg;
+      } else {
+        if (!a.smooth) break;
+      }
+      double eta = fvm::ctrl_pow(fmax(eta_keep, 1e-16), 0.8), prev = -1.0;
+      bool done = stage == -1;
+      ok = done;
+#pragma nounroll
+      for (int itn = 0;; ++itn) {
+        double b = est;
+        if (stage < 2) {
+          fx = apply_J<W>(a.J, R, G, i, active, x) + ci;
+          ++nf;
+          if (done || itn == a.max_newton) break;
+          b = -1.0 * x + dh * fx + rhs;
+        }
+        double dx;
+        const int64_t k = gmres<W, T>(S, G, a.J, R, i, active, 1.0, -dh, 1.0, b, dx, a.krtol, a.restart,
+                                      20 * (int64_t)a.restart);
+        up = up && k >= 0;
+        if (!up) break;
+        nkrylov += k;
+        njvp += k + 1;
+        if (stage == 2) {
+          est = dx;
+          ok = true;
+          break;
+        }
+        x = x + dx;
+        ++nnewton;
+        const double ndz = err_norm(dx, u, x);
+        if (!up || !isfinite(ndz)) break;
+        if (prev >= 0.0) {
+          const double theta = ndz / prev;
+          if (theta >= 1.0) break;
+          eta = theta / (1.0 - theta);
+        }
+        if (eta * ndz <= a.kappa || ndz == 0.0) done = ok = true;
+        prev = ndz;
+      }
+      if (!ok) break;
+      if (stage == -1) {
+        fn = fx;
+        fresh = true;
+      } else if (stage == 0) {
+        z = x;
+        fg = fx;
+        eta_keep = eta;
+      } else if (stage == 1) {
+        u1 = x;
+        f1 = fx;
+        eta_keep = eta;
+        est = TK * h / kG * fn;
+        est = est + -TK * h / (kG * (1 - kG)) * fg;
+        est = est + TK * h / (1 - kG) * f1;
+      }
     }
+    if (!up) break;
     if (!ok) {
       ++nfail;
       ++nreject;
@@ -407,26 +368,8 @@ __global__ __launch_bounds__(kT) void trbdf2_affine_kernel(Trb a) {
       }
       continue;
     }
-    {
-      const double c0 = TK * h / kG, c1 = -TK * h / (kG * (1 - kG)), c2 = TK * h / (1 - kG);
-      vpass(
-          n,
-          [&](int64_t i) {
-            double v = c0 * fn[i];
-            v = v + c1 * fg[i];
-            return v + c2 * f1[i];
-          },
-          [&](int64_t i, double v) { est[i] = v; });
-      bar();
-    }
-    const double* e = est;
-    if (a.smooth) {
-      const int ki = gmres<W>(S, a, est, tmp, d * h, 20 * (int64_t)a.restart);
-      nkrylov += ki;
-      njvp += ki + 1;
-      e = tmp;
-    }
-    const double EEst = err_norm(S, a, e, u, u1);
+    const double EEst = err_norm(est, u, u1);
+    if (!up) break;
     if (!isfinite(EEst)) {
       retcode = 2;  // Unstable
       break;
@@ -437,32 +380,21 @@ __global__ __launch_bounds__(kT) void trbdf2_affine_kernel(Trb a) {
         const double th = fmin(1.0, fmax(0.0, (a.save_t[ks] - t) / h));
         const double t2 = th * th, t3 = t2 * th;
         const double h00 = 2 * t3 - 3 * t2 + 1, h10 = t3 - 2 * t2 + th, h01 = -2 * t3 + 3 * t2, h11 = t3 - t2;
-        const double q0 = h00, q1 = h10 * h, q2 = h01, q3 = h11 * h;
-        double* out = a.saves + ks * n;
-        vpass(
-            n,
-            [&](int64_t i) {
-              double v = q0 * u[i];
-              v = v + q1 * fn[i];
-              v = v + q2 * u1[i];
-              return v + q3 * f1[i];
-            },
-            [&](int64_t i, double v) { out[i] = v; });
+        double v = h00 * u;
+        v = v + h10 * h * fn;
+        v = v + h01 * u1;
+        v = v + h11 * h * f1;
+        if (active) a.saves[ks * n + i] = v;
         ++ks;
       }
-      bar();
-      vpass(n, [&](int64_t i) { return u1[i]; }, [&](int64_t i, double v) { u[i] = v; });
-      bar();
+      u = u1;
       t = tn;
       ++naccept;
       if (a.n_dir > 0) {  // the Dirichlet callback (values constant), then f(u) afresh
-        for (int k = threadIdx.x; k < a.n_dir; k += kT) u[a.dir_idx[k]] = a.dir_val[k];
-        bar();
-        apply_J<W>(a, u, fn, true);
-        ++nf;
+        if (held) u = held_at;
+        fresh = false;
       } else {
-        vpass(n, [&](int64_t i) { return f1[i]; }, [&](int64_t i, double v) { fn[i] = v; });
-        bar();
+        fn = f1;
       }
     } else {
       ++nreject;
@@ -475,7 +407,8 @@ __global__ __launch_bounds__(kT) void trbdf2_affine_kernel(Trb a) {
     }
   }
   if (retcode == 0 && !(t >= a.tf)) retcode = 1;  // MaxIters
-  if (threadIdx.x == 0) {
+  if (active) a.u[i] = u;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     double* st = a.stats;
     st[0] = t;
     st[1] = (double)nf;
@@ -486,18 +419,61 @@ __global__ __launch_bounds__(kT) void trbdf2_affine_kernel(Trb a) {
     st[6] = (double)nkrylov;
     st[7] = (double)nfail;
     st[8] = (double)ks;
-    st[9] = (double)retcode;
+    st[9] = up ? (double)retcode : -1.0;
   }
+}
+
+EllJ ell_of(const fvm_affine_op* op) {
+  EllJ J;
+  J.n = op->n;
+  J.W = op->width;
+  J.col = op->d_col;
+  J.val = op->d_val;
+  J.diag = op->d_diag;
+  J.orp = op->d_ovf_rp;
+  J.ocol = op->d_ovf_col;
+  J.oval = op->d_ovf_val;
+  return J;
+}
+
+// Launches kernel<W, T> cooperatively for an operator of n rows and ELL width w, the
+// widths of triangle meshes as compile-time constants, others at run time.
+#define FVM_TRB_LAUNCH(kernel, w, n, args, st)                                                                  \
+  ([&]() -> hipError_t {                                                                                       \
+    const bool big_ = (n) > kSmallN;                                                                           \
+    const unsigned t_ = big_ ? kRowsL : kRowsS, g_ = (unsigned)(((n) + t_ - 1) / t_);                          \
+    const void* f_ = nullptr;                                                                                  \
+    switch (w) {                                                                                               \
+      case 4: f_ = big_ ? (const void*)kernel<4, kRowsL> : (const void*)kernel<4, kRowsS>; break;               \
+      case 5: f_ = big_ ? (const void*)kernel<5, kRowsL> : (const void*)kernel<5, kRowsS>; break;               \
+      case 6: f_ = big_ ? (const void*)kernel<6, kRowsL> : (const void*)kernel<6, kRowsS>; break;               \
+      case 7: f_ = big_ ? (const void*)kernel<7, kRowsL> : (const void*)kernel<7, kRowsS>; break;               \
+      case 8: f_ = big_ ? (const void*)kernel<8, kRowsL> : (const void*)kernel<8, kRowsS>; break;               \
+      case 9: f_ = big_ ? (const void*)kernel<9, kRowsL> : (const void*)kernel<9, kRowsS>; break;               \
+      case 10: f_ = big_ ? (const void*)kernel<10, kRowsL> : (const void*)kernel<10, kRowsS>; break;            \
+      default: f_ = big_ ? (const void*)kernel<0, kRowsL> : (const void*)kernel<0, kRowsS>;                     \
+    }                                                                                                          \
+    void* p_[] = {&(args)};                                                                                    \
+    return hipLaunchCooperativeKernel(f_, dim3(g_), dim3(t_), p_, 0, (st));                                    \
+  }())
+
+int check_op(const fvm_affine_op* op, const char* who) {
+  FVM_CHECK(op->n > 0 && op->n <= kMaxN, std::string(who) + ": 1 <= n <= 65536");
+  FVM_CHECK(op->width >= 0 && op->d_col && op->d_val && op->d_diag && op->d_ovf_rp,
+            std::string(who) + ": incomplete operator");
+  return FVM_OK;
 }
 
 }  // namespace
 
-extern "C" int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts* o, double* d_u,
-                                 fvm_trbdf2_stats* st, fvm_stream s) {
+extern "C" {
+
+int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts* o, double* d_u, fvm_trbdf2_stats* st,
+                      fvm_stream s) {
   FVM_CHECK(op && o && d_u && st, "fvm_trbdf2_affine: null argument");
-  FVM_CHECK(op->n > 0 && op->n <= kMaxN, "fvm_trbdf2_affine: 1 <= n <= 65536 (one workgroup)");
-  FVM_CHECK(op->width >= 0 && op->d_col && op->d_val && op->d_diag && op->d_ovf_rp && op->d_c,
-            "fvm_trbdf2_affine: incomplete operator");
+  int rc = check_op(op, "fvm_trbdf2_affine");
+  if (rc) return rc;
+  FVM_CHECK(op->d_c, "fvm_trbdf2_affine: incomplete operator");
   FVM_CHECK(op->n_dirichlet == 0 || (op->d_dir_nodes && op->d_dir_values), "fvm_trbdf2_affine: Dirichlet lists");
   FVM_CHECK(o->krylov_restart >= 1 && o->krylov_restart <= kMaxRestart, "fvm_trbdf2_affine: restart 1..30");
   FVM_CHECK(o->max_newton >= 1 && o->abstol > 0 && o->reltol >= 0 && o->maxiters > 0 && o->tf >= o->t0 &&
@@ -506,18 +482,12 @@ extern "C" int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts*
   FVM_CHECK(o->n_save >= 0 && (o->n_save == 0 || (o->save_t && o->d_saves)), "fvm_trbdf2_affine: save times");
   const int64_t n = op->n;
   Trb a;
-  a.n = n;
-  a.W = op->width;
-  a.col = op->d_col;
-  a.val = op->d_val;
-  a.diag = op->d_diag;
-  a.orp = op->d_ovf_rp;
-  a.ocol = op->d_ovf_col;
-  a.oval = op->d_ovf_val;
+  a.J = ell_of(op);
   a.c = op->d_c;
   a.n_dir = op->n_dirichlet;
   a.dir_idx = op->d_dir_nodes;
   a.dir_val = op->d_dir_values;
+  a.u = d_u;
   a.t0 = o->t0;
   a.tf = o->tf;
   a.dt = o->dt;
@@ -531,39 +501,27 @@ extern "C" int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts*
   a.smooth = o->smooth_est;
   a.n_save = o->n_save;
   a.saves = o->d_saves;
-  const int nvec = 14 + o->krylov_restart + 1;
+  const size_t words = fvm::grid_words(n);
   double* base = nullptr;
-  FVM_HIP(hipMalloc((void**)&base, sizeof(double) * ((size_t)nvec * n + (size_t)o->n_save + 16)));
-  for (int k = 0; k < 14; ++k) a.v[k] = base + k * n;
-  a.basis = base + 14 * n;
-  double* tail = base + (size_t)nvec * n;
+  FVM_HIP(hipMalloc((void**)&base, sizeof(double) * (words + (size_t)o->n_save + 16)));
+  a.grid = (uint64_t*)base;
+  double* tail = base + words;
   a.save_t = tail;
   a.stats = tail + o->n_save;
   hipStream_t st_ = (hipStream_t)s;
-  hipError_t e = hipMemcpyAsync(a.v[V_U], d_u, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice, st_);
+  double r[10] = {0};
+  hipError_t e = hipMemsetAsync(base, 0, sizeof(double) * words, st_);
   if (e == hipSuccess && o->n_save > 0)
     e = hipMemcpyAsync(tail, o->save_t, sizeof(double) * (size_t)o->n_save, hipMemcpyHostToDevice, st_);
-  if (e == hipSuccess) {
-    // the ELL widths of triangle meshes as compile-time constants; others at run time
-    switch (a.W) {
-#define FVM_TRB_W(w)                                                               \
-  case w:                                                                          \
-    hipLaunchKernelGGL(trbdf2_affine_kernel<w>, dim3(1), dim3(kT), 0, st_, a); \
-    break;
-      FVM_TRB_W(4) FVM_TRB_W(5) FVM_TRB_W(6) FVM_TRB_W(7) FVM_TRB_W(8) FVM_TRB_W(9) FVM_TRB_W(10)
-      FVM_TRB_W(11) FVM_TRB_W(12)
-#undef FVM_TRB_W
-      default:
-        hipLaunchKernelGGL(trbdf2_affine_kernel<0>, dim3(1), dim3(kT), 0, st_, a);
-    }
-    e = hipGetLastError();
-  }
-  double r[10] = {0};
-  if (e == hipSuccess) e = hipMemcpyAsync(d_u, a.v[V_U], sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice, st_);
+  if (e == hipSuccess) e = FVM_TRB_LAUNCH(trbdf2_affine_kernel, a.J.W, n, a, st_);
   if (e == hipSuccess) e = hipMemcpyAsync(r, a.stats, sizeof r, hipMemcpyDeviceToHost, st_);
   if (e == hipSuccess) e = hipStreamSynchronize(st_);
   (void)hipFree(base);
   if (e != hipSuccess) return fvm::hip_fail(e, "fvm_trbdf2_affine");
+  if (r[9] < 0) {
+    fvm::set_error("fvm_trbdf2_affine: the grid's exchange timed out");
+    return FVM_ERR_HIP;
+  }
   st->t = r[0];
   st->nf = (int64_t)r[1];
   st->njvp = (int64_t)r[2];
@@ -576,3 +534,5 @@ extern "C" int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts*
   st->retcode = (int32_t)r[9];
   return FVM_OK;
 }
+
+}  // extern "C"

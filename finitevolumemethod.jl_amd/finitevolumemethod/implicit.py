@@ -7,8 +7,8 @@ constant J.  The reference hands such problems to TRBDF2 with a KLU factorisatio
 J on its jacobian_sparsity pattern (solve.jl:50-77, 167-183).  Here J is extracted
 once per problem from fvm_jvp probes over a distance-2 colouring of that pattern (one
 probe per colour, about a dozen on a triangle mesh; exact for an affine f), stored in
-ELL form, and fvm_trbdf2_affine integrates the whole problem in one workgroup (no host
-round trip per Krylov iteration).  Problems above 65,536 unknowns, with a user
+ELL form, and fvm_trbdf2_affine integrates the whole problem in one launch of resident
+workgroups (no host round trip per Krylov iteration).  Problems above 65,536 unknowns, with a user
 callback, without save times or outside the affine forms keep the host-driven
 integrator (solve.py).
 """

@@ -469,7 +469,7 @@ int fvm_vec_lincomb_err_norm(int64_t n, int nterms, const double* coefs, const d
 /* ---- TR-BDF2 for small affine problems (solve.jl:167-183 with TRBDF2) -------
  * f(u) = J u + c with J constant (linear fluxes, sources affine in u, conditions
  * constant in t): the whole TR-BDF2 integration (the tutorials' stiff integrator,
- * there with a KLU factorisation of J) in one workgroup: Newton with GMRES on
+ * there with a KLU factorisation of J) in one launch: Newton with GMRES on
  * W = I - d h J per stage, the W^-1-filtered error estimate, the step controller,
  * the Dirichlet update after every accepted step (constant values) and saveat.
  * J comes in ELL form (width columns per row, slot-major [width][n], padding slots

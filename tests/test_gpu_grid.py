@@ -1,0 +1,48 @@
+"""The kernels whose workgroups exchange data without leaving the kernel (fvm_grid.hpp),
+at the sizes where their layout changes: one workgroup, whole and ragged last
+workgroups, 256- and 512-row workgroups, rows wider than the unrolled widths.
+
+fvm_trbdf2_affine against the host integrator on the same problem, both with Newton
+stopped at 1e-7 and GMRES at 1e-9 of their scales: the two then take the same steps and
+differ by the Newton tolerance times the error norm's scale (abstol + reltol |u|, 1e-3
+|u| here) per solve, two solves a step: at most 2e-10 |u| per step, 1e-8 |u| over the
+fifty steps allowed here, and 1e-7 with the step controller's own amplification."""
+import numpy as np
+import pytest
+
+import finitevolumemethod as FVM
+from test_gpu_templates import wheel_triangulation
+
+pytestmark = pytest.mark.gpu
+
+
+def _problem(tri, steps=0.05):
+    mesh = FVM.FVMGeometry(tri)
+    segs = tri.num_boundary_segments()
+    fns = tuple((lambda x, y, t, u, p, k=k: 0.3 * k + 0.0 * u) for k in range(segs))
+    types = tuple(FVM.Dirichlet if k % 2 else FVM.Neumann for k in range(segs))
+    u0 = 1.0 + np.sin(2 * tri.x) * np.cos(3 * tri.y)
+    return FVM.FVMProblem(mesh, FVM.BoundaryConditions(mesh, fns, types),
+                          diffusion_function=lambda x, y, t, u, p: 0.2 + 0.1 * x * y,
+                          source_function=lambda x, y, t, u, p: x - 0.5 * u, initial_condition=u0, final_time=steps)
+
+
+@pytest.mark.parametrize("shape", [(3, 3), (16, 16), (257, 1), (23, 41), (128, 128), (131, 127), "wheel"], ids=str)
+def test_affine_trbdf2_matches_the_host_integrator(gpu, shape):
+    if shape == "wheel":
+        tri = wheel_triangulation()
+    elif shape[1] == 1:  # 257 nodes: one row in the second workgroup
+        g = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 16, 16, single_boundary=True)
+        tri = FVM.triangulate(np.append(g.x, 1.5), np.append(g.y, 0.4))
+    else:
+        tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, *shape, single_boundary=False)
+    prob = _problem(tri)
+    opts = dict(newton_kappa=1e-7, krylov_rtol=1e-9)
+    a = FVM.solve(prob, FVM.TRBDF2(**opts), saveat=[0.02, 0.05])
+    b = FVM.solve(prob, FVM.TRBDF2(device_loop=False, **opts), saveat=[0.02, 0.05])
+    assert a.stats.get("device_loop") and a.retcode == b.retcode == "Success"
+    assert a.stats["naccept"] == b.stats["naccept"] <= 50, (a.stats, b.stats)
+    for x, y in zip(a.u, b.u):
+        assert np.max(np.abs(x - y)) <= 1e-7 * np.max(np.abs(y))
+    again = FVM.solve(prob, FVM.TRBDF2(**opts), saveat=[0.02, 0.05])
+    assert all(np.array_equal(x, y) for x, y in zip(a.u, again.u))  # sums in a fixed order
