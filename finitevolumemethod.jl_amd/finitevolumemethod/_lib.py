@@ -236,6 +236,12 @@ HIP_API = {
     "fvm_vec_mdot_noalloc": [ctypes.c_int64, ctypes.c_int32, ctypes.POINTER(_vp), _vp, _vp, _vp],
     "fvm_vec_maxpy": [ctypes.c_int64, _vp, ctypes.c_int32, _dp, ctypes.POINTER(_vp), _vp],
     "fvm_trbdf2_affine": [_vp, _vp, _vp, _vp, _vp],
+    "fvm_gmres_work_bytes": [ctypes.c_int64],
+    "fvm_gmres_ell": [_vp, ctypes.c_double, ctypes.c_double, ctypes.c_int32, _vp, _vp, ctypes.c_double,
+                      ctypes.c_int32, ctypes.c_int64, _vp, _vp],
+    "fvm_gmres_iterations": [_vp, _i64p, _vp],
+    "fvm_jacobian_ell": [_vp, ctypes.c_int32, ctypes.POINTER(_vp), _vp, ctypes.c_int32, _vp, ctypes.c_double, _vp,
+                         _vp, _vp, _vp],
     "fvm_arnoldi_step_scaled": [ctypes.c_int32, _vp, ctypes.c_int64, _vp, ctypes.c_double, ctypes.c_double,
                                 ctypes.c_double, _vp, _vp, ctypes.c_int32, ctypes.POINTER(_vp), _vp, _dp, _vp],
     "fvm_jit_check": [ctypes.c_char_p, ctypes.c_int32, ctypes.POINTER(ctypes.c_size_t)],
@@ -258,7 +264,7 @@ def hip_lib():
             for name, args in HIP_API.items():
                 f = getattr(L, name)
                 f.argtypes = args
-                f.restype = ctypes.c_int
+                f.restype = ctypes.c_size_t if name == "fvm_gmres_work_bytes" else ctypes.c_int
             _hip = L
     return _hip
 

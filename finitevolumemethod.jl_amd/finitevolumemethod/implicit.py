@@ -86,6 +86,39 @@ def _colouring(rp, col, n):
     return colour.astype(np.int64)
 
 
+class _EllSlots:
+    """Where the entries of a CSR pattern that holds every diagonal lie in ELL form: the
+    off-diagonals of each row in CSR order, slot-major [W][n], the diagonal apart."""
+
+    def __init__(self, rp, col, n):
+        rows = np.repeat(np.arange(n), np.diff(rp))
+        on = col == rows
+        if not np.all(np.bincount(rows[on], minlength=n) == 1):
+            raise ValueError("the pattern must hold every diagonal entry")
+        slot = np.arange(len(col)) - rp[rows]  # position in the row, diagonal included
+        dpos = np.zeros(n, np.int64)
+        dpos[rows[on]] = slot[on]
+        self.n, self.on, self.off = n, on, ~on
+        self.row = rows[self.off]
+        self.slot = (slot - (slot > dpos[rows]))[self.off]  # minus 1 after the diagonal
+        self.col = col[self.off]
+        self.W = int(np.bincount(self.row, minlength=n).max()) if n else 0
+
+    def diagonal(self, v):
+        return v[self.on].copy()
+
+    def columns(self):
+        """The columns, padded with the row's own."""
+        ecol = np.repeat(np.arange(self.n, dtype=np.int32)[None, :], self.W, axis=0)
+        ecol[self.slot, self.row] = self.col
+        return ecol
+
+    def spread(self, v, pad):
+        e = np.full((self.W, self.n), pad, np.asarray(v).dtype)
+        e[self.slot, self.row] = v[self.off]
+        return e
+
+
 class AffineOperator:
     """J (ELL form on the device), c = f(0) and the Dirichlet values of an affine
     problem, built once."""
@@ -111,23 +144,9 @@ class AffineOperator:
         self.n_colours = int(colour.max()) + 1
         f0 = _lib.DeviceArray(n)
         ctx.rhs(zero, f0, t0)
-        # ELL: the off-diagonals of each row, padded with the row's own column
-        diag = val[col == rows].copy() if np.all(np.bincount(rows[col == rows], minlength=n) == 1) else None
-        if diag is None:
-            raise ValueError("the pattern must hold every diagonal entry")
-        off = col != rows
-        cnt = np.bincount(rows[off], minlength=n)
-        W = int(cnt.max()) if n else 0
-        ecol = np.repeat(np.arange(n, dtype=np.int32)[None, :], W, axis=0)
-        eval_ = np.zeros((W, n))
-        slot = np.arange(len(col)) - rp[rows]  # position in the row, diagonal included
-        # slot among the off-diagonals: subtract 1 after the diagonal
-        dpos = np.zeros(n, np.int64)
-        dpos[rows[~off]] = slot[~off]
-        s_off = slot - (slot > dpos[rows])
-        ecol[s_off[off], rows[off]] = col[off]
-        eval_[s_off[off], rows[off]] = val[off]
-        self.W = W
+        slots = _EllSlots(rp, col, n)
+        diag, ecol, eval_ = slots.diagonal(val), slots.columns(), slots.spread(val, 0.0)
+        self.W = slots.W
         self.d_col = _lib.DeviceArray.from_host(ecol.ravel(), np.int32)
         self.d_val = _lib.DeviceArray.from_host(eval_.ravel())
         self.d_diag = _lib.DeviceArray.from_host(diag)
@@ -153,6 +172,66 @@ class AffineOperator:
         o.n_dirichlet = len(self.dir_nodes)
         o.d_dir_nodes, o.d_dir_values = self.d_dir_nodes.ptr, self.d_dir_values.ptr
         return o
+
+
+class FrozenJacobian:
+    """J(u, t) of an FVMProblem in ELL form, taken again at each step's start, and GMRES
+    on a I + b J in one launch (fvm_jacobian_ell, fvm_gmres_ell): the Newton steps of the
+    host TR-BDF2 loop for problems of at most MAX_N unknowns.  The pattern's colouring and
+    slots are kept on the problem."""
+
+    MAX_COLOURS, MAX_WIDTH = 64, 32  # a hub node of a fan: matrix-free (jacobian_diagonal) instead
+
+    @classmethod
+    def of(cls, prob):
+        """A FrozenJacobian for prob, or None where the pattern is not one for it."""
+        from .problem import FVMProblem
+
+        if not isinstance(prob, FVMProblem) or prob.mesh.triangulation.num_points() > MAX_N:
+            return None
+        plan = getattr(prob, "_jacobian_plan", None)
+        if plan is None:
+            n = prob.mesh.triangulation.num_points()
+            rp, col = csr_pattern(prob.mesh.triangulation)
+            colour = _colouring(rp, col, n)
+            slots = _EllSlots(rp, col, n)
+            nc = int(colour.max()) + 1
+            plan = prob._jacobian_plan = (nc, slots.W, None) if nc > cls.MAX_COLOURS or slots.W > cls.MAX_WIDTH else (
+                nc, slots.W, [_lib.DeviceArray.from_host((colour == c).astype(np.float64)) for c in range(nc)],
+                _lib.DeviceArray.from_host(np.concatenate([slots.spread(colour[col].astype(np.uint8), 255),
+                                                           colour.astype(np.uint8)[None, :]]).ravel(), np.uint8),
+                _lib.DeviceArray.from_host(slots.columns().ravel(), np.int32),
+                _lib.DeviceArray.from_host(np.zeros(n + 1, np.int32), np.int32))
+        return cls(prob, plan) if plan[2] is not None else None
+
+    def __init__(self, prob, plan):
+        self.ctx = prob.device_context()
+        self.n = n = prob.mesh.triangulation.num_points()
+        self.n_colours, self.W, self.probes, self.d_colour, self.d_col, self.d_orp = plan
+        self.probe_ptrs = (_lib._vp * self.n_colours)(*[p.ptr for p in self.probes])
+        self.products = _lib.DeviceArray(self.n_colours * n)
+        self.d_val, self.d_diag = _lib.DeviceArray(self.W * n), _lib.DeviceArray(n)
+        self.work = _lib.DeviceArray.zeros(_lib.hip_lib().fvm_gmres_work_bytes(n) // 8)
+        o = self.op = AffineOp()
+        o.n, o.width = n, self.W
+        o.d_col, o.d_val, o.d_diag, o.d_ovf_rp = self.d_col.ptr, self.d_val.ptr, self.d_diag.ptr, self.d_orp.ptr
+
+    def take(self, u, t):
+        """J at (u, t)."""
+        _lib.check(_lib.hip_lib().fvm_jacobian_ell(self.ctx.handle, self.n_colours, self.probe_ptrs, self.d_colour.ptr,
+                                                   self.W, u.ptr, float(t), self.products.ptr, self.d_val.ptr,
+                                                   self.d_diag.ptr, None), "fvm_jacobian_ell")
+
+    def solve(self, a, b, rhs, x, rtol, restart, maxiter, jacobi):
+        """x = (a I + b J)^-1 rhs; does not wait for it."""
+        _lib.check(_lib.hip_lib().fvm_gmres_ell(ctypes.byref(self.op), float(a), float(b), int(jacobi), rhs.ptr, x.ptr,
+                                                float(rtol), int(restart), int(maxiter), self.work.ptr, None),
+                   "fvm_gmres_ell")
+
+    def iterations(self):
+        k = ctypes.c_int64()
+        _lib.check(_lib.hip_lib().fvm_gmres_iterations(self.work.ptr, ctypes.byref(k), None), "fvm_gmres_ell")
+        return k.value
 
 
 def affine_operator(prob):

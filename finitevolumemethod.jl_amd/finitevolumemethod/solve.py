@@ -210,10 +210,13 @@ def solve(prob, alg=None, *, saveat=None, abstol=None, reltol=None, dt=None, max
     has_dir = prob.conditions.has_dirichlet_nodes()
     cb = (lambda u, t: ctx.apply_dirichlet(u, t)) if has_dir else None
     extra = {}
-    if isinstance(alg, TRBDF2) and alg.precond == "jacobi":
-        extra["jac_diag"] = jacobian_diagonal(prob)
-    elif isinstance(alg, TRBDF2) and alg.precond != "none":
-        raise ValueError(f"TRBDF2: unknown precond {alg.precond!r} (\"jacobi\" or \"none\")")
+    if isinstance(alg, TRBDF2):
+        if alg.precond not in ("jacobi", "none"):
+            raise ValueError(f"TRBDF2: unknown precond {alg.precond!r} (\"jacobi\" or \"none\")")
+        if alg.device_loop and 1 <= alg.krylov_restart <= 30:
+            extra["jacobian"] = implicit.FrozenJacobian.of(prob)
+        if extra.get("jacobian") is None and alg.precond == "jacobi":
+            extra["jac_diag"] = jacobian_diagonal(prob)
     return integrate(rhs, prob.initial_condition, prob.initial_time, prob.final_time,
                      alg if alg is not None else Tsit5(), saveat=saveat, abstol=abstol,
                      reltol=reltol, dt=dt, maxiters=maxiters, save_start=save_start,
@@ -286,7 +289,7 @@ def integrate(rhs, u0, t0, tf, alg, *, saveat=None, save_start=True, **kwargs):
 
 def _integrate(rhs, u0, t0, tf, alg, *, saveat=None, abstol=1e-6, reltol=1e-3, dt=None,
                maxiters=10**7, save_start=True, step_callback=None, user_callback=None, jvp=None,
-               op=None, fsal=False, jac_diag=None):
+               op=None, fsal=False, jac_diag=None, jacobian=None):
     """Integrate du/dt = rhs(u, t) on the device from t0 to tf.  Implicit methods
     need jvp(u, v, out, t) = J(u) v.
 
@@ -309,7 +312,7 @@ def _integrate(rhs, u0, t0, tf, alg, *, saveat=None, abstol=1e-6, reltol=1e-3, d
         return _integrate_trbdf2(rhs, jvp, u0, t0, tf, alg, saveat=saveat, abstol=abstol,
                                  reltol=reltol, dt=dt, maxiters=maxiters, save_start=save_start,
                                  step_callback=step_callback, user_callback=user_callback, op=op,
-                                 jac_diag=jac_diag)
+                                 jac_diag=jac_diag, jacobian=jacobian)
     n = len(u0)
     u = _lib.DeviceArray.from_host(np.asarray(u0, np.float64))
     sol = ODESolution()
@@ -445,8 +448,10 @@ _TRB_K = (3 * _TRB_G ** 2 - 4 * _TRB_G + 2) / (6 * (2.0 - _TRB_G))
 
 
 def _integrate_trbdf2(rhs, jvp, u0, t0, tf, alg, *, saveat, abstol, reltol, dt, maxiters,
-                      save_start, step_callback, user_callback, op=None, jac_diag=None):
-    """jac_diag(u, t, out): the diagonal of J(u, t) on the device; with it, GMRES is
+                      save_start, step_callback, user_callback, op=None, jac_diag=None, jacobian=None):
+    """jacobian (implicit.FrozenJacobian): J taken at each step's start and every linear
+    system solved with it in one launch; otherwise GMRES on jvp, matrix-free.
+    jac_diag(u, t, out): the diagonal of J(u, t) on the device; with it, GMRES is
     right-preconditioned by diag(W)^-1, W = I - d h J frozen at the step's start (one
     diagonal per step, its inverse per step size)."""
     from .linsolve import gmres_device, library_arnoldi
@@ -502,6 +507,21 @@ def _integrate_trbdf2(rhs, jvp, u0, t0, tf, alg, *, saveat, abstol, reltol, dt, 
             pre["h"] = h
         return S
 
+    frozen = dict(t=None)
+
+    def solve_W(ubase, tbase, h, b, x):
+        """x = W^-1 b, W = I - d h J(ubase, tbase)."""
+        if jacobian is not None:
+            if frozen["t"] != tbase:
+                jacobian.take(ubase, tbase)
+                frozen["t"] = tbase
+            jacobian.solve(1.0, -_TRB_D * h, b, x, alg.krylov_rtol, alg.krylov_restart, 20 * alg.krylov_restart,
+                           alg.precond == "jacobi")
+            return
+        stats["nkrylov"] += gmres_device(W_apply(ubase, tbase, h), b, x, rtol=alg.krylov_rtol,
+                                         restart=alg.krylov_restart, maxiter=20 * alg.krylov_restart,
+                                         arnoldi=W_arnoldi(ubase, tbase, h), precond=precond(ubase, tbase, h))
+
     nl = dict(eta=1.0)  # Newton's contraction estimate theta / (1 - theta), kept between solves
 
     def newton(z, r, ts, ubase, tbase, h, fz):
@@ -509,16 +529,12 @@ def _integrate_trbdf2(rhs, jvp, u0, t0, tf, alg, *, saveat, abstol, reltol, dt, 
         Stops when eta |dz| <= kappa (Hairer & Wanner, Solving ODEs II, IV.8), eta
         starting from the previous solve's; returns False when Newton diverges or
         does not converge in max_newton iterations."""
-        A = W_apply(ubase, tbase, h)
         eta = ctrl_pow(max(nl["eta"], 1e-16), 0.8)
         prev = None
         for _ in range(alg.max_newton):
             f(z, fz, ts)
             _lib.lincomb(V["G"], (-1.0, _TRB_D * h, 1.0), (z, fz, r))  # -G = r + d h f(z) - z
-            stats["nkrylov"] += gmres_device(A, V["G"], V["dz"], rtol=alg.krylov_rtol,
-                                             restart=alg.krylov_restart, maxiter=20 * alg.krylov_restart,
-                                             arnoldi=W_arnoldi(ubase, tbase, h),
-                                             precond=precond(ubase, tbase, h))
+            solve_W(ubase, tbase, h, V["G"], V["dz"])
             _lib.lincomb(z, (1.0, 1.0), (z, V["dz"]))
             stats["nnewton"] += 1
             ndz = _lib.err_norm(V["dz"], ubase, z, abstol, reltol)
@@ -575,9 +591,7 @@ def _integrate_trbdf2(rhs, jvp, u0, t0, tf, alg, *, saveat, abstol, reltol, dt, 
         _lib.lincomb(est, (_TRB_K * h / _TRB_G, -_TRB_K * h / (_TRB_G * (1 - _TRB_G)),
                            _TRB_K * h / (1 - _TRB_G)), (fn, fg, f1))
         if alg.smooth_est:  # W^-1 est (Hosea & Shampine): keeps stiff components from inflating it
-            stats["nkrylov"] += gmres_device(W_apply(u, t, h), est, V["tmp"], rtol=alg.krylov_rtol,
-                                             restart=alg.krylov_restart, maxiter=20 * alg.krylov_restart,
-                                             arnoldi=W_arnoldi(u, t, h), precond=precond(u, t, h))
+            solve_W(u, t, h, est, V["tmp"])
             est = V["tmp"]
         EEst = _lib.err_norm(est, u, u1, abstol, reltol)
         if not math.isfinite(EEst):
@@ -611,6 +625,9 @@ def _integrate_trbdf2(rhs, jvp, u0, t0, tf, alg, *, saveat, abstol, reltol, dt, 
         dt = h * min(5.0, max(0.2, q))
     if sol.retcode == "Default":
         sol.retcode = "Success" if t >= tf else "MaxIters"
+    if jacobian is not None:
+        stats["nkrylov"] = jacobian.iterations()
+        stats["njvp"] = stats["nkrylov"]
     sol.stats = stats
     sol.final_device = u
     return sol

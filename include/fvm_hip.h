@@ -515,6 +515,27 @@ typedef struct fvm_trbdf2_stats {
 int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts* o, double* d_u, fvm_trbdf2_stats* st,
                       fvm_stream s);
 
+/* The Newton steps' linear systems of a nonlinear problem of at most 65536 unknowns
+ * (solve.jl:50-77, 167-183: there KLU on the Jacobian).
+ * fvm_jacobian_ell: J(u, t) in ELL form from one fvm_jvp per colour of a distance-2
+ * colouring of jacobian_sparsity's pattern: d_probes [n_colours] host array of device
+ * vectors (1 on the colour's columns), d_colour [(width + 1) n] the colour of each
+ * slot's column (255: padding) with the diagonal's in slot width, d_products
+ * [n_colours n] work.
+ * fvm_gmres_ell: x = (a I + b J)^-1 rhs by GMRES(restart <= 30) from x = 0 until
+ * |r| <= rtol |rhs|, right-preconditioned by the diagonal when jacobi != 0, in one
+ * launch; does not wait.  d_work: fvm_gmres_work_bytes(n) bytes, zeroed before its first
+ * use, for one call at a time.
+ * fvm_gmres_iterations: the iterations of all calls on d_work so far; waits, and fails
+ * if one of them did. */
+size_t fvm_gmres_work_bytes(int64_t n);
+int fvm_gmres_ell(const fvm_affine_op* J, double a, double b, int32_t jacobi, const double* d_rhs, double* d_x,
+                  double rtol, int32_t restart, int64_t maxiter, void* d_work, fvm_stream s);
+int fvm_gmres_iterations(const void* d_work, int64_t* iterations, fvm_stream s);
+int fvm_jacobian_ell(fvm_ctx* ctx, int32_t n_colours, const double* const* d_probes, const uint8_t* d_colour,
+                     int32_t width, const double* d_u, double t, double* d_products, double* d_val,
+                     double* d_diag, fvm_stream s);
+
 /* ---- explicit time integration (solve(::FVMProblem), solve.jl:133-220) -----
  * The whole adaptive or fixed-step integration of du/dt = f(u, t) in one call, f one
  * of the library's operators, with the Dirichlet update (dirichlet.jl:78-86) after

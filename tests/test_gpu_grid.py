@@ -46,3 +46,27 @@ def test_affine_trbdf2_matches_the_host_integrator(gpu, shape):
         assert np.max(np.abs(x - y)) <= 1e-7 * np.max(np.abs(y))
     again = FVM.solve(prob, FVM.TRBDF2(**opts), saveat=[0.02, 0.05])
     assert all(np.array_equal(x, y) for x, y in zip(a.u, again.u))  # sums in a fixed order
+
+
+@pytest.mark.parametrize("shape", [(5, 4), (16, 16), (61, 47), (131, 127), "wheel"], ids=str)
+def test_nonlinear_trbdf2_with_a_frozen_jacobian_matches_the_matrix_free_loop(gpu, shape):
+    """The same loop with each linear system solved in one launch on the extracted J
+    (fvm_jacobian_ell, fvm_gmres_ell) or matrix-free: a hub's wide rows keep the latter.
+    Tolerances as above."""
+    from finitevolumemethod import implicit
+
+    wheel = shape == "wheel"
+    tri = wheel_triangulation() if wheel else FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, *shape, jitter=0.2, seed=3)
+    mesh = FVM.FVMGeometry(tri)
+    u0 = 0.5 + 0.4 * np.sin(5 * tri.x) * np.cos(4 * tri.y)
+    prob = FVM.FVMProblem(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.2 * t + 0.0 * u, FVM.Neumann),
+                          diffusion_function=lambda x, y, t, u, p: 0.1 + u ** 2,
+                          source_function=lambda x, y, t, u, p: u * (1 - u), initial_condition=u0, final_time=0.02)
+    assert (implicit.FrozenJacobian.of(prob) is None) == wheel
+    opts = dict(newton_kappa=1e-7, krylov_rtol=1e-9)
+    a = FVM.solve(prob, FVM.TRBDF2(**opts), saveat=[0.01, 0.02])
+    b = FVM.solve(prob, FVM.TRBDF2(device_loop=False, **opts), saveat=[0.01, 0.02])
+    assert a.retcode == b.retcode == "Success"
+    assert a.stats["naccept"] == b.stats["naccept"] <= 50 and a.stats["nnewton"] > 0, (a.stats, b.stats)
+    for x, y in zip(a.u, b.u):
+        assert np.max(np.abs(x - y)) <= 1e-7 * np.max(np.abs(y))
