@@ -2,20 +2,24 @@
 // leaving the kernel: published vectors and grid-wide sums.
 //
 // Every 8-byte word carries 4 bytes of payload and the 4-byte number of its exchange,
-// so a reader polls the word itself until the number matches: a store and a load make
-// one exchange, with no flag, fence or cache write-back between them (a word is one
-// aligned 64-bit store, seen whole).  The words go through agent-scope relaxed
-// accesses, which every XCD's L2 passes on to memory.  Measured on MI355X: a sum over
-// the grid takes 1.35 us on one workgroup, 1.7 us on 4 to 40 and 1.8 us on 64 (a
-// counter barrier with the data stored beside it: 1.2, 1.5 to 2.1 and 2.3 us), where a
-// kernel boundary costs 2.6 us of launch and its own first loads.
+// so a reader polls the words themselves until the numbers match: a store and a load
+// make one exchange, with no flag, fence or cache write-back between them (each word is
+// one aligned 64-bit half of its access, seen whole).  The accesses are of agent scope,
+// which every XCD's L2 passes on to memory.  Measured on MI355X: a sum over the grid takes
+// 1.35 us on one workgroup, 1.7 us on 4 to 40, 1.8 us on 64 and 3.1 us on 256 (a counter
+// barrier with the data stored beside it: 1.2, 1.5 to 2.1, 2.3 and 4.8 us), where a kernel
+// boundary costs 2.6 us of launch and its own first loads.
 //
-// The buffers alternate between two halves by the exchange's parity.  A half is
-// written again only after a later sum, which no workgroup completes before every
-// workgroup has contributed, that is, has read all it needs from the exchanges before:
-// a kernel publishes at most two vectors between two sums.  Every workgroup adds the
-// contributions in the same order, so all of them hold the same sums bit for bit and
-// take the same branches.
+// The buffers alternate between two halves by the exchange's parity, so a half is
+// written again two exchanges later, when every reader must have been through it:
+//   sums: no workgroup completes the next one before every workgroup has contributed,
+//     that is, has read this one;
+//   vectors: a kernel publishes at most two of them between two sums, or the pattern of
+//     its gathers is symmetric (a row then publishes again only after it has read the
+//     next vector's entries from every row that reads its own, which those rows
+//     published after reading).
+// Every workgroup adds the contributions in the same order, so all of them hold the same
+// sums bit for bit and take the same branches.
 //
 // Polls are bounded: a workgroup that waits too long raises the grid's fault word,
 // which ends every other wait too, and the kernel returns with an error.
@@ -25,32 +29,40 @@
 namespace fvm {
 
 constexpr int kGridMaxSums = 32;    // values per grid-wide sum
-constexpr int kGridMaxWgs = 128;    // workgroups of a grid (two per lane in a sum)
+constexpr int kGridMaxWgs = 256;    // workgroups of a grid (four per lane in a sum)
 constexpr unsigned kGridSpin = 1u << 21;
 
 // Device memory of the exchanges of a grid of nwg workgroups over vectors of n:
 // header (words 0..7: next vector and sum numbers, fault, counters of the kernels),
 // then the vector's words, then the sums'.  Zeroed before its first use.
 enum { kGridVec = 0, kGridSum = 1, kGridFault = 2, kGridUser = 3, kGridHead = 8 };
-inline size_t grid_words(int64_t n) { return kGridHead + 4 * (size_t)n + 4 * (size_t)kGridMaxSums * kGridMaxWgs; }
+__host__ __device__ inline size_t grid_words(int64_t n) { return kGridHead + 4 * (size_t)n + 4 * (size_t)kGridMaxSums * kGridMaxWgs; }
 
-__device__ __forceinline__ void grid_store(uint64_t* p, uint64_t v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// The pair of words of one double, moved by one 16-byte access (half the requests of two
+// 8-byte ones; each word still carries its own number), through a buffer descriptor:
+// the base in scalar registers, a 32-bit offset per lane, agent scope.
+typedef uint32_t grid_pair __attribute__((ext_vector_type(4)));  // lo, number, hi, number
+constexpr int kAgentScope = 1 << 4;                   // cache policy: sc1
+constexpr int kVolatile = (int)(1u << 31);
+using grid_rsrc = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ grid_rsrc grid_view(uint64_t* mem, size_t words) {
+  return __builtin_amdgcn_make_buffer_rsrc(mem, 0, (int)(8 * words), 0x00027000);
 }
-__device__ __forceinline__ uint64_t grid_load(const uint64_t* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void grid_put(grid_rsrc m, uint32_t off, double x, uint32_t tag) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x);
+  const grid_pair p = {(uint32_t)u, tag, (uint32_t)(u >> 32), tag};
+  __builtin_amdgcn_raw_buffer_store_b128(p, m, (int)off, 0, kAgentScope | kVolatile);
 }
-__device__ __forceinline__ void grid_put(uint64_t* p, double x, uint32_t tag) {
-  const uint64_t u = (uint64_t)__double_as_longlong(x), t = (uint64_t)tag << 32;
-  grid_store(p, (u & 0xffffffffu) | t);
-  grid_store(p + 1, (u >> 32) | t);
+__device__ __forceinline__ grid_pair grid_get(grid_rsrc m, uint32_t off) {
+  return __builtin_amdgcn_raw_buffer_load_b128(m, (int)off, 0, kAgentScope | kVolatile);
 }
 // 0 when both words are of exchange tag
-__device__ __forceinline__ uint32_t grid_stale(uint64_t lo, uint64_t hi, uint32_t tag) {
-  return ((uint32_t)(lo >> 32) ^ tag) | ((uint32_t)(hi >> 32) ^ tag);
+__device__ __forceinline__ uint32_t grid_stale(grid_pair p, uint32_t tag) { return (p.y ^ tag) | (p.w ^ tag); }
+__device__ __forceinline__ double grid_value(grid_pair p) {
+  return __longlong_as_double((long long)((uint64_t)p.x | ((uint64_t)p.z << 32)));
 }
-__device__ __forceinline__ double grid_value(uint64_t lo, uint64_t hi) {
-  return __longlong_as_double((long long)((lo & 0xffffffffu) | (hi << 32)));
+__device__ __forceinline__ uint64_t grid_fault(const uint64_t* mem) {
+  return __hip_atomic_load(mem + kGridFault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Cross-lane moves of a double in vector registers (a shuffle through the LDS unit
@@ -123,6 +135,7 @@ struct GridShared {
 template <int T>
 struct Grid {
   uint64_t* mem;
+  grid_rsrc view;
   int64_t n;
   int nwg;
   uint32_t vtag, rtag;
@@ -130,6 +143,7 @@ struct Grid {
 
   __device__ __forceinline__ void open(uint64_t* m, int64_t n_, GridShared<T>* s) {
     mem = m;
+    view = grid_view(m, grid_words(n_));
     n = n_;
     nwg = (int)gridDim.x;
     sh = s;
@@ -146,50 +160,52 @@ struct Grid {
       mem[kGridSum] = rtag;
     }
   }
-  __device__ __forceinline__ uint64_t* vec() const { return mem + kGridHead + (vtag & 1 ? 2 * n : 0); }
-  __device__ __forceinline__ uint64_t* sums() const {
-    return mem + kGridHead + 4 * n + (rtag & 1 ? 2 * kGridMaxSums * kGridMaxWgs : 0);
+  // byte offsets of the halves in use
+  __device__ __forceinline__ uint32_t vec() const {
+    return 8u * kGridHead + (vtag & 1 ? 16u * (uint32_t)n : 0u);
+  }
+  __device__ __forceinline__ uint32_t sums() const {
+    return 8u * kGridHead + 32u * (uint32_t)n + (rtag & 1 ? 16u * kGridMaxSums * kGridMaxWgs : 0u);
   }
   __device__ __forceinline__ void give_up() {
-    grid_store(mem + kGridFault, 1);
+    __hip_atomic_store(mem + kGridFault, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     sh->fault = 1;
+  }
+  __device__ __forceinline__ bool waited_long(unsigned spin) const {
+    return spin > kGridSpin || (spin > 1000 && grid_fault(mem));
   }
 
   // x is entry i of the next published vector (active: this thread has an entry)
   __device__ __forceinline__ void publish(int64_t i, double x, bool active) {
     ++vtag;
-    if (active) grid_put(vec() + 2 * i, x, vtag);
+    if (active) grid_put(view, vec() + 16u * (uint32_t)i, x, vtag);
   }
   // the entries at off[0..K) (grid_offset) of the published vector, all loads in flight
-  // together, at 32-bit offsets from a base in scalar registers
+  // together
   template <int K>
   __device__ __forceinline__ void fetch(const uint32_t (&off)[K], double (&x)[K], bool active) {
-    const char* const v = (const char*)vec();
     if (!active) {
 #pragma unroll
       for (int s = 0; s < K; ++s) x[s] = 0.0;
       return;
     }
-    uint64_t lo[K], hi[K];
+    const uint32_t v = vec();
+    grid_pair p[K];
 #pragma nounroll
     for (unsigned spin = 0;; ++spin) {
       uint32_t stale = 0;
 #pragma unroll
-      for (int s = 0; s < K; ++s) {
-        const uint64_t* p = (const uint64_t*)(v + off[s]);
-        lo[s] = grid_load(p);
-        hi[s] = grid_load(p + 1);
-      }
+      for (int s = 0; s < K; ++s) p[s] = grid_get(view, v + off[s]);
 #pragma unroll
-      for (int s = 0; s < K; ++s) stale |= grid_stale(lo[s], hi[s], vtag);
+      for (int s = 0; s < K; ++s) stale |= grid_stale(p[s], vtag);
       if (stale == 0) break;
-      if (spin > kGridSpin || (spin > 1000 && grid_load(mem + kGridFault))) {
+      if (waited_long(spin)) {
         give_up();
         break;
       }
     }
 #pragma unroll
-    for (int s = 0; s < K; ++s) x[s] = grid_value(lo[s], hi[s]);
+    for (int s = 0; s < K; ++s) x[s] = grid_value(p[s]);
   }
   __device__ __forceinline__ double fetch1(int c) {
     const uint32_t off[1] = {grid_offset(c)};
@@ -214,46 +230,45 @@ struct Grid {
     }
     __syncthreads();
     ++rtag;
-    uint64_t* const P = sums();
+    const uint32_t P = sums();
     if ((int)threadIdx.x < k) {
       double s = 0.0;
 #pragma unroll
       for (int w = 0; w < NW; ++w) s += sh->red[w][threadIdx.x];
-      if (nwg > 1) grid_put(P + 2 * ((int64_t)threadIdx.x * kGridMaxWgs + blockIdx.x), s, rtag);
+      if (nwg > 1) grid_put(view, P + 16u * (threadIdx.x * kGridMaxWgs + blockIdx.x), s, rtag);
       else sh->tot[threadIdx.x] = s;
     }
     if (nwg > 1) {
-      // wave w collects sums w, w + NW, ..., kQ of them per round of polls: a round trip
-      // to memory each
-      constexpr int kQ = 4;
-      const bool one = lane < nwg, two = lane + 64 < nwg;
+      // wave w collects sums w, w + NW, ..., kQ of them per round of polls (a round trip
+      // to memory each), 64 workgroups' contributions per load
+      constexpr int kQ = 4, kG = kGridMaxWgs / 64;
       for (int q0 = wave; q0 < k; q0 += kQ * NW) {
         double x[kQ];
 #pragma nounroll
         for (unsigned spin = 0;; ++spin) {
-          uint64_t a[kQ], b[kQ], c[kQ], d[kQ];
+          grid_pair p[kQ][kG];
 #pragma unroll
           for (int r = 0; r < kQ; ++r) {
-            const bool on = q0 + r * NW < k;
-            const uint64_t* p = P + 2 * ((int64_t)(on ? q0 + r * NW : q0) * kGridMaxWgs + lane);
-            a[r] = b[r] = c[r] = d[r] = (uint64_t)rtag << 32;  // 0.0, arrived
-            if (on && one) {
-              a[r] = grid_load(p);
-              b[r] = grid_load(p + 1);
-            }
-            if (on && two) {
-              c[r] = grid_load(p + 128);
-              d[r] = grid_load(p + 129);
+            const uint32_t q = q0 + r * NW < k ? q0 + r * NW : q0;
+#pragma unroll
+            for (int g = 0; g < kG; ++g) {
+              p[r][g] = grid_pair{0u, rtag, 0u, rtag};  // 0.0, arrived
+              if (q0 + r * NW < k && lane + 64 * g < nwg)
+                p[r][g] = grid_get(view, P + 16u * (q * kGridMaxWgs + lane + 64 * g));
             }
           }
           uint32_t stale = 0;
 #pragma unroll
           for (int r = 0; r < kQ; ++r) {
-            stale |= grid_stale(a[r], b[r], rtag) | grid_stale(c[r], d[r], rtag);
-            x[r] = grid_value(a[r], b[r]) + grid_value(c[r], d[r]);
+            x[r] = 0.0;
+#pragma unroll
+            for (int g = 0; g < kG; ++g) {
+              stale |= grid_stale(p[r][g], rtag);
+              x[r] += grid_value(p[r][g]);
+            }
           }
           if (__all(stale == 0)) break;
-          if (spin > kGridSpin || (spin > 1000 && grid_load(mem + kGridFault))) {
+          if (waited_long(spin)) {
             if (lane == 0) give_up();
             break;
           }

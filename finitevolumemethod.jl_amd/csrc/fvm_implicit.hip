@@ -36,10 +36,7 @@ using fvm::GridShared;
 
 constexpr int kMaxRestart = 30;
 constexpr int64_t kMaxN = 65536;
-// Rows per workgroup: 256 up to 64 workgroups, then 512 (128 workgroups at most): a
-// grid-wide sum takes 1.8 us on 64 workgroups, 2.1 us on 128 and 3.1 us on 256.
-constexpr int kRowsS = 256, kRowsL = 512;
-constexpr int64_t kSmallN = 64 * kRowsS;
+constexpr int kRows = 256;  // rows per workgroup: 256 workgroups at most
 // One pass of classical Gram-Schmidt multiplies the basis's loss of orthogonality by
 // |w| / |w'| (the vector's length before and after it; Giraud, Langou, Rozloznik & van
 // den Eshof, Numer. Math. 101, 2005), so the loss is tracked and the pass repeated when
@@ -490,25 +487,23 @@ EllJ ell_of(const fvm_affine_op* op) {
   return J;
 }
 
-// Launches kernel<W, T> cooperatively for an operator of n rows and ELL width w, the
+// Launches kernel<W, kRows> cooperatively for an operator of n rows and ELL width w, the
 // widths of triangle meshes as compile-time constants, others at run time.
-#define FVM_TRB_LAUNCH(kernel, w, n, args, st)                                                                  \
-  ([&]() -> hipError_t {                                                                                       \
-    const bool big_ = (n) > kSmallN;                                                                           \
-    const unsigned t_ = big_ ? kRowsL : kRowsS, g_ = (unsigned)(((n) + t_ - 1) / t_);                          \
-    const void* f_ = nullptr;                                                                                  \
-    switch (w) {                                                                                               \
-      case 4: f_ = big_ ? (const void*)kernel<4, kRowsL> : (const void*)kernel<4, kRowsS>; break;               \
-      case 5: f_ = big_ ? (const void*)kernel<5, kRowsL> : (const void*)kernel<5, kRowsS>; break;               \
-      case 6: f_ = big_ ? (const void*)kernel<6, kRowsL> : (const void*)kernel<6, kRowsS>; break;               \
-      case 7: f_ = big_ ? (const void*)kernel<7, kRowsL> : (const void*)kernel<7, kRowsS>; break;               \
-      case 8: f_ = big_ ? (const void*)kernel<8, kRowsL> : (const void*)kernel<8, kRowsS>; break;               \
-      case 9: f_ = big_ ? (const void*)kernel<9, kRowsL> : (const void*)kernel<9, kRowsS>; break;               \
-      case 10: f_ = big_ ? (const void*)kernel<10, kRowsL> : (const void*)kernel<10, kRowsS>; break;            \
-      default: f_ = big_ ? (const void*)kernel<0, kRowsL> : (const void*)kernel<0, kRowsS>;                     \
-    }                                                                                                          \
-    void* p_[] = {&(args)};                                                                                    \
-    return hipLaunchCooperativeKernel(f_, dim3(g_), dim3(t_), p_, 0, (st));                                    \
+#define FVM_TRB_LAUNCH(kernel, w, n, args, st)                                                           \
+  ([&]() -> hipError_t {                                                                                \
+    const void* f_ = nullptr;                                                                           \
+    switch (w) {                                                                                        \
+      case 4: f_ = (const void*)kernel<4, kRows>; break;                                                \
+      case 5: f_ = (const void*)kernel<5, kRows>; break;                                                \
+      case 6: f_ = (const void*)kernel<6, kRows>; break;                                                \
+      case 7: f_ = (const void*)kernel<7, kRows>; break;                                                \
+      case 8: f_ = (const void*)kernel<8, kRows>; break;                                                \
+      case 9: f_ = (const void*)kernel<9, kRows>; break;                                                \
+      case 10: f_ = (const void*)kernel<10, kRows>; break;                                              \
+      default: f_ = (const void*)kernel<0, kRows>;                                                      \
+    }                                                                                                   \
+    void* p_[] = {&(args)};                                                                             \
+    return hipLaunchCooperativeKernel(f_, dim3((unsigned)(((n) + kRows - 1) / kRows)), dim3(kRows), p_, 0, (st)); \
   }())
 
 int check_op(const fvm_affine_op* op, const char* who) {

@@ -108,12 +108,11 @@ __device__ __forceinline__ int32_t find_directed_edge(const int32_t* __restrict_
 }
 
 
-// fvm_ode_solve's Tsit5 loop for a small ODE template in one workgroup
+// fvm_ode_solve's Tsit5 loop for a small ODE template in one launch
 // (fvm_linalg.hip); FVM_ERR_STATE when the template does not qualify.
-int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, double* const k[7], double* utmp,
-                         double* u, double* unew, double* d_u, double t0, double dt, int64_t it0, int64_t ks0,
-                         const double A[7][6], const double C[7], const double Bt[7], fvm_ode_stats* st,
-                         hipStream_t s);
+int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const double* k0, const double* u, double* d_u,
+                         double t0, double dt, int64_t it0, int64_t ks0, const double A[7][6], const double Bt[7],
+                         fvm_ode_stats* st, hipStream_t s);
 
 // Classical Gram-Schmidt applied twice to w against xs[0..k) (k <= 64) plus |w|^2,
 // intermediates on the device, one host synchronisation: h_host[0..k), h_host[k..2k)

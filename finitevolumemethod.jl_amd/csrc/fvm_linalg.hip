@@ -38,6 +38,7 @@
 #include <vector>
 
 #include "fvm_internal.hpp"
+#include "fvm_tsit5.hpp"
 
 using namespace fvm;
 
@@ -888,206 +889,6 @@ __global__ __launch_bounds__(kRT) void spmv_ell_kernel(int64_t n, SellIdx S, con
 }
 
 // ----------------------------------------------------------------------------
-// Tsit5 on a small ODE template in one workgroup
-// ----------------------------------------------------------------------------
-// The adaptive loop of fvm_ode_solve (fvm_ode.hip) for du/dt = A u + b when the
-// state is small: one workgroup of 1024 threads runs every step (stages, products
-// on the ELL copy of A, error norm, step control, saveat, first same as last) with
-// barriers between the phases, so the integration is one launch instead of ~13
-// launches and a host synchronisation per step.  Each element's arithmetic is the
-// multi-kernel path's: the same row products (sell_slice's order), the same linear
-// combinations (terms left to right), and the error norm's sum in the fixed order
-// of its 512-workgroup grid, emulated here block by block; the step controller's
-// power is fvm_ctrl.hpp's, the host loops' own: the same states bit for bit.
-constexpr int kSmallThreads = 1024;
-// One workgroup pays off below this many unknowns: a step costs about 16 us + 17 ns
-// per unknown on one CU (2,500 unknowns: 60 us; 10,000: 190 us) against about 80 us
-// for the launches of the multi-kernel step on the whole chip.
-constexpr int64_t kSmallTsit5Max = 3600;
-constexpr int kRedBlocksE = 512, kRedThreadsE = 256;  // the grid whose summation order is reproduced
-
-struct SmallTsit5 {
-  int64_t n;
-  SellIdx S;            // the sliced ELL copy of A
-  const int32_t* ecol;  // one of ecol / eoff
-  const int16_t* eoff;
-  const double* eval;
-  const double* diag;
-  const double* b;
-  double* k[7];  // the stages (k[0] = f(u) on entry)
-  double* utmp;
-  double* u;     // the state on entry
-  double* unew;
-  double* u_out;
-  double t0, tf, dt;
-  double abstol, reltol;
-  int64_t maxiters, it0;
-  int32_t fsal;
-  int64_t n_save, ks0;
-  const double* save_t;  // device copy
-  double* saves;
-  double* stats;  // [0] t, [1] naccept, [2] nreject, [3] nf, [4] nsaved, [5] retcode
-  double A[7][6], C[7], Bt[7];
-};
-
-// out = A x + b over the state, the workgroup's 16 waves taking the slices of the
-// sliced ELL copy in turn.
-template <int W, bool OFF>
-__device__ __forceinline__ void small_apply(const SmallTsit5& a, const double* x, double* out) {
-  const int64_t ns = (a.n + kSlice - 1) / kSlice;
-  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kSlice);
-  auto g = [&](int c) { return x[c]; };
-  auto body = [&](int64_t i, double, double acc) { out[i] = acc + a.b[i]; };
-  for (int64_t b = w; b < ns; b += kSmallThreads / kSlice) {
-    if (OFF)
-      sell_slice<false, W>(a.n, b, a.S, a.eoff, a.eval, a.diag, g, body);
-    else
-      sell_slice<false, W>(a.n, b, a.S, a.ecol, a.eval, a.diag, g, body);
-  }
-}
-
-// The pairwise tree of a 256-thread reduction, sh[t] += sh[t + s] for s = 128, ..., 1,
-// for each group of 256 threads of the workgroup at once: the two levels that pair
-// waves go through LDS, the six inside a wave through shuffles (lane l adds lane
-// l + s, the same pairs in the same order).  Thread 0 of each group returns its sum.
-__device__ __forceinline__ double tree256(double* sh, double x) {
-  const int tid = threadIdx.x, lt = tid % kRedThreadsE;
-  sh[tid] = x;
-  __syncthreads();
-  if (lt < 128) sh[tid] = sh[tid] + sh[tid + 128];
-  __syncthreads();
-  double v = 0.0;
-  if (lt < 64) {
-    v = sh[tid] + sh[tid + 64];
-    for (int s = 32; s > 0; s >>= 1) v += __shfl_down(v, s, 64);
-  }
-  __syncthreads();  // sh is free again
-  return v;
-}
-
-template <int W, bool OFF>
-__global__ __launch_bounds__(kSmallThreads) void tsit5_small_kernel(SmallTsit5 a) {
-  __shared__ double sh[kSmallThreads];
-  __shared__ double part[kRedBlocksE];
-  const int tid = threadIdx.x;
-  const int64_t n = a.n;
-  double* k[7];
-  for (int j = 0; j < 7; ++j) k[j] = a.k[j];
-  double* utmp = a.utmp;
-  double* u = a.u;
-  double* unew = a.unew;
-  double t = a.t0, dt = a.dt, qold = 1e-4;
-  int64_t it = a.it0, ks = a.ks0, naccept = 0, nreject = 0, nf = 0;
-  int retcode = FVM_ODE_SUCCESS;
-  const int nblk = (int)((n + kRedThreadsE - 1) / kRedThreadsE);  // nonempty blocks of the emulated grid
-  while (t < a.tf && it < a.maxiters) {
-    ++it;
-    dt = fmin(dt, a.tf - t);
-    for (int j = 1; j < 7; ++j) {
-      double c[7];
-      c[0] = 1.0;
-      for (int i = 0; i < j; ++i) c[i + 1] = dt * a.A[j][i];
-      double* dst = j == 6 ? unew : utmp;
-      for (int64_t e = tid; e < n; e += kSmallThreads) {
-        double v = c[0] * u[e];
-        for (int i = 0; i < j; ++i) v = v + c[i + 1] * k[i][e];
-        dst[e] = v;
-      }
-      __syncthreads();
-      small_apply<W, OFF>(a, dst, k[j]);
-      ++nf;
-      __syncthreads();
-    }
-    // the error norm: per element r = (sum_j dt bt_j k_j) / (abstol + reltol max(|u|, |unew|)),
-    // summed as the 512 x 256 grid of the multi-kernel path sums it
-    double cb[7];
-    for (int j = 0; j < 7; ++j) cb[j] = dt * a.Bt[j];
-    for (int b0 = 0; b0 < nblk; b0 += kSmallThreads / kRedThreadsE) {
-      const int blk = b0 + tid / kRedThreadsE, lt = tid % kRedThreadsE;
-      const int64_t e = (int64_t)blk * kRedThreadsE + lt;
-      double acc = 0.0;
-      if (blk < nblk && e < n) {
-        double v = cb[0] * k[0][e];
-        for (int j = 1; j < 7; ++j) v = v + cb[j] * k[j][e];
-        const double sc = a.abstol + a.reltol * fmax(fabs(u[e]), fabs(unew[e]));
-        const double r = v / sc;
-        acc += r * r;
-      }
-      acc = tree256(sh, acc);
-      if (lt == 0 && blk < nblk) part[blk] = acc;
-    }
-    for (int p = nblk + tid; p < kRedBlocksE; p += kSmallThreads) part[p] = 0.0;
-    __syncthreads();
-    double acc = 0.0;
-    if (tid < kRedThreadsE)
-      for (int i = tid; i < kRedBlocksE; i += kRedThreadsE) acc += part[i];
-    acc = tree256(sh, acc);
-    if (tid == 0) sh[0] = acc;
-    __syncthreads();
-    const double EEst = sqrt(sh[0] / (double)n);
-    __syncthreads();  // every thread has read sh[0]
-    if (!isfinite(EEst)) {
-      retcode = FVM_ODE_UNSTABLE;
-      break;
-    }
-    if (EEst <= 1.0) {
-      const double tn = t + dt;
-      while (ks < a.n_save && a.save_t[ks] <= tn + 1e-12 * fmax(1.0, fabs(tn))) {
-        const double th = fmin(1.0, fmax(0.0, (a.save_t[ks] - t) / dt));
-        const double t2 = th * th, t3 = t2 * th;
-        const double h00 = 2 * t3 - 3 * t2 + 1;
-        const double h10 = t3 - 2 * t2 + th;
-        const double h01 = -2 * t3 + 3 * t2;
-        const double h11 = t3 - t2;
-        const double c0 = h00, c1 = h10 * dt, c2 = h01, c3 = h11 * dt;
-        double* out = a.saves + ks * n;
-        for (int64_t e = tid; e < n; e += kSmallThreads) {
-          double v = c0 * u[e];
-          v = v + c1 * k[0][e];
-          v = v + c2 * unew[e];
-          v = v + c3 * k[6][e];
-          out[e] = v;
-        }
-        ++ks;
-      }
-      double* sw = u;
-      u = unew;
-      unew = sw;
-      t = tn;
-      ++naccept;
-      if (a.fsal) {
-        double* k0 = k[0];
-        k[0] = k[6];
-        k[6] = k0;
-      } else {
-        __syncthreads();
-        small_apply<W, OFF>(a, u, k[0]);
-        ++nf;
-      }
-      double q = fvm::ctrl_pow(fmax(EEst, 1e-16), 7.0 / 50.0) / fvm::ctrl_pow(qold, 2.0 / 25.0);
-      q = fmin(5.0, fmax(0.1, q / 0.9));
-      dt = dt / q;
-      qold = fmax(EEst, 1e-4);
-    } else {
-      ++nreject;
-      const double q = fmin(5.0, fvm::ctrl_pow(fmax(EEst, 1e-16), 7.0 / 50.0) / 0.9);
-      dt = dt / q;
-    }
-    __syncthreads();
-  }
-  if (retcode == FVM_ODE_SUCCESS && !(t >= a.tf)) retcode = FVM_ODE_MAXITERS;
-  for (int64_t e = tid; e < n; e += kSmallThreads) a.u_out[e] = u[e];
-  if (tid == 0) {
-    a.stats[0] = t;
-    a.stats[1] = (double)naccept;
-    a.stats[2] = (double)nreject;
-    a.stats[3] = (double)nf;
-    a.stats[4] = (double)ks;
-    a.stats[5] = (double)retcode;
-  }
-}
-
-// ----------------------------------------------------------------------------
 // host helpers
 // ----------------------------------------------------------------------------
 template <class T>
@@ -1785,27 +1586,32 @@ int fvm_template_solve(fvm_template* t, const fvm_solve_opts* o, double* d_x, fv
 namespace fvm {
 
 // The Tsit5 loop of fvm_ode_solve on the template's ELL copy of A in one launch
-// (tsit5_small_kernel), from time t0 with step dt, it0 steps and ks0 saves done,
-// k[0] = f(u) already computed; the final state goes to d_u.  Returns
-// FVM_ERR_STATE when the template has no ELL copy or n exceeds kSmallTsit5Max, so
+// (fvm_tsit5.hip), from time t0 with step dt, it0 steps and ks0 saves done,
+// k0 = f(u) already computed; the final state goes to d_u.  Returns
+// FVM_ERR_STATE when the template has no ELL copy or n exceeds kTsit5GridMax, so
 // that the caller keeps the multi-kernel loop.
-int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, double* const k[7], double* utmp,
-                         double* u, double* unew, double* d_u, double t0, double dt, int64_t it0, int64_t ks0,
-                         const double A[7][6], const double C[7], const double Bt[7], fvm_ode_stats* st,
-                         hipStream_t s) {
-  if (!t || t->ellW <= 0 || o->n != t->n || o->n > kSmallTsit5Max) return FVM_ERR_STATE;
+int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const double* k0, const double* u, double* d_u,
+                         double t0, double dt, int64_t it0, int64_t ks0, const double A[7][6], const double Bt[7],
+                         fvm_ode_stats* st, hipStream_t s) {
+  // (an assembled ODE template: its pattern is symmetric, as the grid form requires)
+  if (!t || t->kind != 2 || t->ellW <= 0 || o->n != t->n || o->n > kTsit5GridMax) return FVM_ERR_STATE;
+  // one workgroup while its registers hold the rows: 11 us a step at 2,500 rows, where
+  // the grid takes 14
+  const bool local = o->n <= tsit5_rows_local_max(t->ellW);
   SmallTsit5 a;
   a.n = o->n;
-  a.S = sell_idx(t);
+  a.W = t->ellW;
+  a.off = t->sl_off;
+  a.perm = t->sl_perm;
+  a.rem_ptr = t->sl_rem_ptr;
+  a.rem_off = t->sl_rem_off;
   a.ecol = t->ell_col;
   a.eoff = t->ell_off;
   a.eval = t->ellA;
   a.diag = t->diagA;
   a.b = t->b;
-  for (int j = 0; j < 7; ++j) a.k[j] = k[j];
-  a.utmp = utmp;
+  a.k0 = k0;
   a.u = u;
-  a.unew = unew;
   a.u_out = d_u;
   a.t0 = t0;
   a.tf = o->tf;
@@ -1820,38 +1626,36 @@ int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, double* c
   a.saves = o->d_saves;
   for (int j = 0; j < 7; ++j) {
     for (int i = 0; i < 6; ++i) a.A[j][i] = A[j][i];
-    a.C[j] = C[j];
     a.Bt[j] = Bt[j];
   }
-  double* dev = nullptr;  // save times, then 6 result slots
-  FVM_HIP(hipMalloc((void**)&dev, sizeof(double) * (size_t)(o->n_save + 6)));
-  a.save_t = dev;
-  a.stats = dev + o->n_save;
-  int rc = FVM_OK;
+  // exchange words of the grid form, save times, 6 result slots
+  const size_t words = local ? 0 : tsit5_rows_grid_words(o->n);
+  double* dev = nullptr;
+  FVM_HIP(hipMalloc((void**)&dev, sizeof(double) * (words + (size_t)o->n_save + 6)));
+  a.grid = (uint64_t*)dev;
+  a.save_t = dev + words;
+  a.stats = dev + words + o->n_save;
   hipError_t e = hipSuccess;
-  if (o->n_save > 0)
-    e = hipMemcpyAsync(dev, o->save_t, sizeof(double) * (size_t)o->n_save, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) {
-    by_width(t->ellW, [&](auto w) {
-      if (t->ell_off)
-        hipLaunchKernelGGL((tsit5_small_kernel<decltype(w)::value, true>), dim3(1), dim3(kSmallThreads), 0, s, a);
-      else
-        hipLaunchKernelGGL((tsit5_small_kernel<decltype(w)::value, false>), dim3(1), dim3(kSmallThreads), 0, s, a);
-    });
-    e = hipGetLastError();
-  }
+  if (words) e = hipMemsetAsync(dev, 0, sizeof(double) * words, s);
+  if (e == hipSuccess && o->n_save > 0)
+    e = hipMemcpyAsync(dev + words, o->save_t, sizeof(double) * (size_t)o->n_save, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = tsit5_rows(a, local, s);
   double r[6] = {0, 0, 0, 0, 0, 0};
   if (e == hipSuccess) e = hipMemcpyAsync(r, a.stats, sizeof r, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   (void)hipFree(dev);
-  if (e != hipSuccess) return hip_fail(e, "fvm_ode_solve (one-workgroup Tsit5)");
+  if (e != hipSuccess) return hip_fail(e, "fvm_ode_solve (one-launch Tsit5)");
+  if (r[5] < 0) {
+    set_error("fvm_ode_solve: the grid's exchange timed out");
+    return FVM_ERR_HIP;
+  }
   st->t = r[0];
   st->naccept += (int64_t)r[1];
   st->nreject += (int64_t)r[2];
   st->nf += (int64_t)r[3];
   st->nsaved = (int64_t)r[4];
   st->retcode = (int32_t)r[5];
-  return rc;
+  return FVM_OK;
 }
 
 }  // namespace fvm

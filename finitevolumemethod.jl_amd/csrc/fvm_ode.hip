@@ -140,9 +140,9 @@ int tsit5(const fvm_ode_opts* o, const Op& op, double* d_u, fvm_ode_stats* st, f
   int64_t it = 0;
   st->retcode = FVM_ODE_SUCCESS;
   if (op.kind == FVM_OP_TEMPLATE && !op.dirichlet) {
-    // small templates: the whole loop in one workgroup (same arithmetic per element)
-    rc = fvm::template_tsit5_small((const fvm_template*)op.h, o, k, utmp, u, unew, d_u, t, dt, it, ks, kA, kC, kBt,
-                                   st, (hipStream_t)s);
+    // small templates: the whole loop in one launch (same arithmetic per element)
+    rc = fvm::template_tsit5_small((const fvm_template*)op.h, o, k[0], u, d_u, t, dt, it, ks, kA, kBt, st,
+                                   (hipStream_t)s);
     if (rc != FVM_ERR_STATE) return rc;
     rc = FVM_OK;
   }

@@ -1,0 +1,42 @@
+// Arguments of the one-launch Tsit5 loop over a small ODE template (fvm_tsit5.hip).
+#pragma once
+#include "fvm_internal.hpp"
+
+namespace fvm {
+
+struct SmallTsit5 {
+  int64_t n;
+  // the sliced ELL copy of A (fvm_template): W unrolled slots, one of ecol / eoff
+  int W;
+  const int32_t* off;
+  const uint8_t* perm;
+  const int32_t* rem_ptr;
+  const int32_t* rem_off;
+  const int32_t* ecol;
+  const int16_t* eoff;
+  const double* eval;
+  const double* diag;
+  const double* b;
+  const double* k0;  // f(u) on entry
+  const double* u;   // the state on entry
+  double* u_out;
+  uint64_t* grid;    // the grid form's exchange memory, zeroed
+  double t0, tf, dt;
+  double abstol, reltol;
+  int64_t maxiters, it0;
+  int32_t fsal;
+  int64_t n_save, ks0;
+  const double* save_t;  // device copy
+  double* saves;
+  double* stats;  // [0] t, [1] naccept, [2] nreject, [3] nf, [4] nsaved, [5] retcode
+  double A[7][6], Bt[7];
+};
+
+constexpr int64_t kTsit5GridMax = 65536;  // rows of the grid form (256 workgroups of 256)
+// rows of the one-workgroup form for an ELL width, at most
+int64_t tsit5_rows_local_max(int W);
+// 8-byte words of exchange memory of the grid form
+size_t tsit5_rows_grid_words(int64_t n);
+hipError_t tsit5_rows(SmallTsit5& a, bool local, hipStream_t s);
+
+}  // namespace fvm

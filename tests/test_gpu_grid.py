@@ -70,3 +70,38 @@ def test_nonlinear_trbdf2_with_a_frozen_jacobian_matches_the_matrix_free_loop(gp
     assert a.stats["naccept"] == b.stats["naccept"] <= 50 and a.stats["nnewton"] > 0, (a.stats, b.stats)
     for x, y in zip(a.u, b.u):
         assert np.max(np.abs(x - y)) <= 1e-7 * np.max(np.abs(y))
+
+
+@pytest.mark.parametrize("shape", [(3, 3), (16, 16), (32, 32), (64, 40), (13, 197), (45, 46, 0.25), (64, 32, 0.25),
+                                   (90, 80, 0.25), (256, 256), (200, 190, "permuted"), "wheel"], ids=str)
+def test_one_launch_tsit5_is_the_host_loop_bit_for_bit(gpu, shape):
+    """A small ODE template's whole Tsit5 loop in one launch: one workgroup up to the rows
+    its registers hold (2,560 with up to 6 off-diagonals a row, 2,048 with more), a resident
+    grid up to 65,536, 16- and 32-bit columns, a hub's row of 40: every saved state, time
+    and counter equals the multi-kernel arithmetic of the host loop."""
+    from finitevolumemethod.solve import integrate
+    from test_gpu_templates import _permuted
+
+    if shape == "wheel":
+        tri = wheel_triangulation()
+    elif len(shape) == 2:
+        tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, *shape, single_boundary=True)
+    else:
+        tri = FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, *shape[:2], jitter=0.25, seed=5)
+        if shape[2] == "permuted":
+            tri = _permuted(tri, 2)
+    mesh = FVM.FVMGeometry(tri)
+    n = tri.num_points()
+    u0 = np.random.default_rng(n).random(n)
+    prob = FVM.DiffusionEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 1.5, FVM.Neumann),
+                                 diffusion_function=lambda x, y, p: 0.5 + x, initial_condition=u0,
+                                 final_time=25.0 / n)
+    ts = [0.0, 7.0 / n, 25.0 / n]
+    a = FVM.solve(prob, FVM.Tsit5(), saveat=ts)
+    p = prob.problem
+    if shape[-1] == "permuted":
+        assert p.ell_info(index_bytes=True)[2] == 4
+    b = integrate(lambda u, du, t: p.apply(u, du), prob._u0[:n], 0.0, 25.0 / n, FVM.Tsit5(), saveat=ts, fsal=True)
+    assert a.retcode == b.retcode == "Success" and a.stats == b.stats and a.stats["naccept"] > 3, (a.stats, b.stats)
+    for x, y in zip(a.u, b.u):
+        assert np.array_equal(x[:-1], y)
