@@ -27,6 +27,8 @@
 //                       recomputed in FP64 whenever it has dropped by inner_rtol
 //                       (default 0.1), keeping the search direction.
 //   FVM_SOLVE_BICGSTAB  FP64 BiCGStab on M with Jacobi right preconditioning.
+//   FVM_SOLVE_AUTO      FP64 CG preconditioned by a multigrid cycle (fvm_amg.hip), the
+//                       first method where that stops short.
 // Each reduction leaves one partial per workgroup, and every workgroup of the next
 // kernel re-adds all of them in the same fixed order, so solver scalars stay on the
 // device and results are bitwise reproducible; the host reads the scalars only
@@ -37,6 +39,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "fvm_amg.hpp"
 #include "fvm_internal.hpp"
 #include "fvm_tsit5.hpp"
 
@@ -51,6 +54,11 @@ constexpr int kRowsPerBlock = kRT / kLPR;
 constexpr int kRPG = FVM_SPMV_ROWS;      // rows per lane group per step of the SpMV loops
 constexpr int kEllMin = 4, kEllMax = 10; // unrolled slots of the sliced ELL form: the longest row's, in 4..10
 constexpr int kSlice = 64;               // rows per slice of the sliced ELL form: one wave
+// Unknowns from which FVM_SOLVE_AUTO uses the multigrid cycle: at 870 (30 x 29) a solve
+// takes 0.75 ms against 1.75 with Jacobi, the first one with the set-up 1.35; the set-up's
+// 0.6 ms outweighs the gain below about half of that.
+constexpr int64_t kAmgMin = 400;
+constexpr int kAmgMaxIter = 200;         // its iterations, before Jacobi-preconditioned CG takes over
 
 // solver scalars (device doubles)
 // (S_RZ, S_ALPHA, S_RHO and S_OMEGA take two slots each: value of an even / odd iteration)
@@ -107,6 +115,8 @@ struct fvm_template {
   float* diagM32 = nullptr;
   double* ellA = nullptr;      // the same entries of A itself (fvm_template_apply / _spmv)
   double* diagA = nullptr;
+  fvm::Amg* amg = nullptr;     // the multigrid hierarchy of M, built by the first solve that uses it
+  bool amg_tried = false;
 };
 
 namespace {
@@ -657,6 +667,144 @@ __global__ __launch_bounds__(kRT) void cg_update(int64_t n, int k, V* __restrict
 }
 
 // ----------------------------------------------------------------------------
+// CG on M preconditioned by a multigrid cycle (fvm_amg.hip), FP64
+// ----------------------------------------------------------------------------
+// Flexible CG: beta_k = z_k.(r_k - r_{k-1}) / (z_{k-1}.r_{k-1}) = -alpha_{k-1} z_k.q_{k-1}
+// / rz_{k-1}, since M, and with it the cycle, is only close to symmetric.  An iteration
+// is pcg_down (stop test, Q^T r), the cycle below the first level, pcg_up (z, r.z, q.z),
+// pcg_dir (p, q = M p, p.q), pcg_update (x, r, |r|_A^2).
+
+// partials of |r|_A^2
+__global__ __launch_bounds__(kRT) void pcg_start(int64_t n, const double* __restrict__ r,
+                                                 const double* __restrict__ wv, double* sc, double* part) {
+  double wr = 0.0;
+  for (int64_t i = solver_wid() * kRT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRT) {
+    const double w = r[i] * wv[i];
+    wr += w * w;
+  }
+  store_partial(wr, part + PT_WR * kMaxG);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc[S_DONE] = 0.0;
+    sc[S_FLAG] = 0.0;
+    sc[S_ITER] = 0.0;
+  }
+}
+
+// stop test on |r|_A^2; out = Q^T r, kLPR lanes per coarse row
+__global__ __launch_bounds__(kRT) void pcg_down(int64_t nc, int k, double tabs2, const int32_t* __restrict__ qtp,
+                                                const int32_t* __restrict__ qti, const float* __restrict__ qtv,
+                                                const double* __restrict__ r, double* __restrict__ out, double* sc,
+                                                const double* part) {
+  if (wg_done(sc)) return;
+  const double wr = total_of(part + PT_WR * kMaxG);
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  if (lead) sc[S_WR] = wr;
+  if (!(wr > tabs2)) {
+    if (lead) {
+      sc[S_DONE] = 1.0;
+      sc[S_ITER] = (double)k;
+    }
+    return;
+  }
+  const int lane = threadIdx.x % kLPR;
+  for (int64_t c = solver_wid() * kRowsPerBlock + threadIdx.x / kLPR; c < nc;
+       c += (int64_t)gridDim.x * kRowsPerBlock) {
+    const int k1 = qtp[c + 1];
+    double v = 0.0;
+    for (int e = qtp[c] + lane; e < k1; e += kLPR) v += (double)qtv[e] * r[qti[e]];
+    v = group_sum(v);
+    if (lane == 0) out[c] = v;
+  }
+}
+
+// z = S (2 r - M S r) + Q e; partials of r.z and, with the last product q, of q.z
+template <int W, class CI>
+__global__ __launch_bounds__(kRT) void pcg_up(int64_t n, SellIdx S, const CI* __restrict__ ecol,
+                                              const double* __restrict__ eval, const double* __restrict__ diag,
+                                              const double* __restrict__ sw, const uint8_t* __restrict__ qcnt,
+                                              const int32_t* __restrict__ qcol, const float* __restrict__ qv,
+                                              const double* __restrict__ e, const double* __restrict__ r,
+                                              const double* __restrict__ q, double* __restrict__ z, const double* sc,
+                                              double* part) {
+  if (wg_done(sc)) return;
+  double rz = 0.0, qz = 0.0;
+  sell_rows<false, W>(n, S, ecol, eval, diag, [&](int c) { return sw[c] * r[c]; },
+                     [&](int64_t i, double, double ax) {
+                       const double ri = r[i];
+                       double v = sw[i] * (2.0 * ri - ax);
+                       const int m = qcnt[i];
+                       for (int k = 0; k < m; ++k) v += (double)qv[k * n + i] * e[qcol[k * n + i]];
+                       z[i] = v;
+                       rz += ri * v;
+                       qz += q[i] * v;
+                     });
+  store_partial(rz, part + PT_RZ * kMaxG);
+  store_partial(qz, part + PT_TT * kMaxG);
+}
+
+// beta; p = z + beta p_old; q = M p; partials of p.q
+template <int W, class CI>
+__global__ __launch_bounds__(kRT) void pcg_dir(int64_t n, int k, SellIdx S, const CI* __restrict__ ecol,
+                                               const double* __restrict__ eval, const double* __restrict__ diag,
+                                               const double* __restrict__ z, const double* __restrict__ pold,
+                                               double* __restrict__ pnew, double* __restrict__ q, double* sc,
+                                               double* part) {
+  if (wg_done(sc)) return;
+  const double rz = total_of(part + PT_RZ * kMaxG);
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  if (!(rz > 0.0)) {  // the cycle is not positive definite on this residual: stop
+    if (lead) {
+      sc[S_FLAG] = 2.0;
+      sc[S_DONE] = 1.0;
+      sc[S_ITER] = (double)k;
+    }
+    return;
+  }
+  double beta = 0.0;
+  if (k > 0) beta = -sc[S_ALPHA + ((k - 1) & 1)] * total_of(part + PT_TT * kMaxG) / sc[S_RZ + ((k - 1) & 1)];
+  if (lead) sc[S_RZ + (k & 1)] = rz;
+  double pq = 0.0;
+  auto dir = [&](int c) { return k > 0 ? z[c] + beta * pold[c] : z[c]; };
+  sell_rows<false, W>(n, S, ecol, eval, diag, dir, [&](int64_t i, double pi, double qi) {
+    pnew[i] = pi;
+    q[i] = qi;
+    pq += pi * qi;
+  });
+  store_partial(pq, part + PT_PQ * kMaxG);
+}
+
+// alpha = rz / p.q; x += alpha p; r -= alpha q; partials of |r|_A^2
+__global__ __launch_bounds__(kRT) void pcg_update(int64_t n, int k, double* __restrict__ x, double* __restrict__ r,
+                                                  const double* __restrict__ p, const double* __restrict__ q,
+                                                  const double* __restrict__ wv, double* sc, double* part) {
+  if (wg_done(sc)) return;
+  const double pq = total_of(part + PT_PQ * kMaxG);
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  if (!(pq > 0.0)) {  // M is not positive definite on this direction: stop
+    if (lead) {
+      sc[S_FLAG] = 2.0;
+      sc[S_DONE] = 1.0;
+      sc[S_ITER] = (double)k;
+    }
+    return;
+  }
+  const double alpha = sc[S_RZ + (k & 1)] / pq;
+  double wr = 0.0;
+  for (int64_t i = solver_wid() * kRT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kRT) {
+    x[i] = x[i] + alpha * p[i];
+    const double ri = r[i] - alpha * q[i];
+    r[i] = ri;
+    const double w = ri * wv[i];
+    wr += w * w;
+  }
+  store_partial(wr, part + PT_WR * kMaxG);
+  if (lead) {
+    sc[S_ALPHA + (k & 1)] = alpha;
+    sc[S_ITER] = (double)(k + 1);
+  }
+}
+
+// ----------------------------------------------------------------------------
 // BiCGStab on M, FP64, Jacobi right preconditioning
 // ----------------------------------------------------------------------------
 // d = 0, rhat = r, p = v = 0; partials of rhat.r and |r|_A^2
@@ -914,6 +1062,7 @@ void free_tmpl(fvm_template* t) {
                t->diagA};
   for (void* q : p)
     if (q) (void)hipFree(q);
+  delete t->amg;
   delete t;
 }
 
@@ -1221,6 +1370,43 @@ int reliable_cg(fvm_template* t, double* x, double target, double delta, int max
   return FVM_OK;
 }
 
+// CG on M with the multigrid cycle, x updated in place, from r = -V (b - A x): until
+// |r|_A <= sqrt(tabs2), a breakdown or maxit iterations.
+constexpr int kPcgCheck = 4;  // iterations between the host's reads of the solver scalars
+int amg_cg(fvm_template* t, double* x, double tabs2, int maxit, hipStream_t s, int* iters, int* flag) {
+  const int64_t n = t->n;
+  double* w = t->work;
+  double *r = w + n, *z = w + 2 * n, *q = w + 5 * n;
+  double* pp[2] = {w + 3 * n, w + 4 * n};
+  const AmgLevel &L = t->amg->level[0], &C = t->amg->level[1];
+  const double* done = t->sc + S_DONE;
+  hipLaunchKernelGGL(pcg_start, grid(t), dim3(kRT), 0, s, n, r, t->wv, t->sc, t->part);
+  double h[S_COUNT];
+  for (int k = 0;;) {
+    const int batch = std::min(kPcgCheck, maxit - k);
+    for (int j = 0; j < batch; ++j, ++k) {
+      hipLaunchKernelGGL(pcg_down, grid(t), dim3(kRT), 0, s, L.nc, k, tabs2, L.qtp, L.qti, L.qtv, r, C.b, t->sc,
+                         t->part);
+      amg_coarse(t->amg, done, s);
+      by_ell(t, [&](auto wd, auto ec) {
+        constexpr int W = decltype(wd)::value;
+        using CI = ci_t<decltype(ec)>;
+        hipLaunchKernelGGL((pcg_up<W, CI>), grid(t), dim3(kRT), 0, s, n, sell_idx(t), ec, t->ellM, t->diagM, L.s,
+                           L.qcnt, L.qcol, L.qv, C.x, r, k > 0 ? q : r, z, t->sc, t->part);
+        hipLaunchKernelGGL((pcg_dir<W, CI>), grid(t), dim3(kRT), 0, s, n, k, sell_idx(t), ec, t->ellM, t->diagM, z,
+                           pp[k & 1], pp[(k + 1) & 1], q, t->sc, t->part);
+      });
+      hipLaunchKernelGGL(pcg_update, grid(t), dim3(kRT), 0, s, n, k, x, r, pp[(k + 1) & 1], q, t->wv, t->sc, t->part);
+    }
+    const int rc = read_scalars(t, h, s);
+    if (rc) return rc;
+    if (h[S_DONE] != 0.0 || k >= maxit) break;
+  }
+  *iters = (int)h[S_ITER];
+  *flag = (int)h[S_FLAG];
+  return FVM_OK;
+}
+
 int inner_bicgstab(fvm_template* t, double* d, double* r, double tabs2, int maxit, int check, hipStream_t s,
                    int* iters, int* flag) {
   const int64_t n = t->n;
@@ -1515,7 +1701,7 @@ int fvm_template_residual(fvm_template* t, const double* d_x, double* rel, fvm_s
 int fvm_template_solve(fvm_template* t, const fvm_solve_opts* o, double* d_x, fvm_solve_stats* st,
                        fvm_stream s) {
   FVM_CHECK(t && o && d_x && st, "fvm_template_solve: null argument");
-  FVM_CHECK(o->method >= 0 && o->method <= 3, "fvm_template_solve: unknown method");
+  FVM_CHECK(o->method >= 0 && o->method <= FVM_SOLVE_AUTO, "fvm_template_solve: unknown method");
   FVM_CHECK(o->rtol > 0 && o->maxiter > 0, "fvm_template_solve: rtol and maxiter must be positive");
   FVM_CHECK(t->kind != 2, "fvm_template_solve: a diffusion template is an ODE, not a linear system");
   FVM_CHECK(o->spmv_format >= FVM_SPMV_AUTO && o->spmv_format <= FVM_SPMV_ELL,
@@ -1542,6 +1728,34 @@ int fvm_template_solve(fvm_template* t, const fvm_solve_opts* o, double* d_x, fv
   // the recursive residual must reach half the target before the true residual is checked
   const double tabs2 = 0.25 * target * target;
   int total = 0, outer = 0, flag = 0;
+  const int method = o->method == FVM_SOLVE_AUTO ? (int)FVM_SOLVE_CG : o->method;
+  if (o->method == FVM_SOLVE_AUTO && t->use_ell && n >= kAmgMin && res > target) {
+    if (!t->amg_tried) {
+      t->amg_tried = true;
+      rc = amg_build(n, t->row_ptr, t->col, t->valM, &t->amg, str);
+      if (rc == FVM_ERR_ALLOC) rc = FVM_OK;  // no room for the hierarchy: Jacobi-preconditioned
+      if (rc) return rc;
+    }
+    // Jacobi-preconditioned CG finishes what a breakdown or slow convergence leaves
+    int left = std::min(o->maxiter, kAmgMaxIter);
+    while (t->amg && res > target && left > 0 && outer < max_outer && !flag) {
+      int it = 0;
+      rc = amg_cg(t, d_x, tabs2, left, str, &it, &flag);
+      if (rc || (rc = true_res<double>(t, d_x, r, str)) || (rc = read_scalars(t, h, str))) return rc;
+      total += it;
+      left -= it;
+      ++outer;
+      res = std::sqrt(h[S_RES2]);
+      if (!(res == res) || it == 0) break;
+    }
+    if (!(res == res)) {  // a diverged cycle: start over
+      hipLaunchKernelGGL(init_x, grid(t), dim3(kRT), 0, str, n, t->fixed, t->b, d_x, 0);
+      if ((rc = true_res<double>(t, d_x, r, str)) || (rc = read_scalars(t, h, str))) return rc;
+      res = std::sqrt(h[S_RES2]);
+    }
+    flag = res <= target ? flag : 0;
+    outer = 0;
+  }
   if (o->method == FVM_SOLVE_CG_RELIABLE && res > target) {
     const double delta = o->inner_rtol > 0 ? o->inner_rtol : 0.1;
     rc = reliable_cg(t, d_x, target, delta, o->maxiter, o->max_outer > 0 ? o->max_outer : 1000, check, str,
@@ -1550,14 +1764,14 @@ int fvm_template_solve(fvm_template* t, const fvm_solve_opts* o, double* d_x, fv
   }
   while (o->method != FVM_SOLVE_CG_RELIABLE && res > target && total < o->maxiter && outer < max_outer) {
     int it = 0;
-    if (o->method == 1) {
+    if (method == 1) {
       rc = inner_cg<float>(t, t->valM32, t->dinv32, t->wv32, df, rf, zf, p0f, p1f, qf, irt * irt, tabs2,
                            o->maxiter - total, check, str, &it, &flag);
       if (rc) return rc;
       hipLaunchKernelGGL((add_correction<float>), grid(t), dim3(kRT), 0, str, n, df, d_x);
       rc = true_res<float>(t, d_x, rf, str);
     } else {
-      if (o->method == 0)
+      if (method == 0)
         rc = inner_cg<double>(t, t->valM, t->dinv, t->wv, d, r, z, p0, p1, q, 0.0, tabs2, o->maxiter - total,
                               check, str, &it, &flag);
       else

@@ -124,7 +124,7 @@ class SystemDesc(ctypes.Structure):
 
 FLUX_D_POLY_U, FLUX_D_NODAL, FLUX_D_EDGE, FLUX_LINEAR, FLUX_D_POWER, FLUX_JIT = 0, 1, 2, 3, 4, 5
 TEMPLATE_POISSON, TEMPLATE_MEAN_EXIT_TIME, TEMPLATE_DIFFUSION = 0, 1, 2
-SOLVE_CG, SOLVE_CG_MIXED, SOLVE_BICGSTAB, SOLVE_CG_RELIABLE = 0, 1, 2, 3
+SOLVE_CG, SOLVE_CG_MIXED, SOLVE_BICGSTAB, SOLVE_CG_RELIABLE, SOLVE_AUTO = 0, 1, 2, 3, 4
 NODE_NONE, NODE_DIRICHLET, NODE_DUDT = 0, 1, 2
 
 _lock = threading.Lock()

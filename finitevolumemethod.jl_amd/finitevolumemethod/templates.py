@@ -4,9 +4,9 @@ the GPU.
 PoissonsEquation, LaplacesEquation and MeanExitTimeProblem are steady linear
 systems A u = b (the reference hands LinearProblem(sparse(A), b) to LinearSolve);
 here A and b are assembled by fvm_template_create in the CSR pattern of
-jacobian_sparsity and solved by fvm_template_solve (Jacobi-preconditioned CG on
-the volume-scaled operator, FP64 or FP32-inner iterative refinement, or
-BiCGStab).  DiffusionEquation and LinearReactionDiffusionEquation are linear ODEs
+jacobian_sparsity and solved by fvm_template_solve (CG on the volume-scaled
+operator, preconditioned by multigrid (the default) or Jacobi, FP64 or FP32-inner
+iterative refinement, or BiCGStab).  DiffusionEquation and LinearReactionDiffusionEquation are linear ODEs
 du/dt = A u + b (the reference's MatrixOperator of the augmented [A b; 0 0]
 system) integrated on the device with fvm_template_apply as the right-hand side.
 
@@ -224,8 +224,11 @@ class DeviceTemplate:
 
     def solve(self, alg=None, *, rtol=1e-10, maxiter=100000, x=None, max_outer=0, stream=None, spmv_format="auto"):
         """Solve A x = b on the device.  Returns (x DeviceArray, fvm_solve_stats dict).
+        alg: CG(), MixedCG() or BiCGStab(); by default FP64 CG with the library's choice of
+        preconditioner (multigrid, or Jacobi as CG(); FVM_SOLVE_AUTO).
         spmv_format: the form of the scaled operator in the CG direction kernel,
-        "auto" (= "ell"), "ell" or "csr"."""
+        "auto" (= "ell"), "ell" or "csr" (the latter two: Jacobi-preconditioned)."""
+        auto = alg is None and spmv_format == "auto"
         alg = alg if alg is not None else CG()
         if type(alg) not in _METHOD:
             raise TypeError(f"unsupported linear solver {alg!r}; use CG(), MixedCG() or BiCGStab()")
@@ -233,6 +236,8 @@ class DeviceTemplate:
         o.method = _METHOD[type(alg)]
         if isinstance(alg, MixedCG) and alg.update == "reliable":
             o.method = _lib.SOLVE_CG_RELIABLE
+        if auto:
+            o.method = _lib.SOLVE_AUTO
         o.maxiter = int(maxiter)
         o.check_every = int(alg.check_every)
         o.max_outer = int(max_outer)

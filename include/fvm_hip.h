@@ -286,7 +286,10 @@ enum {
   FVM_SOLVE_CG = 0,       /* FP64 Jacobi-PCG on M */
   FVM_SOLVE_CG_MIXED = 1, /* FP64 iterative refinement around FP32 Jacobi-PCG on M */
   FVM_SOLVE_BICGSTAB = 2, /* FP64 Jacobi-BiCGStab on M */
-  FVM_SOLVE_CG_RELIABLE = 3 /* one FP32 Jacobi-PCG sequence with FP64 reliable updates of x and the residual */
+  FVM_SOLVE_CG_RELIABLE = 3, /* one FP32 Jacobi-PCG sequence with FP64 reliable updates of x and the residual */
+  FVM_SOLVE_AUTO = 4      /* FP64 CG on M preconditioned by smoothed-aggregation multigrid (set up by the first
+                             such solve and kept), FVM_SOLVE_CG for small systems and where that breaks down
+                             or converges slowly */
 };
 
 /* Forms of the scaled operator M in the Krylov products: CSR with eight lanes per row, or an ELL

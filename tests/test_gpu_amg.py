@@ -1,0 +1,79 @@
+"""The steady templates' default solver (FVM_SOLVE_AUTO): CG preconditioned by the
+smoothed-aggregation multigrid of fvm_amg.hip, against SuperLU on the same A and b.
+
+Both stop at |b - A x| <= 1e-10 |b|; the solutions then differ by at most
+|A^-1| 1e-10 |b|, measured here as 1e-10 |b| times the norm of A^-1 (power iteration on
+the factorisation), and the same call twice gives the same bits."""
+import numpy as np
+import pytest
+import scipy.sparse.linalg as spla
+
+import finitevolumemethod as FVM
+
+pytestmark = pytest.mark.gpu
+
+
+def _hub(k=300):
+    """A node with k neighbours inside rings of k, k and 60 points: rows longer than the
+    strength mask, transposed lists longer than the sorting network."""
+    pts = [(0.0, 0.0)]
+    for m, r, ph in ((k, 1.0, 0.0), (k, 1.03, 0.5), (60, 1.6, 0.2)):
+        th = 2 * np.pi * (np.arange(m) + ph) / m
+        pts += list(zip(r * np.cos(th), r * np.sin(th)))
+    P = np.array(pts)
+    return FVM.triangulate(P[:, 0], P[:, 1])
+
+
+def _mesh(kind):
+    if kind == "hub":
+        return _hub()
+    if kind == "stretched":  # triangles 30 times longer than wide
+        return FVM.jittered_rectangle(0.0, 30.0, 0.0, 1.0, 41, 43, jitter=0.2, seed=4, single_boundary=False)
+    if kind == "graded":
+        t = FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, 71, 67, jitter=0.2, seed=4, single_boundary=False)
+        return FVM.Triangulation(t.x * (0.1 + 0.9 * t.x), t.y * (0.3 + 0.7 * t.y), t.triangles, t.boundary_edges, t.boundary_segments)
+    nx, ny = kind
+    return FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, nx, ny, jitter=0.25, seed=11, single_boundary=False)
+
+
+# (19, 21) is below the smallest system, (20, 20) the smallest: one coarse level; (33, 32)
+# just over a tail level of 128 rows; (200, 170) four levels
+@pytest.mark.parametrize("kind", [(19, 21), (20, 20), (33, 32), (200, 170), "stretched", "graded", "hub"], ids=str)
+@pytest.mark.parametrize("D", ["one", "varying"])
+def test_default_steady_solve_matches_a_direct_solution(gpu, kind, D):
+    tri = _mesh(kind)
+    mesh = FVM.FVMGeometry(tri)
+    segs = tri.num_boundary_segments()
+    zero = lambda x, y, t, u, p: 0.0 * x  # noqa: E731
+    types = tuple(FVM.Dirichlet if k % 2 == 0 else FVM.Neumann for k in range(segs))
+    Dfun = (lambda x, y, p: 1.0 + 0.0 * x) if D == "one" else (lambda x, y, p: np.exp(1.5 * np.sin(3 * x / tri.x.max()) * np.cos(4 * y)))
+    f = np.random.default_rng(3).uniform(-1, 1, tri.num_points())
+    prob = FVM.PoissonsEquation(mesh, FVM.BoundaryConditions(mesh, (zero,) * segs, types),
+                                FVM.InternalConditions(lambda x, y, t, u, p: 1.0 + 0.0 * x, dirichlet_nodes={7: 0}),
+                                diffusion_function=Dfun, source_function=lambda x, y, p: p, source_parameters=f)
+    a = FVM.solve(prob)
+    assert a.retcode == "Success" and a.resid <= 1e-10, a.stats
+    A, b = prob.A.tocsc(), prob.b
+    lu = spla.splu(A)
+    v = np.random.default_rng(1).standard_normal(len(b))
+    for _ in range(20):  # |A^-1|_2
+        v /= np.linalg.norm(v)
+        v = lu.solve(lu.solve(v), trans="T")
+    bound = 1.1 * np.sqrt(np.linalg.norm(v)) * 1e-10 * np.linalg.norm(b)
+    x = lu.solve(b)
+    assert np.linalg.norm(a.u - x) <= bound + 1e-12 * np.linalg.norm(x)
+    if len(b) >= 400 and kind not in ("stretched", "graded", "hub"):
+        assert a.iters <= 60, a.stats  # Jacobi-preconditioned CG: over 100 from 33 x 32 on
+    assert np.array_equal(FVM.solve(prob).u, a.u)
+
+
+def test_a_singular_system_ends_as_it_does_with_jacobi(gpu):
+    """Zero flux everywhere and a source that does not sum to zero: no solution."""
+    tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 30, 30, single_boundary=True)
+    mesh = FVM.FVMGeometry(tri)
+    prob = FVM.PoissonsEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.0 * x, FVM.Neumann),
+                                source_function=lambda x, y, p: 1.0 + 0.0 * x)
+    from finitevolumemethod import CG
+
+    a, b = FVM.solve(prob, maxiter=500), FVM.solve(prob, CG(), maxiter=500)
+    assert a.retcode == b.retcode == "MaxIters" and np.all(np.isfinite(a.u))
