@@ -121,6 +121,9 @@ int cgs2_norm(int64_t n, int k, const double* const* xs, double* w, double* h_ho
 
 }  // namespace fvm
 
+// Nodes of the meshes that keep node_kernel's lists, at most (see launch_fk).
+constexpr int64_t kNodeMeshMax = 40000;
+
 // Device-resident mesh: geometry SoA in tile (sorted) triangle order plus the
 // tile / fix-up structures from fvmh_tiles_build.
 struct fvm_mesh {
@@ -142,6 +145,12 @@ struct fvm_mesh {
   int32_t* perm = nullptr;                      // sorted -> input triangle
   uint8_t* is_vertex = nullptr;
   double* lcv = nullptr;            // [n_local] control volume of each local-node entry
+  // per-node incidences of the one-launch RHS of small meshes (node_kernel), null on
+  // meshes above kNodeMeshMax
+  int4* node_ent = nullptr;         // [blocks][8]: the triangle's vertices, sorted triangle << 3 |
+                                    // first of another tile << 2 | slot (-1: padding)
+  int32_t* node_next = nullptr;     // [blocks] the node's next block, -1: none
+  int32_t* node_bed = nullptr;      // [N] boundary items: first << 8 | count
   int32_t* qflag = nullptr;         // device flag of the pointwise queries (run_flagged)
   bool convex = false;              // one boundary loop that turns left (or goes straight) at
                                     // every vertex: a point outside a boundary edge is outside

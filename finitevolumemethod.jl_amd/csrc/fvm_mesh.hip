@@ -132,7 +132,8 @@ void free_mesh(fvm_mesh* m) {
                   m->tile_nodes, m->loc, m->inc_start, m->inc, m->part_idx, m->fix_nodes,
                   m->fix_part_start, m->fix_bedge_start, m->fix_bedge, m->fix_bvert_start,
                   m->fix_bvert, m->lcv, m->node_tri_start,
-                  m->node_tri, m->bedges, m->badj, m->perm, m->is_vertex, m->qflag};
+                  m->node_tri, m->bedges, m->badj, m->perm, m->is_vertex, m->qflag,
+                  m->node_ent, m->node_next, m->node_bed};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete m;
@@ -174,6 +175,46 @@ bool convex_domain(const fvm_mesh_desc* d) {
   for (int64_t i = 0; i < N; ++i) nv += isv[i];
   const int64_t E = (3 * T + B) / 2;  // every interior edge in two triangles, boundary edges in one
   return (3 * T + B) % 2 == 0 && nv - E + T == 1;
+}
+
+// The per-node incidences of node_kernel: blocks of eight in ascending triangle order, a
+// node's first block its own index, further ones after all nodes'.
+int node_lists(const fvmh_tiles* tl, fvm_mesh* m) {
+  const int64_t N = m->N, T = m->T;
+  constexpr int L = 8;
+  std::vector<int32_t> tile_of(T), next(N, -1), bed(N, 0);
+  for (int32_t k = 0; k < m->n_tiles; ++k)
+    for (int32_t s = tl->tile_tri_start[k]; s < tl->tile_tri_start[k + 1]; ++s) tile_of[s] = k;
+  std::vector<int4> ent((size_t)N * L);
+  for (int64_t g = 0; g < N; ++g) {
+    for (int k = 0; k < L; ++k) ent[(size_t)g * L + k] = make_int4((int)g, (int)g, (int)g, -1);
+    int64_t blk = g;
+    const int32_t k0 = tl->node_tri_start[g], k1 = tl->node_tri_start[g + 1];
+    for (int32_t k = k0; k < k1; ++k) {
+      if (k > k0 && (k - k0) % L == 0) {
+        next[blk] = (int32_t)next.size();
+        blk = (int64_t)next.size();
+        next.push_back(-1);
+        ent.resize(ent.size() + L, make_int4((int)g, (int)g, (int)g, -1));
+      }
+      const int32_t s = tl->node_tri[k] >> 2;
+      const bool fresh = k > k0 && tile_of[s] != tile_of[tl->node_tri[k - 1] >> 2];
+      int4& e = ent[(size_t)blk * L + (k - k0) % L];
+      e.x = tl->tri_sorted[s];
+      e.y = tl->tri_sorted[T + s];
+      e.z = tl->tri_sorted[2 * T + s];
+      e.w = s << 3 | (int)fresh << 2 | (tl->node_tri[k] & 3);
+    }
+  }
+  for (int32_t f = 0; f < m->n_fix; ++f) {
+    const int32_t b0 = tl->fix_bedge_start[f], nb = tl->fix_bedge_start[f + 1] - b0;
+    if (nb > 255 || b0 >= 1 << 23) return FVM_OK;  // no lists: the tile kernels
+    bed[tl->fix_nodes[f]] = b0 << 8 | nb;
+  }
+  int rc = upload(&m->node_ent, ent.data(), (int64_t)ent.size());
+  if (rc == FVM_OK) rc = upload(&m->node_next, next.data(), (int64_t)next.size());
+  if (rc == FVM_OK) rc = upload(&m->node_bed, bed.data(), N);
+  return rc;
 }
 
 int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
@@ -247,6 +288,7 @@ int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
   UP(m->lcv, (const double*)nullptr, m->n_local);
   UP(m->qflag, (const int32_t*)nullptr, 1);
 #undef UP
+  if (N <= kNodeMeshMax && (rc = node_lists(tl, m)) != FVM_OK) return rc;
   m->convex = convex_domain(d);
   m->n_bedge_items = tl->fix_bedge_start[m->n_fix];
   m->n_bvert_items = tl->fix_bvert_start[m->n_fix];

@@ -85,6 +85,10 @@ KArgs make_args(const fvm_ctx* c) {
   a.bflux = c->bflux;
   a.n_bitems = m->n_bedge_items;
   a.t = 0;
+  a.N = m->N;
+  a.node_ent = m->node_ent;
+  a.node_next = m->node_next;
+  a.node_bed = m->node_bed;
   a.tile_dt = a.dtv = nullptr;
   return a;
 }
@@ -113,6 +117,20 @@ void launch_fix(const KArgs& a, hipStream_t s) {
 
 template <int FK, int MODE>
 int launch_fk(const KArgs& a, int tile_tris, hipStream_t s) {
+  if constexpr (MODE != M_EULER) {
+    // One launch by nodes up to the size where its threefold fluxes cost more than the
+    // second launch.  Measured, us, node against tile kernels (RHS of a quadratic D(u)):
+    // 3.8 / 7.6 at 2,500 nodes, 4.1 / 8.1 at 14,400, 6.2 / 8.1 at 40,000 and 8.2 / 8.3 at
+    // 57,600; nodal D 7.5 / 8.4 at 40,000 and 9.9 / 8.6 at 57,600.  With nine coefficients
+    // per triangle 7.5 / 8.9 at 28,900 and 9.9 / 8.9 at 40,000; with pow in every edge's
+    // flux 8.4 / 11.1 at 14,400 and 11.9 / 11.2 at 28,900.
+    constexpr int64_t kMost = FK == FVM_FLUX_D_POWER ? 20000 : (FK == FVM_FLUX_LINEAR ? 32000 : kNodeMeshMax);
+    if (a.node_ent && a.N <= kMost) {
+      hipLaunchKernelGGL((node_kernel<FK, MODE>), dim3((unsigned)((a.N * kNodeLanes + 255) / 256)), dim3(256), 0, s, a);
+      FVM_HIP(hipGetLastError());
+      return FVM_OK;
+    }
+  }
   launch_tiles<FK, MODE>(a, tile_tris, s);
   launch_fix<FK, MODE>(a, s);
   FVM_HIP(hipGetLastError());

@@ -239,3 +239,42 @@ def test_points_outside_the_triangulation(gpu):
         assert sols[name].retcode == "Success"
     assert np.all(sols["ext"].u[n0:] == 0.0)
     np.testing.assert_allclose(sols["ext"].u[:n0], sols["base"].u, rtol=0, atol=1e-10 * np.abs(sols["base"].u).max())
+
+
+def _fan(d, closed):
+    """A hub with d triangles around it: closed, or with the hub on the boundary."""
+    m = d if closed else d + 1
+    th = (2 * np.pi if closed else 0.9 * np.pi * min(1.0, d / 4)) * np.arange(m) / (m if closed else d)
+    r = 1.0 + 0.2 * np.cos(5 * np.arange(m))
+    x, y = np.concatenate([[0.05], r * np.cos(th)]), np.concatenate([[-0.02], r * np.sin(th)])
+    k = np.arange(d)
+    tris = np.stack([0 * k, 1 + k, 1 + (k + 1) % m], 1).astype(np.int32)
+    edges = tris[:, 1:]
+    if not closed:
+        edges = np.concatenate([[[0, 1]], edges, [[d + 1, 0]]]).astype(np.int32)
+    seg = (np.arange(len(edges)) >= len(edges) // 2).astype(np.int32)
+    return FVM.Triangulation(x, y, tris, edges, seg)
+
+
+@pytest.mark.parametrize("closed,d", [(True, 3), (True, 8), (True, 9), (True, 17), (True, 64), (False, 1),
+                                      (False, 2), (False, 8), (False, 9), (False, 25)])
+def test_nodes_of_any_degree(gpu, closed, d):
+    """The hub's sum runs over one, a full and several blocks of eight incidences, with and
+    without boundary edges; the tangent too (bars of the RHS and JVP tests)."""
+    tri = _fan(d, closed)
+    mesh = FVM.FVMGeometry(tri)
+    BCs = FVM.BoundaryConditions(mesh, (lambda x, y, t, u, p: 0.3 + 0.0 * u, lambda x, y, t, u, p: 0.5 * u),
+                                 (FVM.Neumann, FVM.Dudt))
+    u = np.random.default_rng(d).random(tri.num_points())
+    prob = FVM.FVMProblem(mesh, BCs, diffusion_function=lambda x, y, t, u, p: 0.1 + u ** 2,
+                          source_function=lambda x, y, t, u, p: u * (1 - u), initial_condition=u,
+                          final_time=1.0)
+    orc = oracle_for(prob, dict(builtin=dict(flux_kind=0, dpoly=[0.1, 0, 1, 0], spoly=[0, 1, -1, 0],
+                                             fn=([0.3, 0.0], [0.0, 0.5], [0.0, 0.0]))))
+    du = FVM.fvm_eqs(np.zeros_like(u), u, prob, 0.0)
+    assert_parity(du, orc.rhs(u, 0.0), orc.scale(u, 0.0))
+    v = np.random.default_rng(d + 1).standard_normal(len(u))
+    jv = FVM.DeviceArray(len(u))
+    prob.device_context().jvp(FVM.DeviceArray.from_host(u), FVM.DeviceArray.from_host(v), jv, 0.0)
+    ref = orc.rhs_cs(u + 1e-30j * v, None, 0.0).imag / 1e-30
+    assert np.max(np.abs(jv.to_host() - ref)) <= 1e-11 * np.max(np.abs(ref))
