@@ -108,11 +108,14 @@ __device__ __forceinline__ int32_t find_directed_edge(const int32_t* __restrict_
 }
 
 
-// fvm_ode_solve's Tsit5 loop for a small ODE template in one launch
-// (fvm_linalg.hip); FVM_ERR_STATE when the template does not qualify.
-int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const double* k0, const double* u, double* d_u,
-                         double t0, double dt, int64_t it0, int64_t ks0, const double A[7][6], const double Bt[7],
-                         fvm_ode_stats* st, hipStream_t s);
+struct Tsit5Loop;
+// fvm_ode_solve's Tsit5 loop for a small ODE template or mesh in one launch
+// (fvm_linalg.hip, fvm_tsit5_mesh.hip), from start's time, step, state and k0 (its
+// other members are set there); FVM_ERR_STATE when it does not qualify.
+int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const Tsit5Loop& start, fvm_ode_stats* st,
+                         hipStream_t s);
+int problem_tsit5_small(const fvm_ctx* c, const fvm_ode_opts* o, const Tsit5Loop& start, fvm_ode_stats* st,
+                        hipStream_t s);
 
 // Classical Gram-Schmidt applied twice to w against xs[0..k) (k <= 64) plus |w|^2,
 // intermediates on the device, one host synchronisation: h_host[0..k), h_host[k..2k)
@@ -123,6 +126,29 @@ int cgs2_norm(int64_t n, int k, const double* const* xs, double* w, double* h_ho
 
 // Nodes of the meshes that keep node_kernel's lists, at most (see launch_fk).
 constexpr int64_t kNodeMeshMax = 40000;
+
+// A mesh of up to 65,536 nodes cut into blocks of kBlockNodes nodes, one per workgroup
+// of the one-launch Tsit5 loop (fvm_tsit5_mesh.hip), with every triangle of a block's
+// nodes.  Lists in one device array, made by mesh_blocks (fvm_mesh.hip).
+constexpr int kBlockNodes = 256;
+constexpr int kBlockTris = 512;    // triangles per list: inner ones, and those with nodes of other blocks
+constexpr int kBlockHalo = 512;    // nodes of other blocks, at most
+constexpr int kBlockItems = 256;   // boundary items, at most
+constexpr int kBlockFlux = 2 * kBlockTris + 1;  // row length of the block's fluxes
+struct MeshBlocks {
+  int32_t n = 0;                   // blocks, 0: no lists
+  const int32_t* node = nullptr;   // [n][256] node, -1: none (the last block's end)
+  const int32_t* bitem = nullptr;  // [n][256] its boundary items in the block: first << 8 | count
+  const int32_t* deg = nullptr;    // [n][256] its triangles
+  const int32_t* more = nullptr;   // [n][256] where those past the eighth stand in rest
+  const uint16_t* inc = nullptr;   // [n][256][8] slot kBlockFlux + local triangle, | 0x8000: first of another tile
+  const int32_t* rest = nullptr;   // such entries
+  const int32_t* tri = nullptr;    // [n][1024] sorted triangle (-1: none), inner ones in the first half
+  const int32_t* loc = nullptr;    // [n][1024] its vertices' local ids a | b << 10 | c << 20 (256 +: halo)
+  const int32_t* halo = nullptr;   // [n][512] position 256 block + local id, -1: none
+  const int32_t* item = nullptr;   // [n][256] boundary edge << 1 | endpoint, -1: none
+  const int32_t* iloc = nullptr;   // [n][256] its triangle's vertices, as loc
+};
 
 // Device-resident mesh: geometry SoA in tile (sorted) triangle order plus the
 // tile / fix-up structures from fvmh_tiles_build.
@@ -151,6 +177,8 @@ struct fvm_mesh {
                                     // first of another tile << 2 | slot (-1: padding)
   int32_t* node_next = nullptr;     // [blocks] the node's next block, -1: none
   int32_t* node_bed = nullptr;      // [N] boundary items: first << 8 | count
+  int32_t* block_mem = nullptr;     // the lists of blocks
+  MeshBlocks blocks;
   int32_t* qflag = nullptr;         // device flag of the pointwise queries (run_flagged)
   bool convex = false;              // one boundary loop that turns left (or goes straight) at
                                     // every vertex: a point outside a boundary edge is outside

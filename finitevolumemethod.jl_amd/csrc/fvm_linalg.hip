@@ -1800,20 +1800,17 @@ int fvm_template_solve(fvm_template* t, const fvm_solve_opts* o, double* d_x, fv
 namespace fvm {
 
 // The Tsit5 loop of fvm_ode_solve on the template's ELL copy of A in one launch
-// (fvm_tsit5.hip), from time t0 with step dt, it0 steps and ks0 saves done,
-// k0 = f(u) already computed; the final state goes to d_u.  Returns
-// FVM_ERR_STATE when the template has no ELL copy or n exceeds kTsit5GridMax, so
-// that the caller keeps the multi-kernel loop.
-int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const double* k0, const double* u, double* d_u,
-                         double t0, double dt, int64_t it0, int64_t ks0, const double A[7][6], const double Bt[7],
-                         fvm_ode_stats* st, hipStream_t s) {
+// (fvm_tsit5.hip); FVM_ERR_STATE when the template has no ELL copy or n exceeds
+// kTsit5GridMax, so that the caller keeps the multi-kernel loop.
+int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const Tsit5Loop& start, fvm_ode_stats* st,
+                         hipStream_t s) {
   // (an assembled ODE template: its pattern is symmetric, as the grid form requires)
   if (!t || t->kind != 2 || t->ellW <= 0 || o->n != t->n || o->n > kTsit5GridMax) return FVM_ERR_STATE;
   // one workgroup while its registers hold the rows: 11 us a step at 2,500 rows, where
   // the grid takes 14
   const bool local = o->n <= tsit5_rows_local_max(t->ellW);
   SmallTsit5 a;
-  a.n = o->n;
+  static_cast<Tsit5Loop&>(a) = start;
   a.W = t->ellW;
   a.off = t->sl_off;
   a.perm = t->sl_perm;
@@ -1824,52 +1821,7 @@ int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const dou
   a.eval = t->ellA;
   a.diag = t->diagA;
   a.b = t->b;
-  a.k0 = k0;
-  a.u = u;
-  a.u_out = d_u;
-  a.t0 = t0;
-  a.tf = o->tf;
-  a.dt = dt;
-  a.abstol = o->abstol;
-  a.reltol = o->reltol;
-  a.maxiters = o->maxiters;
-  a.it0 = it0;
-  a.fsal = o->fsal;
-  a.n_save = o->n_save;
-  a.ks0 = ks0;
-  a.saves = o->d_saves;
-  for (int j = 0; j < 7; ++j) {
-    for (int i = 0; i < 6; ++i) a.A[j][i] = A[j][i];
-    a.Bt[j] = Bt[j];
-  }
-  // exchange words of the grid form, save times, 6 result slots
-  const size_t words = local ? 0 : tsit5_rows_grid_words(o->n);
-  double* dev = nullptr;
-  FVM_HIP(hipMalloc((void**)&dev, sizeof(double) * (words + (size_t)o->n_save + 6)));
-  a.grid = (uint64_t*)dev;
-  a.save_t = dev + words;
-  a.stats = dev + words + o->n_save;
-  hipError_t e = hipSuccess;
-  if (words) e = hipMemsetAsync(dev, 0, sizeof(double) * words, s);
-  if (e == hipSuccess && o->n_save > 0)
-    e = hipMemcpyAsync(dev + words, o->save_t, sizeof(double) * (size_t)o->n_save, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = tsit5_rows(a, local, s);
-  double r[6] = {0, 0, 0, 0, 0, 0};
-  if (e == hipSuccess) e = hipMemcpyAsync(r, a.stats, sizeof r, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(dev);
-  if (e != hipSuccess) return hip_fail(e, "fvm_ode_solve (one-launch Tsit5)");
-  if (r[5] < 0) {
-    set_error("fvm_ode_solve: the grid's exchange timed out");
-    return FVM_ERR_HIP;
-  }
-  st->t = r[0];
-  st->naccept += (int64_t)r[1];
-  st->nreject += (int64_t)r[2];
-  st->nf += (int64_t)r[3];
-  st->nsaved = (int64_t)r[4];
-  st->retcode = (int32_t)r[5];
-  return FVM_OK;
+  return tsit5_run(a, local ? 0 : tsit5_rows_grid_words(o->n), &a.grid, o, [&] { return tsit5_rows(a, local, s); }, st, s);
 }
 
 }  // namespace fvm

@@ -6,6 +6,7 @@
 // FMA contraction off (the library is built with -ffp-contract=off): the
 // shape-function determinant cancels badly on small triangles far from the
 // origin, so any other evaluation order changes s1..s9 well above 1e-12.
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -133,7 +134,7 @@ void free_mesh(fvm_mesh* m) {
                   m->fix_part_start, m->fix_bedge_start, m->fix_bedge, m->fix_bvert_start,
                   m->fix_bvert, m->lcv, m->node_tri_start,
                   m->node_tri, m->bedges, m->badj, m->perm, m->is_vertex, m->qflag,
-                  m->node_ent, m->node_next, m->node_bed};
+                  m->node_ent, m->node_next, m->node_bed, m->block_mem};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete m;
@@ -217,6 +218,113 @@ int node_lists(const fvmh_tiles* tl, fvm_mesh* m) {
   return rc;
 }
 
+// The lists of MeshBlocks; none (m->blocks.n = 0) when a block would not fit its bounds.
+// Blocks are runs of the nodes in the order in which the triangles, sorted along a
+// space-filling curve, first reach them: compact patches, whatever the numbering.
+int mesh_blocks(const fvmh_tiles* tl, fvm_mesh* m) {
+  constexpr int NB = kBlockNodes, NT = 2 * kBlockTris, NH = kBlockHalo, NI = kBlockItems;
+  const int64_t N = m->N, T = m->T;
+  const int32_t* tri = tl->tri_sorted;
+  std::vector<int32_t> pos(N, -1), order;
+  order.reserve(N);
+  for (int64_t s = 0; s < T; ++s)
+    for (int v = 0; v < 3; ++v) {
+      const int32_t g = tri[v * T + s];
+      if (pos[g] < 0) pos[g] = (int32_t)order.size(), order.push_back(g);
+    }
+  for (int64_t g = 0; g < N; ++g)
+    if (pos[g] < 0) pos[g] = (int32_t)order.size(), order.push_back((int32_t)g);
+  std::vector<int32_t> tile_of(T), fix_of(N, -1);
+  for (int32_t k = 0; k < m->n_tiles; ++k)
+    for (int32_t s = tl->tile_tri_start[k]; s < tl->tile_tri_start[k + 1]; ++s) tile_of[s] = k;
+  for (int32_t f = 0; f < m->n_fix; ++f) fix_of[tl->fix_nodes[f]] = f;
+
+  const int64_t n = (N + NB - 1) / NB;
+  // all lists in one array, rest behind the others
+  const int64_t per[] = {NB * 4, NB, NB, NB, NB, NT, NT, NH, NI, NI};
+  int64_t at[11] = {0};
+  for (int k = 0; k < 10; ++k) at[k + 1] = at[k] + n * per[k];
+  std::vector<int32_t> all(at[10], 0);
+  uint16_t* inc = (uint16_t*)all.data();
+  int32_t *node = &all[at[1]], *bitem = &all[at[2]], *deg = &all[at[3]], *more = &all[at[4]], *btri = &all[at[5]],
+          *loc = &all[at[6]], *halo = &all[at[7]], *item = &all[at[8]], *iloc = &all[at[9]];
+  for (int32_t* p : {node, btri, halo, item}) {
+    const int64_t* k = std::find(at, at + 10, p - all.data());
+    std::fill(p, p + (k[1] - k[0]), -1);
+  }
+  std::vector<int32_t> rest;
+  std::vector<int32_t> tri_at(T, -1), tri_in(T, -1), halo_at(N, -1), halo_in(N, -1);  // local id, of which block
+  for (int64_t b = 0; b < n; ++b) {
+    const int64_t p0 = b * NB, p1 = std::min(N, p0 + NB);
+    int n_in = 0, n_out = 0, n_halo = 0, n_item = 0;
+    auto local = [&](int32_t g) {
+      return pos[g] >= p0 && pos[g] < p1 ? pos[g] - (int32_t)p0 : (halo_in[g] == b ? NB + halo_at[g] : -1);
+    };
+    auto vertices = [&](int32_t s) {
+      return local(tri[s]) | local(tri[T + s]) << 10 | local(tri[2 * T + s]) << 20;
+    };
+    for (int64_t p = p0; p < p1; ++p) {
+      const int32_t g = order[p];
+      node[p] = g;
+      const int32_t k0 = tl->node_tri_start[g], k1 = tl->node_tri_start[g + 1];
+      deg[p] = k1 - k0;
+      more[p] = (int32_t)rest.size();
+      for (int32_t k = k0; k < k1; ++k) {
+        const int32_t s = tl->node_tri[k] >> 2;
+        if (tri_in[s] != b) {
+          bool inner = true;
+          for (int v = 0; v < 3; ++v) {
+            const int32_t h = tri[v * T + s];
+            if (local(h) >= 0 && local(h) < NB) continue;
+            inner = false;
+            if (local(h) >= 0) continue;
+            if (n_halo == NH) return FVM_OK;
+            halo_in[h] = (int32_t)b;
+            halo_at[h] = n_halo;
+            halo[b * NH + n_halo++] = pos[h];
+          }
+          if (inner && n_in == kBlockTris) inner = false;
+          if (!inner && n_out == kBlockTris) return FVM_OK;
+          tri_in[s] = (int32_t)b;
+          tri_at[s] = inner ? n_in++ : kBlockTris + n_out++;
+          btri[b * NT + tri_at[s]] = s;
+          loc[b * NT + tri_at[s]] = vertices(s);
+        }
+        const bool fresh = k > k0 && tile_of[s] != tile_of[tl->node_tri[k - 1] >> 2];
+        const int e = (tl->node_tri[k] & 3) * kBlockFlux + tri_at[s] + (fresh ? 0x8000 : 0);
+        if (k - k0 < 8) inc[(size_t)p * 8 + (k - k0)] = (uint16_t)e;
+        else rest.push_back(e);
+      }
+      if (fix_of[g] < 0) continue;
+      const int32_t b0 = tl->fix_bedge_start[fix_of[g]], b1 = tl->fix_bedge_start[fix_of[g] + 1];
+      if (n_item + (b1 - b0) > NI || b1 - b0 > 255) return FVM_OK;
+      bitem[p] = n_item << 8 | (b1 - b0);
+      for (int32_t q = b0; q < b1; ++q, ++n_item) {
+        item[b * NI + n_item] = tl->fix_bedge[q];
+        iloc[b * NI + n_item] = vertices(tl->badj_sorted[tl->fix_bedge[q] >> 1]);
+        if (iloc[b * NI + n_item] < 0) return FVM_OK;  // a boundary edge beside a triangle without its node
+      }
+    }
+  }
+  all.insert(all.end(), rest.begin(), rest.end());
+  const int rc = upload(&m->block_mem, all.data(), (int64_t)all.size());
+  if (rc != FVM_OK) return rc;
+  MeshBlocks& B = m->blocks;
+  B.n = (int32_t)n;
+  B.inc = (const uint16_t*)m->block_mem;
+  B.node = m->block_mem + at[1];
+  B.bitem = m->block_mem + at[2];
+  B.deg = m->block_mem + at[3];
+  B.more = m->block_mem + at[4];
+  B.tri = m->block_mem + at[5];
+  B.loc = m->block_mem + at[6];
+  B.halo = m->block_mem + at[7];
+  B.item = m->block_mem + at[8];
+  B.iloc = m->block_mem + at[9];
+  B.rest = m->block_mem + at[10];
+  return FVM_OK;
+}
+
 int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
   // Tiles of up to 512 triangles run on 256-thread workgroups with room for 512
   // local nodes; tiles of up to 1024 triangles on 512-thread workgroups with 1024.
@@ -289,6 +397,7 @@ int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
   UP(m->qflag, (const int32_t*)nullptr, 1);
 #undef UP
   if (N <= kNodeMeshMax && (rc = node_lists(tl, m)) != FVM_OK) return rc;
+  if (N <= 65536 && !tri_group && (rc = mesh_blocks(tl, m)) != FVM_OK) return rc;
   m->convex = convex_domain(d);
   m->n_bedge_items = tl->fix_bedge_start[m->n_fix];
   m->n_bvert_items = tl->fix_bvert_start[m->n_fix];

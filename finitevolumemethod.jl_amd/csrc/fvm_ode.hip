@@ -17,6 +17,7 @@
 #include <cmath>
 
 #include "fvm_internal.hpp"
+#include "fvm_tsit5.hpp"
 
 using namespace fvm;
 
@@ -139,10 +140,26 @@ int tsit5(const fvm_ode_opts* o, const Op& op, double* d_u, fvm_ode_stats* st, f
     if ((rc = save(o, ks++, u, s))) return rc;
   int64_t it = 0;
   st->retcode = FVM_ODE_SUCCESS;
-  if (op.kind == FVM_OP_TEMPLATE && !op.dirichlet) {
-    // small templates: the whole loop in one launch (same arithmetic per element)
-    rc = fvm::template_tsit5_small((const fvm_template*)op.h, o, k[0], u, d_u, t, dt, it, ks, kA, kBt, st,
-                                   (hipStream_t)s);
+  if ((op.kind == FVM_OP_TEMPLATE && !op.dirichlet) || op.kind == FVM_OP_PROBLEM) {
+    // small templates and meshes: the whole loop in one launch (same arithmetic per element)
+    fvm::Tsit5Loop a = {};
+    a.n = n;
+    a.t0 = t;
+    a.dt = dt;
+    a.it0 = it;
+    a.ks0 = ks;
+    a.dirichlet = op.dirichlet;
+    a.k0 = k[0];
+    a.u = u;
+    a.u_out = d_u;
+    for (int j = 0; j < 7; ++j) {
+      for (int i = 0; i < 6; ++i) a.A[j][i] = kA[j][i];
+      a.Bt[j] = kBt[j];
+      a.C[j] = kC[j];
+    }
+    rc = op.kind == FVM_OP_TEMPLATE
+             ? fvm::template_tsit5_small((const fvm_template*)op.h, o, a, st, (hipStream_t)s)
+             : fvm::problem_tsit5_small((const fvm_ctx*)op.h, o, a, st, (hipStream_t)s);
     if (rc != FVM_ERR_STATE) return rc;
     rc = FVM_OK;
   }

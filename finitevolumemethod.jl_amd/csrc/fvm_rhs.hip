@@ -28,7 +28,7 @@ using namespace fvm;
 
 using namespace fvm_k;
 
-namespace {
+namespace fvm_k {
 
 KArgs make_args(const fvm_ctx* c) {
   const fvm_mesh* m = c->m;
@@ -91,6 +91,21 @@ KArgs make_args(const fvm_ctx* c) {
   a.node_bed = m->node_bed;
   a.tile_dt = a.dtv = nullptr;
   return a;
+}
+
+}  // namespace fvm_k
+
+namespace {
+
+__global__ __launch_bounds__(256) void dirichlet_kernel(int n, const int32_t* __restrict__ nodes,
+                                                        const int32_t* __restrict__ fidx,
+                                                        const double* __restrict__ X,
+                                                        const double* __restrict__ Y, CondTable C,
+                                                        double t, double* __restrict__ u) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
+  const int g = nodes[k];
+  u[g] = eval_cond(C, fidx[g], X[g], Y[g], t, u[g], C.node_g ? C.node_g[g] : 0.0);
 }
 
 // Grid: the boundary workgroups followed by one workgroup per tile.

@@ -67,6 +67,10 @@ struct KArgs {
   const double* dtv;      // M_EULER: time step per node (fix-up nodes)
 };
 
+#ifndef __HIPCC_RTC__
+KArgs make_args(const fvm_ctx* c);  // (fvm_rhs.hip)
+#endif
+
 // How much of the triangle record the tile kernels rebuild from the vertex
 // coordinates instead of streaming it (the rebuilt values equal the stored ones
 // bit for bit: same operations as the geometry kernel):
@@ -206,24 +210,80 @@ __device__ __forceinline__ BGeo bgeo(const KArgs& a, int e) {
   return G;
 }
 
+// A boundary CV edge (endpoint ep of boundary edge e): what its flux takes besides u, for
+// kernels that evaluate it many times.  (bedge_flux through these would cost the tile
+// kernels registers: 12.5 -> 12.8 us a call at 155,701 nodes, an ensemble's Euler steps
+// 3.17 -> 3.49 ms.)
+template <int FK>
+struct BItem {
+  double nx, ny, mx, my, ell, g;
+  double s[9];                               // of the adjacent triangle
+  double d[FK == FVM_FLUX_LINEAR ? 3 : 1];   // D there, or the coefficients
+  int nf;                                    // its condition, -1: the flux of the interior
+};
+template <int FK>
+__device__ __forceinline__ BItem<FK> boundary_item(const KArgs& a, int e, int ep, int va, int vb, int vc) {
+  const BGeo G = bgeo(a, e);
+  const int64_t Tt = a.badj[e];
+  BItem<FK> b;
+#pragma unroll
+  for (int f = 0; f < 9; ++f) b.s[f] = a.props[f * a.T + Tt];
+  b.nx = G.nx;
+  b.ny = G.ny;
+  b.mx = ep ? G.mx[1] : G.mx[0];
+  b.my = ep ? G.my[1] : G.my[0];
+  b.ell = G.ell;
+  b.nf = a.bneu[e];
+  b.g = a.C.bedge_g ? a.C.bedge_g[2 * e + ep] : 0.0;
+  if constexpr (FK == FVM_FLUX_LINEAR) {
+    const double* c = a.d_bedge + 3 * (2 * e + ep);  // projected onto n, times the length
+#pragma unroll
+    for (int k = 0; k < 3; ++k) b.d[k] = c[k];
+  } else if (FK == FVM_FLUX_D_NODAL) {
+    const double Da = exp(a.log_d[va]), Db = exp(a.log_d[vb]), Dc = exp(a.log_d[vc]);
+    const double da = b.s[0] * Da + b.s[1] * Db + b.s[2] * Dc;
+    const double db = b.s[3] * Da + b.s[4] * Db + b.s[5] * Dc;
+    const double dg = b.s[6] * Da + b.s[7] * Db + b.s[8] * Dc;
+    b.d[0] = da * b.mx + db * b.my + dg;
+  } else {
+    b.d[0] = d_of_u(FK) ? 0.0 : a.d_bedge[2 * e + ep];
+  }
+  return b;
+}
+
+// The flux through it, times its length: bedge_flux's operations.
+template <int FK>
+__device__ __forceinline__ double boundary_flux(const KArgs& a, const BItem<FK>& b, double ua, double ub, double uc) {
+  const double* s = b.s;
+  const double al = s[0] * ua + s[1] * ub + s[2] * uc;
+  const double be = s[3] * ua + s[4] * ub + s[5] * uc;
+  const double ga = s[6] * ua + s[7] * ub + s[8] * uc;
+  if (b.nf >= 0) return eval_cond(a.C, b.nf, b.mx, b.my, a.t, al * b.mx + be * b.my + ga, b.g) * b.ell;
+  if constexpr (FK == FVM_FLUX_LINEAR) return b.d[0] * al + b.d[1] * be + b.d[2] * ga;
+  const double D = d_of_u(FK) ? dfun<FK>(a, al * b.mx + be * b.my + ga, b.mx, b.my) : b.d[0];
+  const double qx = -D * al, qy = -D * be;
+  const double qn = qx * b.nx + qy * b.ny;
+  return qn * b.ell;
+}
+
 // Flux through the boundary CV edge of endpoint ep of boundary edge e, times its
 // length (get_boundary_fluxes, boundary_edge_contributions.jl:2-48), or its
-// directional derivative; u(g) and v(g) give the nodes' values.
-template <int FK, int MODE, class U, class V>
-__device__ __forceinline__ double bedge_flux_of(const KArgs& a, int e, int ep, U u, V v) {
+// directional derivative.
+template <int FK, int MODE>
+__device__ double bedge_flux(const KArgs& a, int e, int ep) {
   const BGeo G = bgeo(a, e);
   const int64_t Tt = a.badj[e];
   const int va = a.tri[Tt], vb = a.tri[a.T + Tt], vc = a.tri[2 * a.T + Tt];
   double s[9];
 #pragma unroll
   for (int f = 0; f < 9; ++f) s[f] = a.props[f * a.T + Tt];
-  const double ua = u(va), ub = u(vb), uc = u(vc);
+  const double ua = a.u[va], ub = a.u[vb], uc = a.u[vc];
   const double al = s[0] * ua + s[1] * ub + s[2] * uc;
   const double be = s[3] * ua + s[4] * ub + s[5] * uc;
   const double ga = s[6] * ua + s[7] * ub + s[8] * uc;
   double dal = 0, dbe = 0, dga = 0;
   if (MODE == M_JVP) {
-    const double wa = v(va), wb = v(vb), wc = v(vc);
+    const double wa = a.v[va], wb = a.v[vb], wc = a.v[vc];
     dal = s[0] * wa + s[1] * wb + s[2] * wc;
     dbe = s[3] * wa + s[4] * wb + s[5] * wc;
     dga = s[6] * wa + s[7] * wb + s[8] * wc;
@@ -265,11 +325,6 @@ __device__ __forceinline__ double bedge_flux_of(const KArgs& a, int e, int ep, U
       qn = a.C.cu[nf] * (dal * mx + dbe * my + dga);
   }
   return qn * G.ell;
-}
-
-template <int FK, int MODE>
-__device__ double bedge_flux(const KArgs& a, int e, int ep) {
-  return bedge_flux_of<FK, MODE>(a, e, ep, [&](int g) { return a.u[g]; }, [&](int g) { return a.v[g]; });
 }
 
 // ---------------------------------------------------------------------------
@@ -965,17 +1020,6 @@ __global__ __launch_bounds__(256) void vjp_fix_kernel(KArgs a) {
   }
   a.out[g] = acc + node_adj<FK>(a, g, a.u[g]);
   if (a.out2) a.out2[g] = accl;
-}
-
-__global__ __launch_bounds__(256) void dirichlet_kernel(int n, const int32_t* __restrict__ nodes,
-                                                        const int32_t* __restrict__ fidx,
-                                                        const double* __restrict__ X,
-                                                        const double* __restrict__ Y, CondTable C,
-                                                        double t, double* __restrict__ u) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const int g = nodes[k];
-  u[g] = eval_cond(C, fidx[g], X[g], Y[g], t, u[g], C.node_g ? C.node_g[g] : 0.0);
 }
 
 }  // namespace fvm_k

@@ -19,49 +19,15 @@
 // sell_slice's order, the linear combinations with their terms left to right, the
 // error norm summed in the order of that path's 512 x 256 grid, and the step
 // controller's power fvm_ctrl.hpp's: the same states bit for bit.
-#include <algorithm>
-#include <cmath>
-
 #include "fvm_grid.hpp"
 #include "fvm_tsit5.hpp"
+#include "fvm_tsit5_loop.hpp"
 
 using namespace fvm;
 
 namespace {
 
-constexpr int kBlk = 256;        // elements per partial sum of the error norm
 constexpr int kSlice = 64;       // rows per slice of the sliced ELL form
-constexpr int kDppShl4 = 0x104, kDppShl2 = 0x102, kDppShl1 = 0x101;
-
-// Lane 0: the wave's sum in the order of shuffles down by 32, 16, 8, 4, 2, 1.
-__device__ __forceinline__ double wave_tree(double x) {
-  x = half_sums<32>(x, x);
-  x = half_sums<16>(x, x);
-  x += dpp<kDppRor8>(x);
-  x += dpp<kDppShl4>(x);
-  x += dpp<kDppShl2>(x);
-  return x + dpp<kDppShl1>(x);
-}
-
-__device__ __forceinline__ double first_lane(double x) {
-  const uint64_t u = (uint64_t)__double_as_longlong(x);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
-  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-
-// ctrl_pow's operations with its divisions by small integers as Markstein's corrected
-// products (div_rn: the same quotients bit for bit): 20 dependent divisions are 2 us of
-// latency in a step of 7 us.
-__device__ __forceinline__ double step_pow(double x, double p) {
-  const double y = p * ctrl_log(x);
-  const double k = floor(y / 0.69314718055994531 + 0.5);
-  const double r = y - k * 0.69314718055994531;
-  double e = 1.0;
-#pragma unroll
-  for (int i = 20; i >= 1; --i) e = 1.0 + div_rn(e * r, (double)i, 1.0 / (double)i);
-  return ldexp(e, (int)k);
-}
 
 // The rows of one thread: W off-diagonal slots (padding: the row itself, value 0) as
 // where to find the neighbour and value.  kLocal: two 16-bit LDS byte offsets per register,
@@ -128,7 +94,7 @@ __global__ __launch_bounds__(T) void tsit5_rows_kernel(SmallTsit5 a) {
   auto u_of = [&](int r) -> double& { return kLocal ? S.u[tid + r * T] : u0; };
 
   // out = A x + b on the thread's rows, x handed to the other rows first
-  auto apply = [&](const double (&x)[RPT], double (&out)[RPT]) {
+  auto apply = [&](const double (&x)[RPT], double (&out)[RPT], double) {
     double* const X = S.X + (kLocal ? xbuf * T * RPT : 0);
     if (kLocal) {
 #pragma unroll
@@ -180,6 +146,7 @@ __global__ __launch_bounds__(T) void tsit5_rows_kernel(SmallTsit5 a) {
   // sum over the grid's rows of q[r], in the order of 512 workgroups of 256 threads
   // and their sum by one more: pairwise trees of 256 elements, then of the partial sums
   auto norm_sum = [&](const double (&q)[RPT]) -> double {
+    if (!kLocal) ++G.rtag;
     const int lt = tid % kBlk;
 #pragma unroll
     for (int r = 0; r < RPT; ++r) S.tree[r][tid] = q[r];
@@ -200,26 +167,7 @@ __global__ __launch_bounds__(T) void tsit5_rows_kernel(SmallTsit5 a) {
       __syncthreads();
       if (lane < T * RPT / kBlk) p[0] = S.part[lane];
     } else {
-      if (tid < 64) {
-        const int nb = (int)((n + kBlk - 1) / kBlk);
-        const uint32_t P = G.sums();
-#pragma nounroll
-        for (unsigned spin = 0;; ++spin) {
-          uint32_t stale = 0;
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (lane + 64 * j < nb) {
-              const grid_pair w = grid_get(G.view, P + 16u * (lane + 64 * j));
-              stale |= grid_stale(w, G.rtag);
-              p[j] = grid_value(w);
-            }
-          if (__all(stale == 0)) break;
-          if (G.waited_long(spin)) {
-            if (lane == 0) G.give_up();
-            break;
-          }
-        }
-      }
+      if (tid < 64) grid_parts(G, (int)((n + kBlk - 1) / kBlk), p);
     }
     const double t = wave_tree((p[0] + p[2]) + (p[1] + p[3]));
     if (kLocal) return first_lane(t);
@@ -229,101 +177,9 @@ __global__ __launch_bounds__(T) void tsit5_rows_kernel(SmallTsit5 a) {
     return S.part[0];
   };
 
-  double t = a.t0, dt = a.dt, qold = 1e-4;
-  int64_t it = a.it0, ks = a.ks0, naccept = 0, nreject = 0, nf = 0;
-  int retcode = FVM_ODE_SUCCESS;
-  while (t < a.tf && it < a.maxiters) {
-    ++it;
-    dt = fmin(dt, a.tf - t);
-#pragma unroll
-    for (int j = 1; j < 7; ++j) {
-#pragma unroll
-      for (int r = 0; r < RPT; ++r) {
-        double v = 1.0 * u_of(r);
-#pragma unroll
-        for (int i = 0; i < j; ++i) v = v + dt * a.A[j][i] * k[i][r];
-        un[r] = v;
-      }
-      apply(un, k[j]);
-      ++nf;
-    }
-    // the error norm: per element r = (sum_j dt bt_j k_j) / (abstol + reltol max(|u|, |unew|))
-    double q2[RPT];
-#pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-      double v = dt * a.Bt[0] * k[0][r];
-#pragma unroll
-      for (int j = 1; j < 7; ++j) v = v + dt * a.Bt[j] * k[j][r];
-      const double sc = a.abstol + a.reltol * fmax(fabs(u_of(r)), fabs(un[r]));
-      const double e = v / sc;
-      q2[r] = i0 + (int64_t)r * T < n ? e * e : 0.0;
-    }
-    if (!kLocal) ++G.rtag;
-    const double EEst = sqrt(norm_sum(q2) / (double)n);
-    if (!up) break;
-    if (!isfinite(EEst)) {
-      retcode = FVM_ODE_UNSTABLE;
-      break;
-    }
-    // max(EEst, 1e-16)^(7/50) in the even lanes, qold^(2/25) in the odd ones
-    const double pw = step_pow(lane & 1 ? qold : fmax(EEst, 1e-16), lane & 1 ? 2.0 / 25.0 : 7.0 / 50.0);
-    const double pe = first_lane(pw), po = first_lane(dpp<kDppXor1>(pw));
-    if (EEst <= 1.0) {
-      const double tn = t + dt;
-      while (ks < a.n_save && a.save_t[ks] <= tn + 1e-12 * fmax(1.0, fabs(tn))) {
-        const double th = fmin(1.0, fmax(0.0, (a.save_t[ks] - t) / dt));
-        const double t2 = th * th, t3 = t2 * th;
-        const double h00 = 2 * t3 - 3 * t2 + 1;
-        const double h10 = t3 - 2 * t2 + th;
-        const double h01 = -2 * t3 + 3 * t2;
-        const double h11 = t3 - t2;
-        const double c0 = h00, c1 = h10 * dt, c2 = h01, c3 = h11 * dt;
-#pragma unroll
-        for (int r = 0; r < RPT; ++r) {
-          const int64_t i = i0 + (int64_t)r * T;
-          double v = c0 * u_of(r);
-          v = v + c1 * k[0][r];
-          v = v + c2 * un[r];
-          v = v + c3 * k[6][r];
-          if (i < n) a.saves[ks * n + i] = v;
-        }
-        ++ks;
-      }
-#pragma unroll
-      for (int r = 0; r < RPT; ++r) u_of(r) = un[r];
-      t = tn;
-      ++naccept;
-      if (a.fsal) {
-#pragma unroll
-        for (int r = 0; r < RPT; ++r) k[0][r] = k[6][r];
-      } else {
-        apply(un, k[0]);
-        ++nf;
-      }
-      double q = pe / po;
-      q = fmin(5.0, fmax(0.1, q / 0.9));
-      dt = dt / q;
-      qold = fmax(EEst, 1e-4);
-    } else {
-      ++nreject;
-      const double q = fmin(5.0, pe / 0.9);
-      dt = dt / q;
-    }
-  }
-  if (retcode == FVM_ODE_SUCCESS && !(t >= a.tf)) retcode = FVM_ODE_MAXITERS;
-#pragma unroll
-  for (int r = 0; r < RPT; ++r) {
-    const int64_t i = i0 + (int64_t)r * T;
-    if (i < n) a.u_out[i] = u_of(r);
-  }
-  if (blockIdx.x == 0 && tid == 0) {
-    a.stats[0] = t;
-    a.stats[1] = (double)naccept;
-    a.stats[2] = (double)nreject;
-    a.stats[3] = (double)nf;
-    a.stats[4] = (double)ks;
-    a.stats[5] = up ? (double)retcode : -1.0;
-  }
+  auto row = [&](int r) { return i0 + (int64_t)r * T; };
+  auto no_dirichlet = [](double x, double) { return x; };
+  tsit5_loop<RPT, false>(a, k, un, u_of, row, apply, norm_sum, no_dirichlet, up);
 }
 
 constexpr int kLocalT = 512, kGridT = 256;
@@ -355,6 +211,44 @@ hipError_t run(SmallTsit5& a, bool local, hipStream_t s) {
 namespace fvm {
 
 int64_t tsit5_rows_local_max(int W) { return (int64_t)kLocalT * (W <= 6 ? 5 : 4); }
+
+int tsit5_run(Tsit5Loop& a, size_t words, uint64_t** grid, const fvm_ode_opts* o, const std::function<hipError_t()>& launch,
+              fvm_ode_stats* st, hipStream_t s) {
+  a.tf = o->tf;
+  a.abstol = o->abstol;
+  a.reltol = o->reltol;
+  a.maxiters = o->maxiters;
+  a.fsal = o->fsal;
+  a.n_save = o->n_save;
+  a.saves = o->d_saves;
+  // exchange words of the grid forms, save times, 6 result slots
+  double* dev = nullptr;
+  FVM_HIP(hipMalloc((void**)&dev, sizeof(double) * (words + (size_t)o->n_save + 6)));
+  *grid = (uint64_t*)dev;
+  a.save_t = dev + words;
+  a.stats = dev + words + o->n_save;
+  hipError_t e = hipSuccess;
+  if (words) e = hipMemsetAsync(dev, 0, sizeof(double) * words, s);
+  if (e == hipSuccess && o->n_save > 0)
+    e = hipMemcpyAsync(dev + words, o->save_t, sizeof(double) * (size_t)o->n_save, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = launch();
+  double r[6] = {0, 0, 0, 0, 0, 0};
+  if (e == hipSuccess) e = hipMemcpyAsync(r, a.stats, sizeof r, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  (void)hipFree(dev);
+  if (e != hipSuccess) return hip_fail(e, "fvm_ode_solve (one-launch Tsit5)");
+  if (r[5] < 0) {
+    set_error("fvm_ode_solve: the grid's exchange timed out");
+    return FVM_ERR_HIP;
+  }
+  st->t = r[0];
+  st->naccept += (int64_t)r[1];
+  st->nreject += (int64_t)r[2];
+  st->nf += (int64_t)r[3];
+  st->nsaved = (int64_t)r[4];
+  st->retcode = (int32_t)r[5];
+  return FVM_OK;
+}
 
 size_t tsit5_rows_grid_words(int64_t n) { return grid_words(n); }
 

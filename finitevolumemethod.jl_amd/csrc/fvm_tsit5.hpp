@@ -1,11 +1,34 @@
 // Arguments of the one-launch Tsit5 loop over a small ODE template (fvm_tsit5.hip).
 #pragma once
+#include <functional>
+
 #include "fvm_internal.hpp"
 
 namespace fvm {
 
-struct SmallTsit5 {
+// What the loop itself takes (fvm_tsit5_loop.hpp).
+struct Tsit5Loop {
   int64_t n;
+  double t0, tf, dt;
+  double abstol, reltol;
+  int64_t maxiters, it0;
+  int32_t fsal, dirichlet;
+  int64_t n_save, ks0;
+  const double* save_t;  // device copy
+  double* saves;
+  const double* k0;      // f(u) on entry
+  const double* u;       // the state on entry
+  double* u_out;
+  double* stats;         // [0] t, [1] naccept, [2] nreject, [3] nf, [4] nsaved, [5] retcode
+  double A[7][6], Bt[7], C[7];
+};
+
+// The options' part of a, its device memory (words of exchange memory, zeroed, to *grid
+// before launch()), the launch and the results to st.
+int tsit5_run(Tsit5Loop& a, size_t words, uint64_t** grid, const fvm_ode_opts* o, const std::function<hipError_t()>& launch,
+              fvm_ode_stats* st, hipStream_t s);
+
+struct SmallTsit5 : Tsit5Loop {
   // the sliced ELL copy of A (fvm_template): W unrolled slots, one of ecol / eoff
   int W;
   const int32_t* off;
@@ -17,19 +40,7 @@ struct SmallTsit5 {
   const double* eval;
   const double* diag;
   const double* b;
-  const double* k0;  // f(u) on entry
-  const double* u;   // the state on entry
-  double* u_out;
   uint64_t* grid;    // the grid form's exchange memory, zeroed
-  double t0, tf, dt;
-  double abstol, reltol;
-  int64_t maxiters, it0;
-  int32_t fsal;
-  int64_t n_save, ks0;
-  const double* save_t;  // device copy
-  double* saves;
-  double* stats;  // [0] t, [1] naccept, [2] nreject, [3] nf, [4] nsaved, [5] retcode
-  double A[7][6], Bt[7];
 };
 
 constexpr int64_t kTsit5GridMax = 65536;  // rows of the grid form (256 workgroups of 256)

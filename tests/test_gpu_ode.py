@@ -11,7 +11,11 @@ import pytest
 import finitevolumemethod as FVM
 from finitevolumemethod import _lib
 from finitevolumemethod.solve import fsal_ok, integrate
-from problems import annulus_problem, brusselator_system, mixed_problem
+from problems import (annulus_problem, brusselator_system, dxy_problem, heat_convection_problem, mixed_problem,
+                      nodal_problem, nonlinear_problem)
+from test_gpu_linear_flux import CASES as LINEAR_CASES, problem as linear_problem
+from test_gpu_power_law import power_problem
+from test_gpu_rhs import _fan
 
 pytestmark = pytest.mark.gpu
 
@@ -86,6 +90,52 @@ def test_tsit5_time_dependent_dirichlet_matches_host_loop(gpu):
     tri = prob.mesh.triangulation
     inner = np.unique(tri.boundary_edges[tri.boundary_segments == 1])
     np.testing.assert_allclose(a.final_device.to_host()[inner], 50 * (1 - np.exp(-0.3 / 2)), rtol=1e-13)
+
+
+def shuffled_problem():
+    """Scattered numbering and points that are no vertices: blocks far from the order of
+    the nodes, empty stars."""
+    base = FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, 31, 29, jitter=0.25, seed=4)
+    rng = np.random.default_rng(8)
+    n = len(base.x) + 3
+    new = rng.permutation(n)
+    x, y = np.full(n, 0.5), np.full(n, 0.5)
+    x[new[:-3]], y[new[:-3]] = base.x, base.y
+    tri = FVM.Triangulation(x, y, new[base.triangles], new[base.boundary_edges], base.boundary_segments)
+    mesh = FVM.FVMGeometry(tri)
+    BCs = FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.2 * x + 0.1 * t + 0.0 * u, FVM.Neumann)
+    return FVM.FVMProblem(mesh, BCs, diffusion_function=lambda x, y, t, u, p: 0.1 + u ** 2,
+                          source_function=lambda x, y, t, u, p: u * (1 - u), initial_condition=rng.random(n),
+                          final_time=1.0)
+
+
+def fan_problem(d, closed):
+    mesh = FVM.FVMGeometry(_fan(d, closed))
+    BCs = FVM.BoundaryConditions(mesh, (lambda x, y, t, u, p: 0.3 + 0.0 * u, lambda x, y, t, u, p: 0.5 * u),
+                                 (FVM.Neumann, FVM.Dudt))
+    return FVM.FVMProblem(mesh, BCs, diffusion_function=lambda x, y, t, u, p: 0.1 + u ** 2,
+                          initial_condition=np.random.default_rng(d).random(len(mesh.triangulation.x)),
+                          final_time=d ** -3.0)
+
+
+@pytest.mark.parametrize("build", [
+    lambda: nonlinear_problem(4, 3)[0], lambda: nonlinear_problem(16, 16)[0], lambda: nonlinear_problem(257, 2)[0],
+    lambda: nonlinear_problem(255, 257)[0], lambda: nonlinear_problem(257, 256)[0], lambda: nodal_problem(33, 31)[0],
+    lambda: dxy_problem(30)[0], lambda: linear_problem(*LINEAR_CASES["anisotropic"])[0],
+    lambda: power_problem()[0], lambda: heat_convection_problem(40)[0], lambda: fan_problem(40, True),
+    lambda: fan_problem(9, False), lambda: fan_problem(600, True), shuffled_problem],
+    ids=["tiny", "one_block", "strip", "most_blocks", "over_them", "nodal", "edge", "linear", "power", "neumann", "hub",
+         "boundary_hub", "wide_hub", "shuffled"])
+def test_tsit5_on_resident_blocks_matches_host_loop(gpu, build):
+    """One block of 256 nodes, several, the most, and meshes that keep the multi-kernel
+    loop (more nodes, a hub beyond a block's triangles); every flux kind."""
+    prob = build()
+    cv = prob.mesh.cv_volumes
+    t0, h2 = prob.initial_time, cv[cv > 0].min()
+    prob.final_time = t0 + (4.0 if prob.final_time > 10 else min(6 * h2, prob.final_time))
+    a = FVM.solve(prob, FVM.Tsit5(), saveat=np.linspace(t0, prob.final_time, 3), maxiters=200)
+    b = host_loop(prob, FVM.Tsit5(), saveat=np.linspace(t0, prob.final_time, 3), maxiters=200)
+    assert_same(a, b)
 
 
 def test_system_matches_host_loop(gpu):
