@@ -552,7 +552,7 @@ int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts* o, double*
   a.saves = o->d_saves;
   const size_t words = fvm::grid_words(n);
   double* base = nullptr;
-  FVM_HIP(hipMalloc((void**)&base, sizeof(double) * (words + (size_t)o->n_save + 16)));
+  FVM_HIP(fvm::dev_alloc((void**)&base, sizeof(double) * (words + (size_t)o->n_save + 16)));
   a.grid = (uint64_t*)base;
   double* tail = base + words;
   a.save_t = tail;
@@ -565,7 +565,7 @@ int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts* o, double*
   if (e == hipSuccess) e = FVM_TRB_LAUNCH(trbdf2_affine_kernel, a.J.W, n, a, st_);
   if (e == hipSuccess) e = hipMemcpyAsync(r, a.stats, sizeof r, hipMemcpyDeviceToHost, st_);
   if (e == hipSuccess) e = hipStreamSynchronize(st_);
-  (void)hipFree(base);
+  (void)fvm::dev_free(base);
   if (e != hipSuccess) return fvm::hip_fail(e, "fvm_trbdf2_affine");
   if (r[9] < 0) {
     fvm::set_error("fvm_trbdf2_affine: the grid's exchange timed out");

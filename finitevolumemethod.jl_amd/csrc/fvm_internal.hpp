@@ -42,6 +42,11 @@ namespace fvm {
 
 void set_error(const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
+
+// Device memory by way of the kept blocks (fvm_runtime.hip); dev_free takes any pointer of
+// hipMalloc too, and waits for the device.
+hipError_t dev_alloc(void** p, size_t bytes);
+hipError_t dev_free(void* p);
 // fvm_mesh_create with the triangles of each tri_group kept contiguous (NULL: one group)
 int mesh_create_grouped(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh** out);
 // One forward-Euler step of fvm_eqs! in place, fused into the RHS kernels:

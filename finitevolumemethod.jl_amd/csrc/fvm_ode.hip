@@ -74,7 +74,7 @@ struct Op {
 struct Work {
   double* base = nullptr;
   ~Work() {
-    if (base) (void)hipFree(base);
+    if (base) (void)dev_free(base);
   }
 };
 
@@ -121,7 +121,7 @@ int save(const fvm_ode_opts* o, int64_t k, const double* v, fvm_stream s) {
 int tsit5(const fvm_ode_opts* o, const Op& op, double* d_u, fvm_ode_stats* st, fvm_stream s) {
   const int64_t n = o->n;
   Work w;
-  FVM_HIP(hipMalloc((void**)&w.base, sizeof(double) * (size_t)(n > 0 ? n : 1) * 11));
+  FVM_HIP(dev_alloc((void**)&w.base, sizeof(double) * (size_t)(n > 0 ? n : 1) * 11));
   double* k[7];
   for (int j = 0; j < 7; ++j) k[j] = w.base + j * n;
   double *utmp = w.base + 7 * n, *unew = w.base + 8 * n, *interp = w.base + 9 * n, *u = w.base + 10 * n;
@@ -232,7 +232,7 @@ int tsit5(const fvm_ode_opts* o, const Op& op, double* d_u, fvm_ode_stats* st, f
 int fixed_step(const fvm_ode_opts* o, const Op& op, double* d_u, fvm_ode_stats* st, fvm_stream s) {
   const int64_t n = o->n;
   Work w;
-  FVM_HIP(hipMalloc((void**)&w.base, sizeof(double) * (size_t)(n > 0 ? n : 1) * 4));
+  FVM_HIP(dev_alloc((void**)&w.base, sizeof(double) * (size_t)(n > 0 ? n : 1) * 4));
   double *k1 = w.base, *u1 = w.base + n, *u2 = w.base + 2 * n, *u = w.base + 3 * n;
   FVM_HIP(hipMemcpyAsync(u, d_u, sizeof(double) * (size_t)n, hipMemcpyDeviceToDevice, (hipStream_t)s));
   const double h = o->dt;

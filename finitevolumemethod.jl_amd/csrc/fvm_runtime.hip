@@ -1,6 +1,9 @@
 // Runtime part of the C ABI: errors, device memory, streams, events.
 #include <cstdio>
 #include <cstring>
+#include <mutex>
+#include <unordered_map>
+#include <vector>
 
 #include "fvm_internal.hpp"
 
@@ -14,6 +17,115 @@ int hip_fail(hipError_t e, const char* what) {
   return e == hipErrorOutOfMemory ? FVM_ERR_ALLOC : FVM_ERR_HIP;
 }
 const std::string& last_error() { return g_last_error; }
+
+// Device memory: a block of 1 to 128 MiB is kept when it is freed and handed out again for
+// the same size on the same device.  hipMalloc and hipFree map and unmap such a block
+// (12 us each, measured at 8 and 64 MiB; 0.7 us below 1 MiB, which stay with HIP): a
+// gradient of 10^6 nodes, whose five arrays come and go with each call, 213 -> 110 us.
+// A free waits for the device first, as hipFree does, so whatever stream used the block
+// has finished with it and any stream may have it next.  At most 512 MiB are kept, none
+// longer than the next 64 frees, and all are given back when an allocation would fail.
+namespace {
+constexpr size_t kKeepMin = (size_t)1 << 20, kKeepMax = (size_t)128 << 20, kKeepTotal = (size_t)512 << 20;
+constexpr uint64_t kKeepFrees = 64;
+struct Block {
+  void* p;
+  size_t bytes;
+  int dev;
+  uint64_t freed;  // number of the free that kept it
+};
+std::mutex g_mem;
+std::unordered_map<void*, Block>* const g_live = new std::unordered_map<void*, Block>;  // handed out, of kept sizes
+std::vector<Block>* const g_kept = new std::vector<Block>;  // (never destroyed: frees may come at exit)
+size_t g_kept_bytes = 0;
+uint64_t g_frees = 0;
+
+// with g_mem held: give back the kept blocks that go(block) names
+template <class F>
+void give_back(F go) {
+  size_t w = 0;
+  for (Block& b : *g_kept) {
+    if (go(b)) {
+      g_kept_bytes -= b.bytes;
+      (void)hipFree(b.p);
+    } else {
+      (*g_kept)[w++] = b;
+    }
+  }
+  g_kept->resize(w);
+}
+}  // namespace
+
+hipError_t dev_alloc(void** p, size_t bytes) {
+  *p = nullptr;
+  if (bytes < kKeepMin || bytes > kKeepMax) {
+    hipError_t e = hipMalloc(p, bytes > 0 ? bytes : 1);
+    if (e != hipErrorOutOfMemory) return e;
+    std::lock_guard<std::mutex> lock(g_mem);
+    if (g_kept->empty()) return e;
+    (void)hipGetLastError();
+    give_back([](const Block&) { return true; });
+    return hipMalloc(p, bytes > 0 ? bytes : 1);
+  }
+  Block b{nullptr, (bytes + 0xffff) & ~(size_t)0xffff, 0, 0};
+  hipError_t e = hipGetDevice(&b.dev);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(g_mem);
+  for (size_t k = g_kept->size(); k-- > 0;) {
+    const Block& c = (*g_kept)[k];
+    if (c.bytes != b.bytes || c.dev != b.dev) continue;
+    b.p = c.p;
+    g_kept_bytes -= b.bytes;
+    g_kept->erase(g_kept->begin() + (long)k);
+    break;
+  }
+  if (!b.p) {
+    e = hipMalloc(&b.p, b.bytes);
+    if (e == hipErrorOutOfMemory && !g_kept->empty()) {
+      (void)hipGetLastError();
+      give_back([](const Block&) { return true; });
+      e = hipMalloc(&b.p, b.bytes);
+    }
+    if (e != hipSuccess) return e;
+  }
+  (*g_live)[b.p] = b;
+  *p = b.p;
+  return hipSuccess;
+}
+
+hipError_t dev_free(void* p) {
+  if (!p) return hipSuccess;
+  int dev = 0;
+  {
+    std::lock_guard<std::mutex> lock(g_mem);
+    auto it = g_live->find(p);
+    if (it == g_live->end()) return hipFree(p);
+    dev = it->second.dev;
+  }
+  // the wait outside the lock: other threads allocate and free meanwhile
+  int now = 0;
+  hipError_t e = hipGetDevice(&now);
+  if (e == hipSuccess && now != dev) e = hipSetDevice(dev);
+  if (e == hipSuccess) e = hipDeviceSynchronize();
+  if (now != dev) (void)hipSetDevice(now);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(g_mem);
+  auto it = g_live->find(p);
+  if (it == g_live->end()) return hipErrorInvalidValue;
+  Block b = it->second;
+  g_live->erase(it);
+  b.freed = ++g_frees;
+  g_kept->push_back(b);
+  g_kept_bytes += b.bytes;
+  // the oldest first (the list is in the order of the frees)
+  size_t over = g_kept_bytes > kKeepTotal ? g_kept_bytes - kKeepTotal : 0;
+  give_back([&](const Block& c) {
+    const bool go = over > 0 || g_frees - c.freed >= kKeepFrees;
+    if (go) over -= c.bytes < over ? c.bytes : over;
+    return go;
+  });
+  return hipSuccess;
+}
 }  // namespace fvm
 
 extern "C" {
@@ -52,14 +164,13 @@ int fvm_device_synchronize(void) {
 int fvm_alloc(void** d_ptr, size_t bytes) {
   FVM_CHECK(d_ptr, "fvm_alloc: null output");
   *d_ptr = nullptr;
-  if (bytes == 0) bytes = 1;
-  FVM_HIP(hipMalloc(d_ptr, bytes));
+  FVM_HIP(fvm::dev_alloc(d_ptr, bytes));
   return FVM_OK;
 }
 
 int fvm_free(void* d_ptr) {
   if (!d_ptr) return FVM_OK;
-  FVM_HIP(hipFree(d_ptr));
+  FVM_HIP(fvm::dev_free(d_ptr));
   return FVM_OK;
 }
 

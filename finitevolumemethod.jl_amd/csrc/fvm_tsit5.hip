@@ -223,7 +223,7 @@ int tsit5_run(Tsit5Loop& a, size_t words, uint64_t** grid, const fvm_ode_opts* o
   a.saves = o->d_saves;
   // exchange words of the grid forms, save times, 6 result slots
   double* dev = nullptr;
-  FVM_HIP(hipMalloc((void**)&dev, sizeof(double) * (words + (size_t)o->n_save + 6)));
+  FVM_HIP(dev_alloc((void**)&dev, sizeof(double) * (words + (size_t)o->n_save + 6)));
   *grid = (uint64_t*)dev;
   a.save_t = dev + words;
   a.stats = dev + words + o->n_save;
@@ -235,7 +235,7 @@ int tsit5_run(Tsit5Loop& a, size_t words, uint64_t** grid, const fvm_ode_opts* o
   double r[6] = {0, 0, 0, 0, 0, 0};
   if (e == hipSuccess) e = hipMemcpyAsync(r, a.stats, sizeof r, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(dev);
+  (void)dev_free(dev);
   if (e != hipSuccess) return hip_fail(e, "fvm_ode_solve (one-launch Tsit5)");
   if (r[5] < 0) {
     set_error("fvm_ode_solve: the grid's exchange timed out");

@@ -269,8 +269,7 @@ def fsal_ok(prob):
     if not prob.conditions.has_dirichlet_nodes():
         return True
     fn = prob.device_context().physics["fn"]
-    kind, fidx, _ = prob.conditions.flatten(prob.mesh.triangulation)
-    used = np.unique(fidx[kind == _lib.NODE_DIRICHLET])
+    used = set(prob.conditions.dirichlet_nodes.values())
     coef = [np.asarray(fn[1]), np.asarray(fn[2])] + ([np.asarray(fn[5])] if len(fn) > 5 else [])
     return all(float(c[f]) == 0.0 for c in coef for f in used)
 
