@@ -27,7 +27,8 @@
 //                       recomputed in FP64 whenever it has dropped by inner_rtol
 //                       (default 0.1), keeping the search direction.
 //   FVM_SOLVE_BICGSTAB  FP64 BiCGStab on M with Jacobi right preconditioning.
-//   FVM_SOLVE_AUTO      FP64 CG preconditioned by a multigrid cycle (fvm_amg.hip), the
+//   FVM_SOLVE_AUTO      up to kSmallMax unknowns the first method in one workgroup, above
+//                       FP64 CG preconditioned by a multigrid cycle (fvm_amg.hip), the
 //                       first method where that stops short.
 // Each reduction leaves one partial per workgroup, and every workgroup of the next
 // kernel re-adds all of them in the same fixed order, so solver scalars stay on the
@@ -40,6 +41,7 @@
 #include <vector>
 
 #include "fvm_amg.hpp"
+#include "fvm_grid.hpp"
 #include "fvm_internal.hpp"
 #include "fvm_tsit5.hpp"
 
@@ -54,9 +56,16 @@ constexpr int kRowsPerBlock = kRT / kLPR;
 constexpr int kRPG = FVM_SPMV_ROWS;      // rows per lane group per step of the SpMV loops
 constexpr int kEllMin = 4, kEllMax = 10; // unrolled slots of the sliced ELL form: the longest row's, in 4..10
 constexpr int kSlice = 64;               // rows per slice of the sliced ELL form: one wave
-// Unknowns from which FVM_SOLVE_AUTO uses the multigrid cycle: at 870 (30 x 29) a solve
-// takes 0.75 ms against 1.75 with Jacobi, the first one with the set-up 1.35; the set-up's
-// 0.6 ms outweighs the gain below about half of that.
+// Unknowns up to which FVM_SOLVE_AUTO first runs Jacobi-preconditioned CG in one
+// workgroup (cg_small), and the iterations it gives that.  Measured, ms, against the
+// cycle: 0.31 / 0.75 at 930 unknowns, 0.44 / 0.95 at 1,640, 0.65 / 1.06 at 2,813 (254
+// iterations); six rows a thread fill the registers.  500 iterations take as long as
+// the cycle with its set-up, which then goes on where they ended.
+constexpr int kSmallT = 512, kSmallRows = 6;
+constexpr int64_t kSmallMax = (int64_t)kSmallT * kSmallRows;
+constexpr int kSmallIter = 500;
+// Unknowns from which the multigrid cycle is used, on what cg_small leaves or does not
+// take; below that its set-up (0.6 ms) is most of a solve.
 constexpr int64_t kAmgMin = 400;
 constexpr int kAmgMaxIter = 200;         // its iterations, before Jacobi-preconditioned CG takes over
 
@@ -1317,6 +1326,160 @@ int inner_cg(fvm_template* t, const V* valM, const V* dinv, const V* wv, V* d, V
   return FVM_OK;
 }
 
+// Jacobi-preconditioned CG of a small system in one workgroup: inner_cg's iteration with
+// everything but the gathered direction in registers (a thread's rows: W of
+// the table's Wm slots as values and 16-bit LDS offsets, x, r, p, 1 / D and the norm's
+// weight; what longer rows have beyond W stays in memory).  On entry
+// r = -V (b - A x); x is updated in place until |r|_A^2 <= tabs2 or maxit iterations.
+// Bound by latency and LDS gathers: three barriers an iteration, 2.3 us at 2,813 rows
+// where the kernels of an iteration take 12: the solve 3.1 -> 0.65 ms.
+template <int W, int RPT>
+__global__ __launch_bounds__(kSmallT) void cg_small(int n, SellIdx S, const int32_t* __restrict__ ecol,
+                                                    const int16_t* __restrict__ eoff,
+                                                    const double* __restrict__ eval, const double* __restrict__ diag,
+                                                    const double* __restrict__ dinv, const double* __restrict__ wv,
+                                                    const double* __restrict__ r0, double* __restrict__ x, int Wm,
+                                                    double tabs2, int maxit, double* __restrict__ sc) {
+  static_assert(W % 2 == 0 && kSmallT * RPT <= 8192, "16-bit byte offsets");
+  __shared__ double P[kSmallT * RPT];
+  __shared__ double red[2][2][kSmallT / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // the lane that holds row i inside its slice: the inverse of perm
+  auto slot_of = [&](int i) { return __builtin_amdgcn_ds_permute((i < n ? (int)S.perm[i] : lane) << 2, lane); };
+  uint32_t c[RPT][W / 2], longer = 0;  // longer: slices with rows beyond W slots, bit r
+  double v[RPT][W], dg[RPT], dv[RPT], w[RPT], xr[RPT], r[RPT], p[RPT];
+#pragma unroll
+  for (int k = 0; k < RPT; ++k) {
+    const int i = tid + k * kSmallT, b = i / kSlice;
+    const bool in = i < n;
+    const int pos = slot_of(i);
+#pragma unroll
+    for (int s = 0; s < W; ++s) {
+      const int e0 = in && s < Wm ? S.off[(Wm + 1) * b + s] : 0, e1 = in && s < Wm ? S.off[(Wm + 1) * b + s + 1] : 0;
+      const bool on = e0 + pos < e1;
+      const int col = on ? (eoff ? i + (int)eoff[e0 + pos] : ecol[e0 + pos]) : i;
+      if (s % 2 == 0) c[k][s / 2] = (uint32_t)col * 8u;
+      else c[k][s / 2] |= (uint32_t)col << 19;
+      v[k][s] = on ? eval[e0 + pos] : 0.0;
+    }
+    if (__any(in && (S.rem_ptr[b + 1] > S.rem_ptr[b] ||
+                     (W < Wm && S.off[(Wm + 1) * b + Wm] > S.off[(Wm + 1) * b + W]))))
+      longer |= 1u << k;
+    dg[k] = in ? diag[i] : 0.0;
+    dv[k] = in ? dinv[i] : 0.0;
+    w[k] = in ? wv[i] : 0.0;
+    xr[k] = in ? x[i] : 0.0;
+    r[k] = in ? r0[i] : 0.0;
+    p[k] = 0.0;
+  }
+  // sums over the workgroup; the buffers alternate, so one barrier each
+  int buf = 0;
+  auto sum2 = [&](double& a, double& b) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if (lane == 0) {
+      red[buf][0][wave] = a;
+      red[buf][1][wave] = b;
+    }
+    __syncthreads();
+    a = b = 0.0;
+#pragma unroll
+    for (int q = 0; q < kSmallT / 64; ++q) {
+      a += red[buf][0][q];
+      b += red[buf][1][q];
+    }
+    buf ^= 1;
+  };
+  auto residual = [&](double& rz, double& wr) {
+    rz = wr = 0.0;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      rz += r[k] * (dv[k] * r[k]);
+      const double t = r[k] * w[k];
+      wr += t * t;
+    }
+    sum2(rz, wr);
+  };
+  double rz, wr, old = 0.0;
+  residual(rz, wr);
+  int it = 0, flag = 0;
+  while (wr > tabs2 && it < maxit) {  // (not on NaN)
+    const double beta = it == 0 ? 0.0 : rz / old;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      p[k] = dv[k] * r[k] + beta * p[k];
+      P[tid + k * kSmallT] = p[k];
+    }
+    __syncthreads();
+    double q[RPT], pq = 0.0, none = 0.0;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      double g[W];
+#pragma unroll
+      for (int s = 0; s < W; s += 2) {
+        uint32_t o = c[k][s / 2];
+        asm volatile("" : "+v"(o));  // taken apart here, not once outside the loop
+        g[s] = *(const double*)((const char*)P + (o & 0xffffu));
+        g[s + 1] = *(const double*)((const char*)P + (o >> 16));
+      }
+      double acc = 0.0;
+#pragma unroll
+      for (int s = 0; s < W; ++s) acc += v[k][s] * g[s];
+      if (longer & (1u << k)) {
+        const int i = tid + k * kSmallT, b = i / kSlice, pos = slot_of(i);
+        if (i < n) {
+          auto slot = [&](int e, int end) {
+            if (e < end) acc += eval[e] * P[eoff ? i + (int)eoff[e] : ecol[e]];
+          };
+          for (int j = W; j < Wm; ++j) slot(S.off[(Wm + 1) * b + j] + pos, S.off[(Wm + 1) * b + j + 1]);
+          int st = S.off[(Wm + 1) * b + Wm];
+          for (int j = S.rem_ptr[b]; j < S.rem_ptr[b + 1]; ++j) {
+            slot(st + pos, S.rem_off[j]);
+            st = S.rem_off[j];
+          }
+        }
+      }
+      q[k] = acc + dg[k] * p[k];
+      pq += p[k] * q[k];
+      __builtin_amdgcn_sched_barrier(0);  // all rows' gathers at once would spill
+    }
+    sum2(pq, none);
+    if (!(pq > 0.0)) {  // M is not positive definite on this direction: stop
+      flag = 2;
+      break;
+    }
+    const double alpha = rz / pq;
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+      xr[k] = xr[k] + alpha * p[k];
+      r[k] = r[k] - alpha * q[k];
+    }
+    old = rz;
+    residual(rz, wr);
+    ++it;
+  }
+#pragma unroll
+  for (int k = 0; k < RPT; ++k)
+    if (tid + k * kSmallT < n) x[tid + k * kSmallT] = xr[k];
+  if (tid == 0) {
+    sc[S_ITER] = (double)it;
+    sc[S_FLAG] = (double)flag;
+    sc[S_DONE] = 1.0;
+  }
+}
+
+template <int W>
+void cg_small_rows(fvm_template* t, const double* r, double* x, double tabs2, int maxit, hipStream_t s) {
+  const int rows = (int)((t->n + kSmallT - 1) / kSmallT);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kSmallT), 0, s, (int)t->n, sell_idx(t), t->ell_col, t->ell_off, t->ellM,
+                       t->diagM, t->dinv, t->wv, r, x, t->ellW, tabs2, maxit, t->sc);
+  };
+  if (rows <= 2) go(cg_small<W, 2>);
+  else if (rows <= 4) go(cg_small<W, 4>);
+  else go(cg_small<W, kSmallRows>);
+}
+
 // FP32 CG with reliable updates (Sleijpen & van der Vorst 1996): one Krylov
 // sequence for the whole solve.  Each step goes straight into the FP64 x (an FP32
 // correction vector would carry a rounding error of about eps32 kappa(M) of the
@@ -1729,6 +1892,27 @@ int fvm_template_solve(fvm_template* t, const fvm_solve_opts* o, double* d_x, fv
   const double tabs2 = 0.25 * target * target;
   int total = 0, outer = 0, flag = 0;
   const int method = o->method == FVM_SOLVE_AUTO ? (int)FVM_SOLVE_CG : o->method;
+  if (o->method == FVM_SOLVE_AUTO && t->use_ell && n <= kSmallMax) {
+    int left = std::min(o->maxiter, kSmallIter);
+    while (res > target && left > 0 && outer < max_outer && !flag) {
+      if (t->ellW <= 6) cg_small_rows<6>(t, r, d_x, tabs2, left, str);
+      else cg_small_rows<8>(t, r, d_x, tabs2, left, str);
+      if ((rc = true_res<double>(t, d_x, r, str)) || (rc = read_scalars(t, h, str))) return rc;
+      const int it = (int)h[S_ITER];
+      flag = (int)h[S_FLAG];
+      total += it;
+      left -= it;
+      ++outer;
+      res = std::sqrt(h[S_RES2]);
+      if (!(res == res) || it == 0) break;
+    }
+    if (!(res == res)) {
+      hipLaunchKernelGGL(init_x, grid(t), dim3(kRT), 0, str, n, t->fixed, t->b, d_x, 0);
+      if ((rc = true_res<double>(t, d_x, r, str)) || (rc = read_scalars(t, h, str))) return rc;
+      res = std::sqrt(h[S_RES2]);
+    }
+    if (res > target) outer = flag = 0;
+  }
   if (o->method == FVM_SOLVE_AUTO && t->use_ell && n >= kAmgMin && res > target) {
     if (!t->amg_tried) {
       t->amg_tried = true;
@@ -1737,7 +1921,7 @@ int fvm_template_solve(fvm_template* t, const fvm_solve_opts* o, double* d_x, fv
       if (rc) return rc;
     }
     // Jacobi-preconditioned CG finishes what a breakdown or slow convergence leaves
-    int left = std::min(o->maxiter, kAmgMaxIter);
+    int left = std::min(o->maxiter - total, kAmgMaxIter);
     while (t->amg && res > target && left > 0 && outer < max_outer && !flag) {
       int it = 0;
       rc = amg_cg(t, d_x, tabs2, left, str, &it, &flag);

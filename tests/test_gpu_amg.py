@@ -36,9 +36,11 @@ def _mesh(kind):
     return FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, nx, ny, jitter=0.25, seed=11, single_boundary=False)
 
 
-# (19, 21) is below the smallest system, (20, 20) the smallest: one coarse level; (33, 32)
-# just over a tail level of 128 rows; (200, 170) four levels
-@pytest.mark.parametrize("kind", [(19, 21), (20, 20), (33, 32), (200, 170), "stretched", "graded", "hub"], ids=str)
+# up to 3,072 unknowns one workgroup's CG (two, four and six rows a thread: (3, 3), (31, 33),
+# (32, 33), (64, 32) and (48, 64), the most), then the cycle: (439, 7) just over, (200, 170)
+# four levels; hub: rows far beyond the eight slots
+@pytest.mark.parametrize("kind", [(3, 3), (31, 33), (32, 33), (64, 32), (48, 64), (439, 7), (200, 170), "stretched",
+                                  "graded", "hub"], ids=str)
 @pytest.mark.parametrize("D", ["one", "varying"])
 def test_default_steady_solve_matches_a_direct_solution(gpu, kind, D):
     tri = _mesh(kind)
@@ -62,8 +64,8 @@ def test_default_steady_solve_matches_a_direct_solution(gpu, kind, D):
     bound = 1.1 * np.sqrt(np.linalg.norm(v)) * 1e-10 * np.linalg.norm(b)
     x = lu.solve(b)
     assert np.linalg.norm(a.u - x) <= bound + 1e-12 * np.linalg.norm(x)
-    if len(b) >= 400 and kind not in ("stretched", "graded", "hub"):
-        assert a.iters <= 60, a.stats  # Jacobi-preconditioned CG: over 100 from 33 x 32 on
+    if kind == (200, 170):
+        assert a.iters <= 60, a.stats  # Jacobi-preconditioned CG takes hundreds
     assert np.array_equal(FVM.solve(prob).u, a.u)
 
 
