@@ -180,8 +180,8 @@ struct fvm_mesh {
   // meshes above kNodeMeshMax
   int4* node_ent = nullptr;         // [blocks][8]: the triangle's vertices, sorted triangle << 3 |
                                     // first of another tile << 2 | slot (-1: padding)
-  int32_t* node_next = nullptr;     // [blocks] the node's next block, -1: none
-  int32_t* node_bed = nullptr;      // [N] boundary items: first << 8 | count
+  int32_t* node_next = nullptr;     // [blocks] the node's next block, -1: none (behind node_ent)
+  int32_t* node_bed = nullptr;      // [N] boundary items: first << 8 | count (behind node_next)
   int32_t* block_mem = nullptr;     // the lists of blocks
   MeshBlocks blocks;
   int32_t* qflag = nullptr;         // device flag of the pointwise queries (run_flagged)

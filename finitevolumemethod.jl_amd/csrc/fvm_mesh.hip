@@ -7,7 +7,9 @@
 // shape-function determinant cancels badly on small triangles far from the
 // origin, so any other evaluation order changes s1..s9 well above 1e-12.
 #include <algorithm>
+#include <array>
 #include <cstring>
+#include <future>
 #include <vector>
 
 #include "fvm_internal.hpp"
@@ -134,7 +136,7 @@ void free_mesh(fvm_mesh* m) {
                   m->fix_part_start, m->fix_bedge_start, m->fix_bedge, m->fix_bvert_start,
                   m->fix_bvert, m->lcv, m->node_tri_start,
                   m->node_tri, m->bedges, m->badj, m->perm, m->is_vertex, m->qflag,
-                  m->node_ent, m->node_next, m->node_bed, m->block_mem};
+                  m->node_ent, m->block_mem};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete m;
@@ -180,11 +182,15 @@ bool convex_domain(const fvm_mesh_desc* d) {
 
 // The per-node incidences of node_kernel: blocks of eight in ascending triangle order, a
 // node's first block its own index, further ones after all nodes'.
-int node_lists(const fvmh_tiles* tl, fvm_mesh* m) {
-  const int64_t N = m->N, T = m->T;
+struct NodeLists {
+  std::vector<int4> ent;
+  std::vector<int32_t> next, bed;  // empty: no lists
+};
+NodeLists node_lists(const fvmh_tiles* tl) {
+  const int64_t N = tl->n_points, T = tl->n_tri;
   constexpr int L = 8;
   std::vector<int32_t> tile_of(T), next(N, -1), bed(N, 0);
-  for (int32_t k = 0; k < m->n_tiles; ++k)
+  for (int32_t k = 0; k < tl->n_tiles; ++k)
     for (int32_t s = tl->tile_tri_start[k]; s < tl->tile_tri_start[k + 1]; ++s) tile_of[s] = k;
   std::vector<int4> ent((size_t)N * L);
   for (int64_t g = 0; g < N; ++g) {
@@ -207,23 +213,25 @@ int node_lists(const fvmh_tiles* tl, fvm_mesh* m) {
       e.w = s << 3 | (int)fresh << 2 | (tl->node_tri[k] & 3);
     }
   }
-  for (int32_t f = 0; f < m->n_fix; ++f) {
+  for (int32_t f = 0; f < tl->n_fix; ++f) {
     const int32_t b0 = tl->fix_bedge_start[f], nb = tl->fix_bedge_start[f + 1] - b0;
-    if (nb > 255 || b0 >= 1 << 23) return FVM_OK;  // no lists: the tile kernels
+    if (nb > 255 || b0 >= 1 << 23) return {};  // the tile kernels
     bed[tl->fix_nodes[f]] = b0 << 8 | nb;
   }
-  int rc = upload(&m->node_ent, ent.data(), (int64_t)ent.size());
-  if (rc == FVM_OK) rc = upload(&m->node_next, next.data(), (int64_t)next.size());
-  if (rc == FVM_OK) rc = upload(&m->node_bed, bed.data(), N);
-  return rc;
+  return {std::move(ent), std::move(next), std::move(bed)};
 }
 
-// The lists of MeshBlocks; none (m->blocks.n = 0) when a block would not fit its bounds.
+// The lists of MeshBlocks; none (n = 0) when a block would not fit its bounds.
 // Blocks are runs of the nodes in the order in which the triangles, sorted along a
 // space-filling curve, first reach them: compact patches, whatever the numbering.
-int mesh_blocks(const fvmh_tiles* tl, fvm_mesh* m) {
+struct BlockLists {
+  int64_t n = 0;
+  std::vector<int32_t> all;   // inc, node, bitem, deg, more, tri, loc, halo, item, iloc, rest
+  std::array<int64_t, 11> at;  // where each begins
+};
+BlockLists mesh_blocks(const fvmh_tiles* tl) {
   constexpr int NB = kBlockNodes, NT = 2 * kBlockTris, NH = kBlockHalo, NI = kBlockItems;
-  const int64_t N = m->N, T = m->T;
+  const int64_t N = tl->n_points, T = tl->n_tri;
   const int32_t* tri = tl->tri_sorted;
   std::vector<int32_t> pos(N, -1), order;
   order.reserve(N);
@@ -235,21 +243,23 @@ int mesh_blocks(const fvmh_tiles* tl, fvm_mesh* m) {
   for (int64_t g = 0; g < N; ++g)
     if (pos[g] < 0) pos[g] = (int32_t)order.size(), order.push_back((int32_t)g);
   std::vector<int32_t> tile_of(T), fix_of(N, -1);
-  for (int32_t k = 0; k < m->n_tiles; ++k)
+  for (int32_t k = 0; k < tl->n_tiles; ++k)
     for (int32_t s = tl->tile_tri_start[k]; s < tl->tile_tri_start[k + 1]; ++s) tile_of[s] = k;
-  for (int32_t f = 0; f < m->n_fix; ++f) fix_of[tl->fix_nodes[f]] = f;
+  for (int32_t f = 0; f < tl->n_fix; ++f) fix_of[tl->fix_nodes[f]] = f;
 
+  BlockLists out;
   const int64_t n = (N + NB - 1) / NB;
-  // all lists in one array, rest behind the others
   const int64_t per[] = {NB * 4, NB, NB, NB, NB, NT, NT, NH, NI, NI};
-  int64_t at[11] = {0};
+  auto& at = out.at;
+  at[0] = 0;
   for (int k = 0; k < 10; ++k) at[k + 1] = at[k] + n * per[k];
-  std::vector<int32_t> all(at[10], 0);
+  std::vector<int32_t>& all = out.all;
+  all.assign(at[10], 0);
   uint16_t* inc = (uint16_t*)all.data();
   int32_t *node = &all[at[1]], *bitem = &all[at[2]], *deg = &all[at[3]], *more = &all[at[4]], *btri = &all[at[5]],
           *loc = &all[at[6]], *halo = &all[at[7]], *item = &all[at[8]], *iloc = &all[at[9]];
   for (int32_t* p : {node, btri, halo, item}) {
-    const int64_t* k = std::find(at, at + 10, p - all.data());
+    const int64_t* k = std::find(at.data(), at.data() + 10, p - all.data());
     std::fill(p, p + (k[1] - k[0]), -1);
   }
   std::vector<int32_t> rest;
@@ -278,13 +288,13 @@ int mesh_blocks(const fvmh_tiles* tl, fvm_mesh* m) {
             if (local(h) >= 0 && local(h) < NB) continue;
             inner = false;
             if (local(h) >= 0) continue;
-            if (n_halo == NH) return FVM_OK;
+            if (n_halo == NH) return {};
             halo_in[h] = (int32_t)b;
             halo_at[h] = n_halo;
             halo[b * NH + n_halo++] = pos[h];
           }
           if (inner && n_in == kBlockTris) inner = false;
-          if (!inner && n_out == kBlockTris) return FVM_OK;
+          if (!inner && n_out == kBlockTris) return {};
           tri_in[s] = (int32_t)b;
           tri_at[s] = inner ? n_in++ : kBlockTris + n_out++;
           btri[b * NT + tri_at[s]] = s;
@@ -297,20 +307,27 @@ int mesh_blocks(const fvmh_tiles* tl, fvm_mesh* m) {
       }
       if (fix_of[g] < 0) continue;
       const int32_t b0 = tl->fix_bedge_start[fix_of[g]], b1 = tl->fix_bedge_start[fix_of[g] + 1];
-      if (n_item + (b1 - b0) > NI || b1 - b0 > 255) return FVM_OK;
+      if (n_item + (b1 - b0) > NI || b1 - b0 > 255) return {};
       bitem[p] = n_item << 8 | (b1 - b0);
       for (int32_t q = b0; q < b1; ++q, ++n_item) {
         item[b * NI + n_item] = tl->fix_bedge[q];
         iloc[b * NI + n_item] = vertices(tl->badj_sorted[tl->fix_bedge[q] >> 1]);
-        if (iloc[b * NI + n_item] < 0) return FVM_OK;  // a boundary edge beside a triangle without its node
+        if (iloc[b * NI + n_item] < 0) return {};  // a boundary edge beside a triangle without its node
       }
     }
   }
   all.insert(all.end(), rest.begin(), rest.end());
-  const int rc = upload(&m->block_mem, all.data(), (int64_t)all.size());
+  out.n = n;
+  return out;
+}
+
+int upload_blocks(const BlockLists& b, fvm_mesh* m) {
+  if (b.n == 0) return FVM_OK;
+  const int rc = upload(&m->block_mem, b.all.data(), (int64_t)b.all.size());
   if (rc != FVM_OK) return rc;
   MeshBlocks& B = m->blocks;
-  B.n = (int32_t)n;
+  const auto& at = b.at;
+  B.n = (int32_t)b.n;
   B.inc = (const uint16_t*)m->block_mem;
   B.node = m->block_mem + at[1];
   B.bitem = m->block_mem + at[2];
@@ -360,6 +377,11 @@ int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
             "fvm_mesh_create: mesh too large (the node and tile-node arrays must stay below 4 GiB: "
             "at most 536,870,911 points and tile-node slots)");
   int rc;
+  // made beside the uploads and the geometry kernels
+  std::future<NodeLists> nodes;
+  std::future<BlockLists> blocks;
+  if (N <= kNodeMeshMax) nodes = std::async(node_lists, (const fvmh_tiles*)tl);
+  if (N <= 65536 && !tri_group) blocks = std::async(mesh_blocks, (const fvmh_tiles*)tl);
 #define UP(dst, src, n) \
   if ((rc = upload(&(dst), src, n)) != FVM_OK) return rc
   UP(m->x, d->x, N);
@@ -396,8 +418,6 @@ int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
   UP(m->lcv, (const double*)nullptr, m->n_local);
   UP(m->qflag, (const int32_t*)nullptr, 1);
 #undef UP
-  if (N <= kNodeMeshMax && (rc = node_lists(tl, m)) != FVM_OK) return rc;
-  if (N <= 65536 && !tri_group && (rc = mesh_blocks(tl, m)) != FVM_OK) return rc;
   m->convex = convex_domain(d);
   m->n_bedge_items = tl->fix_bedge_start[m->n_fix];
   m->n_bvert_items = tl->fix_bvert_start[m->n_fix];
@@ -422,6 +442,19 @@ int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
   if (e == hipSuccess) e = hipDeviceSynchronize();
   (void)hipFree(sub);
   if (e != hipSuccess) return hip_fail(e, "fvm_mesh_create: geometry kernels");
+  if (nodes.valid()) {
+    const NodeLists L = nodes.get();
+    if (!L.bed.empty()) {  // in one array
+      std::vector<int32_t> all(4 * L.ent.size());
+      memcpy(all.data(), L.ent.data(), sizeof(int4) * L.ent.size());
+      all.insert(all.end(), L.next.begin(), L.next.end());
+      all.insert(all.end(), L.bed.begin(), L.bed.end());
+      if ((rc = upload((int32_t**)&m->node_ent, all.data(), (int64_t)all.size())) != FVM_OK) return rc;
+      m->node_next = (int32_t*)(m->node_ent + L.ent.size());
+      m->node_bed = m->node_next + L.next.size();
+    }
+  }
+  if (blocks.valid() && (rc = upload_blocks(blocks.get(), m)) != FVM_OK) return rc;
   return FVM_OK;
 }
 
