@@ -85,10 +85,6 @@ KArgs make_args(const fvm_ctx* c) {
   a.bflux = c->bflux;
   a.n_bitems = m->n_bedge_items;
   a.t = 0;
-  a.N = m->N;
-  a.node_ent = m->node_ent;
-  a.node_next = m->node_next;
-  a.node_bed = m->node_bed;
   a.tile_dt = a.dtv = nullptr;
   return a;
 }
@@ -131,7 +127,7 @@ void launch_fix(const KArgs& a, hipStream_t s) {
 }
 
 template <int FK, int MODE>
-int launch_fk(const KArgs& a, int tile_tris, hipStream_t s) {
+int launch_fk(const fvm_mesh* m, const KArgs& a, hipStream_t s) {
   if constexpr (MODE != M_EULER) {
     // One launch by nodes up to the size where its threefold fluxes cost more than the
     // second launch.  Measured, us, node against tile kernels (RHS of a quadratic D(u)):
@@ -140,13 +136,15 @@ int launch_fk(const KArgs& a, int tile_tris, hipStream_t s) {
     // per triangle 7.5 / 8.9 at 28,900 and 9.9 / 8.9 at 40,000; with pow in every edge's
     // flux 8.4 / 11.1 at 14,400 and 11.9 / 11.2 at 28,900.
     constexpr int64_t kMost = FK == FVM_FLUX_D_POWER ? 20000 : (FK == FVM_FLUX_LINEAR ? 32000 : kNodeMeshMax);
-    if (a.node_ent && a.N <= kMost) {
-      hipLaunchKernelGGL((node_kernel<FK, MODE>), dim3((unsigned)((a.N * kNodeLanes + 255) / 256)), dim3(256), 0, s, a);
+    if (m->node_ent && m->N <= kMost) {
+      const NodeArgs nodes = {m->N, m->node_ent, m->node_next, m->node_bed};
+      hipLaunchKernelGGL((node_kernel<FK, MODE>), dim3((unsigned)((m->N * kNodeLanes + 255) / 256)), dim3(256), 0, s, a,
+                         nodes);
       FVM_HIP(hipGetLastError());
       return FVM_OK;
     }
   }
-  launch_tiles<FK, MODE>(a, tile_tris, s);
+  launch_tiles<FK, MODE>(a, m->tile_tris, s);
   launch_fix<FK, MODE>(a, s);
   FVM_HIP(hipGetLastError());
   return FVM_OK;
@@ -166,11 +164,11 @@ template <int MODE>
 int launch(const fvm_ctx* c, const KArgs& a, hipStream_t s) {
   switch (c->flux_kind) {
     case FVM_FLUX_JIT: return launch_jit(c, a, MODE, s);
-    case FVM_FLUX_D_POLY_U: return launch_fk<FVM_FLUX_D_POLY_U, MODE>(a, c->m->tile_tris, s);
-    case FVM_FLUX_D_NODAL: return launch_fk<FVM_FLUX_D_NODAL, MODE>(a, c->m->tile_tris, s);
-    case FVM_FLUX_LINEAR: return launch_fk<FVM_FLUX_LINEAR, MODE>(a, c->m->tile_tris, s);
-    case FVM_FLUX_D_POWER: return launch_fk<FVM_FLUX_D_POWER, MODE>(a, c->m->tile_tris, s);
-    default: return launch_fk<FVM_FLUX_D_EDGE, MODE>(a, c->m->tile_tris, s);
+    case FVM_FLUX_D_POLY_U: return launch_fk<FVM_FLUX_D_POLY_U, MODE>(c->m, a, s);
+    case FVM_FLUX_D_NODAL: return launch_fk<FVM_FLUX_D_NODAL, MODE>(c->m, a, s);
+    case FVM_FLUX_LINEAR: return launch_fk<FVM_FLUX_LINEAR, MODE>(c->m, a, s);
+    case FVM_FLUX_D_POWER: return launch_fk<FVM_FLUX_D_POWER, MODE>(c->m, a, s);
+    default: return launch_fk<FVM_FLUX_D_EDGE, MODE>(c->m, a, s);
   }
 }
 

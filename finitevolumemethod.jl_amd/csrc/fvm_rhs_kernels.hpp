@@ -59,10 +59,6 @@ struct KArgs {
   const double* lcv;     // per local entry: control volume
   double* bflux;         // boundary terms per work item
   double t;
-  int64_t N;
-  const int4* node_ent;     // per node kNodeLanes incidences (node_kernel), or null
-  const int32_t* node_next; // per block of them the node's next one, -1: none
-  const int32_t* node_bed;  // per node its boundary items: first << 8 | count
   const double* tile_dt;  // M_EULER: time step of each tile's nodes
   const double* dtv;      // M_EULER: time step per node (fix-up nodes)
 };
@@ -622,15 +618,23 @@ struct NodeSum {
 // so the results are the same bit for bit.  2,500 nodes: 7.6 -> 3.8 us a call (a plain
 // empty launch 2.6).  Lanes by triangle rather than by node spread the loads of a node
 // over a wave; eight cover the interior nodes of a usual mesh in one pass.
+// (The lists are an argument of their own: 32 more bytes of KArgs cost the tile kernels
+// 1 % of a call at 155,701 nodes.)
 constexpr int kNodeLanes = 8;
+struct NodeArgs {
+  int64_t N;
+  const int4* ent;      // per node kNodeLanes incidences
+  const int32_t* next;  // per block of them the node's next one, -1: none
+  const int32_t* bed;   // per node its boundary items: first << 8 | count
+};
 template <int FK, int MODE>
-__global__ __launch_bounds__(256) void node_kernel(KArgs a) {
+__global__ __launch_bounds__(256) void node_kernel(KArgs a, NodeArgs nodes) {
   static_assert(kGeo >= 3, "the whole record rebuilt from the coordinates");
   const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
   const int lane = threadIdx.x % kNodeLanes;
-  const int g = (int)(q / kNodeLanes < a.N ? q / kNodeLanes : a.N - 1);
-  int4 w = a.node_ent[(long long)g * kNodeLanes + lane];
-  const int bed = a.node_bed[g];
+  const int g = (int)(q / kNodeLanes < nodes.N ? q / kNodeLanes : nodes.N - 1);
+  int4 w = nodes.ent[(long long)g * kNodeLanes + lane];
+  const int bed = nodes.bed[g];
   const double ug = a.u[g], V = a.cv[g];
   const double vg = MODE == M_JVP ? a.v[g] : 0.0;
   const int c = a.code[g];
@@ -680,9 +684,9 @@ __global__ __launch_bounds__(256) void node_kernel(KArgs a) {
     FVM_NODE_ADD(6);
     FVM_NODE_ADD(7);
 #undef FVM_NODE_ADD
-    blk = m8 == 255u ? a.node_next[blk] : -1;  // only a full block may go on
+    blk = m8 == 255u ? nodes.next[blk] : -1;  // only a full block may go on
     if (!__any(blk >= 0)) break;
-    w = blk >= 0 ? a.node_ent[(long long)blk * kNodeLanes + lane] : make_int4(g, g, g, -1);
+    w = blk >= 0 ? nodes.ent[(long long)blk * kNodeLanes + lane] : make_int4(g, g, g, -1);
     if (blk < 0) blk = g;
   }
   double acc = S.value();
@@ -698,7 +702,7 @@ __global__ __launch_bounds__(256) void node_kernel(KArgs a) {
       if (k0 + k < nb) acc = acc - b;
     }
   }
-  if (lane == 0 && q / kNodeLanes < a.N) a.out[g] = finish_pre<FK, MODE>(a, g, acc, ug, vg, c, V, 0.0);
+  if (lane == 0 && q / kNodeLanes < nodes.N) a.out[g] = finish_pre<FK, MODE>(a, g, acc, ug, vg, c, V, 0.0);
 }
 
 // ---------------------------------------------------------------------------
