@@ -79,3 +79,18 @@ def test_a_singular_system_ends_as_it_does_with_jacobi(gpu):
 
     a, b = FVM.solve(prob, maxiter=500), FVM.solve(prob, CG(), maxiter=500)
     assert a.retcode == b.retcode == "MaxIters" and np.all(np.isfinite(a.u))
+
+
+def test_a_source_of_one_mode_needs_no_cycle(gpu):
+    """sin(pi x) sin(pi y) on a uniform grid is an eigenvector of the scaled operator: the
+    Jacobi-preconditioned steps before the cycle meet the target, as CG() does."""
+    from finitevolumemethod import CG
+
+    tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 70, 70, single_boundary=True)
+    mesh = FVM.FVMGeometry(tri)
+    prob = FVM.PoissonsEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.0 * x, FVM.Dirichlet),
+                                source_function=lambda x, y, p: -np.sin(np.pi * x) * np.sin(np.pi * y))
+    a, b = FVM.solve(prob), FVM.solve(prob, CG())
+    assert a.retcode == "Success" and a.resid <= 1e-10 and a.iters <= 3
+    # both residuals are below 1e-10 |b| and |A^-1| <= 1 / (2 pi^2) here, up to the grid's error
+    assert np.linalg.norm(a.u - b.u) <= 2e-10 * np.linalg.norm(prob.b) / 19.0 + 1e-12 * np.linalg.norm(b.u)
