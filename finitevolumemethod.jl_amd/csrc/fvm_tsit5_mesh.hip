@@ -10,7 +10,7 @@
 // Triangles between blocks are formed in each: a sixth more fluxes, and no partial sums to
 // exchange.  The exchange is what a stage waits for (2 us and more), then the fluxes' and
 // sums' chains; the same loop as kernels was bound by about 20 launches a step: 63 steps
-// at 62,451 nodes (D(u) quadratic) 7.0 -> 2.1 ms a solve, 1.3 ms of it this kernel (20 us
+// at 62,451 nodes (D(u) quadratic) 7.0 -> 1.4 ms a solve, 1.3 ms of it this kernel (20 us
 // a step); 10 steps at 1,600 nodes 1.38 -> 0.54 ms, at 144 nodes (one workgroup, no
 // exchange) 0.90 -> 0.31 ms.  Every size it takes is the faster form.
 //

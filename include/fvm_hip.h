@@ -288,8 +288,8 @@ enum {
   FVM_SOLVE_BICGSTAB = 2, /* FP64 Jacobi-BiCGStab on M */
   FVM_SOLVE_CG_RELIABLE = 3, /* one FP32 Jacobi-PCG sequence with FP64 reliable updates of x and the residual */
   FVM_SOLVE_AUTO = 4      /* FP64 CG on M preconditioned by smoothed-aggregation multigrid (set up by the first
-                             such solve and kept), FVM_SOLVE_CG for small systems and where that breaks down
-                             or converges slowly */
+                             such solve and kept) above 3,072 unknowns, FVM_SOLVE_CG in one workgroup up to
+                             there and in its own form where that breaks down or converges slowly */
 };
 
 /* Forms of the scaled operator M in the Krylov products: CSR with eight lanes per row, or an ELL
