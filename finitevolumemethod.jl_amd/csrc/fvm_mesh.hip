@@ -9,6 +9,7 @@
 #include <algorithm>
 #include <array>
 #include <cstring>
+#include <exception>
 #include <future>
 #include <vector>
 
@@ -471,7 +472,13 @@ int mesh_create_grouped(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_me
   FVM_CHECK(d->x && d->y && d->triangles, "fvm_mesh_create: null mesh array");
   FVM_CHECK(d->n_boundary_edges == 0 || d->boundary_edges, "fvm_mesh_create: null boundary edges");
   fvm_mesh* m = new fvm_mesh();
-  int rc = build(d, tri_group, m);
+  int rc;
+  try {
+    rc = build(d, tri_group, m);
+  } catch (const std::exception& e) {  // of the lists: no host memory
+    set_error(std::string("fvm_mesh_create: ") + e.what());
+    rc = FVM_ERR_ALLOC;
+  }
   if (rc != FVM_OK) {
     free_mesh(m);
     return rc;

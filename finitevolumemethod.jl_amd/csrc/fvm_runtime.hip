@@ -1,6 +1,7 @@
 // Runtime part of the C ABI: errors, device memory, streams, events.
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -88,7 +89,12 @@ hipError_t dev_alloc(void** p, size_t bytes) {
     }
     if (e != hipSuccess) return e;
   }
-  (*g_live)[b.p] = b;
+  try {
+    (*g_live)[b.p] = b;
+  } catch (const std::exception&) {  // no host memory for the entry
+    (void)hipFree(b.p);
+    return hipErrorOutOfMemory;
+  }
   *p = b.p;
   return hipSuccess;
 }
@@ -115,7 +121,11 @@ hipError_t dev_free(void* p) {
   Block b = it->second;
   g_live->erase(it);
   b.freed = ++g_frees;
-  g_kept->push_back(b);
+  try {
+    g_kept->push_back(b);
+  } catch (const std::exception&) {
+    return hipFree(p);
+  }
   g_kept_bytes += b.bytes;
   // the oldest first (the list is in the order of the frees)
   size_t over = g_kept_bytes > kKeepTotal ? g_kept_bytes - kKeepTotal : 0;
