@@ -149,7 +149,9 @@ struct Grid {
     sh = s;
     vtag = __builtin_amdgcn_readfirstlane((uint32_t)m[kGridVec]);
     rtag = __builtin_amdgcn_readfirstlane((uint32_t)m[kGridSum]);
-    if (threadIdx.x == 0) s->fault = 0;
+    // a fault of an earlier kernel on this memory stands: its exchange numbers are unknown,
+    // so every workgroup gives up after its first sum
+    if (threadIdx.x == 0) s->fault = grid_fault(m) != 0;
     __syncthreads();
   }
   // the numbers the next kernel on this memory starts from (every workgroup has read

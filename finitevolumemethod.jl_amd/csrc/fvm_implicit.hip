@@ -453,7 +453,8 @@ __global__ __launch_bounds__(T) void gmres_kernel(Gm p) {
   double x;
   const int64_t k = gmres<W, T>(S, G, p.J, R, i, active, p.a, p.bj, scale, active ? p.b[i] : 0.0, x, p.rtol,
                                 p.restart, p.maxiter);
-  if (active) p.x[i] = x;
+  // no solution when the grid gave up: the host's norms of x see it at once
+  if (active) p.x[i] = k < 0 ? __longlong_as_double(0x7ff8000000000000ll) : x;
   if (k > 0 && blockIdx.x == 0 && threadIdx.x == 0) p.grid[fvm::kGridUser] += (uint64_t)k;
   G.close();
 }

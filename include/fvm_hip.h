@@ -528,7 +528,8 @@ int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts* o, double*
  * fvm_gmres_ell: x = (a I + b J)^-1 rhs by GMRES(restart <= 30) from x = 0 until
  * |r| <= rtol |rhs|, right-preconditioned by the diagonal when jacobi != 0, in one
  * launch; does not wait.  d_work: fvm_gmres_work_bytes(n) bytes, zeroed before its first
- * use, for one call at a time.
+ * use, for one call at a time.  A call that fails on the device (its workgroups' exchange
+ * timed out) and every later one on that d_work set x to NaN.
  * fvm_gmres_iterations: the iterations of all calls on d_work so far; waits, and fails
  * if one of them did. */
 size_t fvm_gmres_work_bytes(int64_t n);

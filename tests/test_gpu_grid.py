@@ -72,6 +72,41 @@ def test_nonlinear_trbdf2_with_a_frozen_jacobian_matches_the_matrix_free_loop(gp
         assert np.max(np.abs(x - y)) <= 1e-7 * np.max(np.abs(y))
 
 
+def _frozen(nx, ny):
+    from finitevolumemethod import implicit
+
+    tri = FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, nx, ny, jitter=0.2, seed=3)
+    mesh = FVM.FVMGeometry(tri)
+    u0 = 0.5 + 0.4 * np.sin(5 * tri.x) * np.cos(4 * tri.y)
+    prob = FVM.FVMProblem(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.0 * u, FVM.Neumann),
+                          diffusion_function=lambda x, y, t, u, p: 0.1 + u ** 2, initial_condition=u0, final_time=0.01)
+    return prob, implicit.FrozenJacobian.of(prob)
+
+
+@pytest.mark.parametrize("shape", [(5, 4), (61, 47)], ids=str)  # one workgroup, several
+def test_a_failed_gmres_leaves_no_stale_solution(gpu, shape):
+    """The work memory's fault word, set here by the host, as a timed-out exchange leaves it:
+    the solves on that memory give NaN, not what x held, and the count of iterations raises."""
+    from finitevolumemethod import _lib
+
+    prob, J = _frozen(*shape)
+    n = J.n
+    u = FVM.DeviceArray.from_host(prob.initial_condition)
+    J.take(u, 0.0)
+    b, x = FVM.DeviceArray.from_host(np.random.default_rng(0).random(n)), FVM.DeviceArray.from_host(np.full(n, 3.0))
+    J.solve(1.0, -1e-4, b, x, 1e-3, 20, 400, True)
+    assert np.all(np.isfinite(x.to_host())) and J.iterations() > 0
+    w = J.work.to_host()
+    w.view(np.uint64)[2] = 1  # kGridFault
+    J.work.upload(w)
+    for _ in range(2):
+        x.upload(np.full(n, 3.0))
+        J.solve(1.0, -1e-4, b, x, 1e-3, 20, 400, True)
+        assert np.all(np.isnan(x.to_host()))
+    with pytest.raises(_lib.FVMError, match="timed out"):
+        J.iterations()
+
+
 @pytest.mark.parametrize("shape", [(3, 3), (16, 16), (32, 32), (64, 40), (13, 197), (45, 46, 0.25), (64, 32, 0.25),
                                    (90, 80, 0.25), (256, 256), (200, 190, "permuted"), "wheel"], ids=str)
 def test_one_launch_tsit5_is_the_host_loop_bit_for_bit(gpu, shape):
