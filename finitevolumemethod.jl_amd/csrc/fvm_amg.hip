@@ -752,7 +752,7 @@ int amg_build(int64_t n0, const int32_t* rp, const int32_t* col, const double* v
   auto carve = [&](Arena& A, auto&& layout) -> int {  // sizes first, then one allocation
     layout(A);
     const size_t bytes = A.at;
-    FVM_HIP(hipMalloc((void**)&A.base, bytes));
+    FVM_HIP(fvm::dev_malloc((void**)&A.base, bytes));
     A.at = 0;
     layout(A);
     return FVM_OK;
@@ -879,7 +879,7 @@ int amg_build(int64_t n0, const int32_t* rp, const int32_t* col, const double* v
   const AmgLevel& B = a->level[nl - 1];
   if (B.A.n <= kDense) {
     double* inv = nullptr;
-    FVM_HIP(hipMalloc((void**)&inv, sizeof(double) * kDense * kDense));
+    FVM_HIP(fvm::dev_malloc((void**)&inv, sizeof(double) * kDense * kDense));
     a->mem.push_back(inv);
     a->inverse = inv;
     hipLaunchKernelGGL(invert_kernel, dim3(1), dim3(1024), 0, st, B.A, inv);

@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void euler_update(int64_t n, double* __restric
 template <class T>
 int dcopy(T** dst, const T* src, int64_t n) {
   *dst = nullptr;
-  FVM_HIP(hipMalloc((void**)dst, sizeof(T) * (size_t)(n > 0 ? n : 1)));
+  FVM_HIP(fvm::dev_malloc((void**)dst, sizeof(T) * (size_t)(n > 0 ? n : 1)));
   if (n > 0 && src) FVM_HIP(hipMemcpy(*dst, src, sizeof(T) * (size_t)n, hipMemcpyHostToDevice));
   return FVM_OK;
 }

@@ -43,8 +43,10 @@ namespace fvm {
 void set_error(const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
 
-// Device memory by way of the kept blocks (fvm_runtime.hip); dev_free takes any pointer of
-// hipMalloc too, and waits for the device.
+// Device memory (fvm_runtime.hip).  dev_malloc: hipMalloc, the kept blocks given back where it
+// would fail; freed by hipFree.  dev_alloc: by way of the kept blocks; freed by dev_free, which
+// takes any pointer of hipMalloc too and waits for the device.
+hipError_t dev_malloc(void** p, size_t bytes);
 hipError_t dev_alloc(void** p, size_t bytes);
 hipError_t dev_free(void* p);
 // fvm_mesh_create with the triangles of each tri_group kept contiguous (NULL: one group)

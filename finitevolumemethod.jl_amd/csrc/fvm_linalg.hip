@@ -1055,7 +1055,7 @@ __global__ __launch_bounds__(kRT) void spmv_ell_kernel(int64_t n, SellIdx S, con
 template <class T>
 int dalloc(T** dst, int64_t n) {
   *dst = nullptr;
-  FVM_HIP(hipMalloc((void**)dst, sizeof(T) * (size_t)(n > 0 ? n : 1)));
+  FVM_HIP(fvm::dev_malloc((void**)dst, sizeof(T) * (size_t)(n > 0 ? n : 1)));
   return FVM_OK;
 }
 

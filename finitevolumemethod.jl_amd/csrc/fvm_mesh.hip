@@ -23,7 +23,7 @@ template <class T>
 int upload(T** dst, const T* src, int64_t n) {
   *dst = nullptr;
   size_t bytes = sizeof(T) * (size_t)(n > 0 ? n : 1);
-  FVM_HIP(hipMalloc((void**)dst, bytes));
+  FVM_HIP(fvm::dev_malloc((void**)dst, bytes));
   if (n > 0 && src) FVM_HIP(hipMemcpy(*dst, src, sizeof(T) * (size_t)n, hipMemcpyHostToDevice));
   return FVM_OK;
 }
@@ -429,7 +429,7 @@ int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
   m->h_fix_part_start.assign(tl->fix_part_start, tl->fix_part_start + m->n_fix + 1);
   m->h_fix_bedge_start.assign(tl->fix_bedge_start, tl->fix_bedge_start + m->n_fix + 1);
   double* sub = nullptr;
-  FVM_HIP(hipMalloc((void**)&sub, sizeof(double) * 3 * (size_t)(T > 0 ? T : 1)));
+  FVM_HIP(fvm::dev_malloc((void**)&sub, sizeof(double) * 3 * (size_t)(T > 0 ? T : 1)));
   if (T > 0)
     hipLaunchKernelGGL(geometry_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, 0, T, m->tri,
                        m->x, m->y, m->props, sub);
@@ -534,7 +534,7 @@ int fvm_mesh_rebuilt_geometry(const fvm_mesh* m, double* props) {
   FVM_CHECK(m && props, "fvm_mesh_rebuilt_geometry: null argument");
   const int64_t T = m->T;
   double* d = nullptr;
-  FVM_HIP(hipMalloc((void**)&d, sizeof(double) * (size_t)P_COUNT * T));
+  FVM_HIP(fvm::dev_malloc((void**)&d, sizeof(double) * (size_t)P_COUNT * T));
   hipLaunchKernelGGL(rebuild_kernel, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, 0, T, m->tri, m->x,
                      m->y, d);
   std::vector<double> soa((size_t)P_COUNT * T);

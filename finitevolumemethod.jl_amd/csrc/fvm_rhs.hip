@@ -190,7 +190,7 @@ int launch_vjp_fk(const KArgs& a, int tile_tris, hipStream_t s) {
 template <class T>
 int dev_copy(T** dst, const T* src, int64_t n) {
   *dst = nullptr;
-  FVM_HIP(hipMalloc((void**)dst, sizeof(T) * (size_t)(n > 0 ? n : 1)));
+  FVM_HIP(fvm::dev_malloc((void**)dst, sizeof(T) * (size_t)(n > 0 ? n : 1)));
   if (n > 0 && src) FVM_HIP(hipMemcpy(*dst, src, sizeof(T) * (size_t)n, hipMemcpyHostToDevice));
   return FVM_OK;
 }

@@ -25,8 +25,20 @@ const std::string& last_error() { return g_last_error; }
 // gradient of 10^6 nodes, whose five arrays come and go with each call, 213 -> 110 us.
 // A free waits for the device first, as hipFree does, so whatever stream used the block
 // has finished with it and any stream may have it next.  At most 512 MiB are kept, none
-// longer than the next 64 frees, and all are given back when an allocation would fail.
+// longer than the next 64 frees, and all are given back when an allocation of the library
+// would fail (dev_malloc, for every array).
 namespace {
+thread_local int64_t g_fail_after = 0, g_fail_count = 0;  // fvm_test_fail_allocations
+hipError_t raw_malloc(void** p, size_t bytes) {
+  if (g_fail_after > 0) {
+    --g_fail_after;
+  } else if (g_fail_count > 0) {
+    --g_fail_count;
+    bytes = (size_t)1 << 60;  // more than any device holds: HIP's own failure
+  }
+  return hipMalloc(p, bytes > 0 ? bytes : 1);
+}
+
 constexpr size_t kKeepMin = (size_t)1 << 20, kKeepMax = (size_t)128 << 20, kKeepTotal = (size_t)512 << 20;
 constexpr uint64_t kKeepFrees = 64;
 struct Block {
@@ -57,38 +69,37 @@ void give_back(F go) {
 }
 }  // namespace
 
+hipError_t dev_malloc(void** p, size_t bytes) {
+  *p = nullptr;
+  const hipError_t e = raw_malloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  {
+    std::lock_guard<std::mutex> lock(g_mem);
+    give_back([](const Block&) { return true; });
+  }
+  return raw_malloc(p, bytes);
+}
+
 hipError_t dev_alloc(void** p, size_t bytes) {
   *p = nullptr;
-  if (bytes < kKeepMin || bytes > kKeepMax) {
-    hipError_t e = hipMalloc(p, bytes > 0 ? bytes : 1);
-    if (e != hipErrorOutOfMemory) return e;
-    std::lock_guard<std::mutex> lock(g_mem);
-    if (g_kept->empty()) return e;
-    (void)hipGetLastError();
-    give_back([](const Block&) { return true; });
-    return hipMalloc(p, bytes > 0 ? bytes : 1);
-  }
+  if (bytes < kKeepMin || bytes > kKeepMax) return dev_malloc(p, bytes);
   Block b{nullptr, (bytes + 0xffff) & ~(size_t)0xffff, 0, 0};
   hipError_t e = hipGetDevice(&b.dev);
   if (e != hipSuccess) return e;
-  std::lock_guard<std::mutex> lock(g_mem);
-  for (size_t k = g_kept->size(); k-- > 0;) {
-    const Block& c = (*g_kept)[k];
-    if (c.bytes != b.bytes || c.dev != b.dev) continue;
-    b.p = c.p;
-    g_kept_bytes -= b.bytes;
-    g_kept->erase(g_kept->begin() + (long)k);
-    break;
-  }
-  if (!b.p) {
-    e = hipMalloc(&b.p, b.bytes);
-    if (e == hipErrorOutOfMemory && !g_kept->empty()) {
-      (void)hipGetLastError();
-      give_back([](const Block&) { return true; });
-      e = hipMalloc(&b.p, b.bytes);
+  {
+    std::lock_guard<std::mutex> lock(g_mem);
+    for (size_t k = g_kept->size(); k-- > 0;) {
+      const Block& c = (*g_kept)[k];
+      if (c.bytes != b.bytes || c.dev != b.dev) continue;
+      b.p = c.p;
+      g_kept_bytes -= b.bytes;
+      g_kept->erase(g_kept->begin() + (long)k);
+      break;
     }
-    if (e != hipSuccess) return e;
   }
+  if (!b.p && (e = dev_malloc(&b.p, b.bytes)) != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(g_mem);
   try {
     (*g_live)[b.p] = b;
   } catch (const std::exception&) {  // no host memory for the entry
@@ -139,6 +150,13 @@ hipError_t dev_free(void* p) {
 }  // namespace fvm
 
 extern "C" {
+
+// For tests (not in fvm_hip.h): of the calling thread's following device allocations the first
+// `after` are made as usual and the next `count` attempts fail as without memory.
+void fvm_test_fail_allocations(int64_t after, int64_t count) {
+  fvm::g_fail_after = after;
+  fvm::g_fail_count = count;
+}
 
 int fvm_last_error(char* buf, size_t n) {
   if (!buf || n == 0) return FVM_ERR_ARG;

@@ -506,7 +506,7 @@ __global__ __launch_bounds__(256) void sys_flux_query_kernel(SysArgs a, const in
 template <class T>
 int dcopy(T** dst, const T* src, int64_t n) {
   *dst = nullptr;
-  FVM_HIP(hipMalloc((void**)dst, sizeof(T) * (size_t)(n > 0 ? n : 1)));
+  FVM_HIP(fvm::dev_malloc((void**)dst, sizeof(T) * (size_t)(n > 0 ? n : 1)));
   if (n > 0 && src) FVM_HIP(hipMemcpy(*dst, src, sizeof(T) * (size_t)n, hipMemcpyHostToDevice));
   return FVM_OK;
 }

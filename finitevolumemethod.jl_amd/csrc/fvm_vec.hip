@@ -265,14 +265,14 @@ double* g_mscratch = nullptr;  // kMaxDots * kRedBlocks partials + kMaxDots resu
 
 int red_scratch(double** out) {
   std::lock_guard<std::mutex> lk(g_mu);
-  if (!g_scratch) FVM_HIP(hipMalloc((void**)&g_scratch, sizeof(double) * (kRedBlocks + 8)));
+  if (!g_scratch) FVM_HIP(fvm::dev_malloc((void**)&g_scratch, sizeof(double) * (kRedBlocks + 8)));
   *out = g_scratch;
   return FVM_OK;
 }
 
 int mscratch(double** out) {
   std::lock_guard<std::mutex> lk(g_mu);
-  if (!g_mscratch) FVM_HIP(hipMalloc((void**)&g_mscratch, sizeof(double) * (size_t)kMaxDots * (kRedBlocks + 1)));
+  if (!g_mscratch) FVM_HIP(fvm::dev_malloc((void**)&g_mscratch, sizeof(double) * (size_t)kMaxDots * (kRedBlocks + 1)));
   *out = g_mscratch;
   return FVM_OK;
 }
@@ -333,7 +333,7 @@ int cgs2_norm(int64_t n, int k, const double* const* xs, double* w, double* h_ho
   if (rc || (rc = red_scratch(&red))) return rc;
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (!g_ascratch) FVM_HIP(hipMalloc((void**)&g_ascratch, sizeof(double) * (2 * kMaxDots + 8)));
+    if (!g_ascratch) FVM_HIP(fvm::dev_malloc((void**)&g_ascratch, sizeof(double) * (2 * kMaxDots + 8)));
   }
   std::lock_guard<std::mutex> use(g_use);
   AxpyTerms t;

@@ -1,5 +1,9 @@
 """Device memory of fvm_alloc / fvm_free: blocks of 1 to 128 MiB are kept for the next
-allocation of their size (at most 512 MiB, none longer than 64 frees)."""
+allocation of their size (at most 512 MiB, none longer than 64 frees), and what happens
+when the device has no memory left (the library asks HIP for more than it holds:
+fvm_test_fail_allocations)."""
+import contextlib
+import ctypes
 import threading
 
 import numpy as np
@@ -68,3 +72,50 @@ def test_kept_memory_is_bounded_and_given_back(gpu):
     for _ in range(64):
         FVM.DeviceArray(MiB // 8)
     assert start - _free_bytes() <= 64 * MiB
+
+
+@contextlib.contextmanager
+def _failing(after, count):
+    f = _lib.hip_lib().fvm_test_fail_allocations
+    f.argtypes, f.restype = [ctypes.c_int64, ctypes.c_int64], None
+    f(after, count)
+    try:
+        yield
+    finally:
+        f(0, 0)
+
+
+def _poisson(nx, ny):
+    tri = FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, nx, ny, jitter=0.25, seed=3)
+    mesh = FVM.FVMGeometry(tri)
+    f = np.random.default_rng(1).random(tri.num_points())
+    return FVM.PoissonsEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.0 * x, FVM.Dirichlet),
+                                diffusion_function=lambda x, y, p: 1.0 + x, source_function=lambda x, y, p: p,
+                                source_parameters=f)
+
+
+@pytest.mark.parametrize("what", ["mesh", "template", "context", "hierarchy"])
+def test_kept_blocks_are_given_back_to_every_allocation(gpu, what):
+    """An allocation that fails once has the kept blocks' memory the second time."""
+    prob = _poisson(80, 70)
+    x = FVM.DeviceArray.from_host(np.zeros(len(prob.b)))
+    tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 9, 9, single_boundary=True)
+    mesh = FVM.FVMGeometry(tri)
+    mesh.handle
+    zero = FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.0 * x, FVM.Dirichlet)
+    make = {"mesh": lambda: FVM.FVMGeometry(tri).handle,
+            "template": lambda: FVM.PoissonsEquation(mesh, zero, diffusion_function=lambda x, y, p: 1.0 + x,
+                                                     source_function=lambda x, y, p: x).problem,
+            "context": lambda: FVM.FVMProblem(mesh, zero, diffusion_function=lambda x, y, t, u, p: 0.1 + u ** 2,
+                                              initial_condition=tri.x, final_time=1.0).device_context(),
+            "hierarchy": lambda: prob.problem.solve(x=x)}[what]
+    for _ in range(65):  # what earlier work left
+        FVM.DeviceArray(MiB // 8)
+    blocks = [FVM.DeviceArray(8 * MiB) for _ in range(4)]  # 256 MiB
+    del blocks
+    before = _free_bytes()
+    with _failing(0, 1):
+        made = make()
+    assert _free_bytes() - before >= 192 * MiB  # HIP accounts for memory in chunks of its own
+    if what == "hierarchy":
+        assert made[1]["converged"] and made[1]["iterations"] < 60
