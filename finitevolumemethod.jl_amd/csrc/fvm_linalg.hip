@@ -1933,10 +1933,14 @@ int fvm_template_solve(fvm_template* t, const fvm_solve_opts* o, double* d_x, fv
   }
   if (o->method == FVM_SOLVE_AUTO && t->use_ell && n >= kAmgMin && res > target) {
     if (!t->amg_tried) {
-      t->amg_tried = true;
-      rc = amg_build(n, t->row_ptr, t->col, t->valM, &t->amg, str);
-      if (rc == FVM_ERR_ALLOC) rc = FVM_OK;  // no room for the hierarchy: Jacobi-preconditioned
-      if (rc) return rc;
+      try {
+        rc = amg_build(n, t->row_ptr, t->col, t->valM, &t->amg, str);
+      } catch (const std::exception&) {  // of its lists: no host memory
+        rc = FVM_ERR_ALLOC;
+      }
+      // no room for the hierarchy: this solve Jacobi-preconditioned, the next one tries again
+      t->amg_tried = rc != FVM_ERR_ALLOC;
+      if (rc && t->amg_tried) return rc;
     }
     // Jacobi-preconditioned CG finishes what a breakdown or slow convergence leaves
     int left = std::min(o->maxiter - total, kAmgMaxIter);

@@ -14,6 +14,9 @@ thread_local std::string g_last_error;
 }
 void set_error(const std::string& msg) { g_last_error = msg; }
 int hip_fail(hipError_t e, const char* what) {
+  // reported here: the runtime keeps its last error until it is read, and the next check of a
+  // launch, of a caller that goes on after this failure, would take it for its own
+  (void)hipGetLastError();
   g_last_error = std::string(what) + ": " + hipGetErrorString(e);
   return e == hipErrorOutOfMemory ? FVM_ERR_ALLOC : FVM_ERR_HIP;
 }

@@ -94,6 +94,27 @@ def _poisson(nx, ny):
                                 source_parameters=f)
 
 
+# the hierarchy's allocations one after the other: the scratch, the first level, the next ones
+@pytest.mark.parametrize("after", [0, 1, 2, 4])
+def test_no_room_for_the_hierarchy(gpu, after):
+    """The default steady solve without memory for the multigrid hierarchy is the
+    Jacobi-preconditioned one, not an error, and the next solve uses the cycle again."""
+    from finitevolumemethod import CG
+
+    prob = _poisson(80, 70)
+    n = len(prob.b)
+    x = FVM.DeviceArray.from_host(np.zeros(n))
+    with _failing(after, 1000):
+        _, st = prob.problem.solve(x=x)
+    ref = FVM.solve(prob, CG())
+    assert st["converged"] and st["iterations"] > 60  # the cycle takes under 60, Jacobi some 150
+    # both residuals are below 1e-10 |b|; |A^-1| <= 1 / (2 pi^2) for D >= 1, 0.06 with the mesh's error
+    bound = 2e-10 * 0.06 * np.linalg.norm(prob.b)
+    assert np.linalg.norm(x.to_host() - ref.u) <= bound
+    again = FVM.solve(prob)
+    assert again.retcode == "Success" and again.iters < 60 and np.linalg.norm(again.u - ref.u) <= bound
+
+
 @pytest.mark.parametrize("what", ["mesh", "template", "context", "hierarchy"])
 def test_kept_blocks_are_given_back_to_every_allocation(gpu, what):
     """An allocation that fails once has the kept blocks' memory the second time."""
@@ -119,3 +140,11 @@ def test_kept_blocks_are_given_back_to_every_allocation(gpu, what):
     assert _free_bytes() - before >= 192 * MiB  # HIP accounts for memory in chunks of its own
     if what == "hierarchy":
         assert made[1]["converged"] and made[1]["iterations"] < 60
+
+
+def test_a_reported_failure_leaves_no_error_behind(gpu):
+    """What a caller does after a failed allocation is not taken for that failure."""
+    u = FVM.DeviceArray.from_host(np.ones(100))
+    with _failing(0, 1000), pytest.raises(_lib.FVMError, match="memory"):
+        FVM.DeviceArray(16 * MiB)
+    assert _lib.dot(u, u) == 100.0
