@@ -488,24 +488,34 @@ EllJ ell_of(const fvm_affine_op* op) {
   return J;
 }
 
-// Launches kernel<W, kRows> cooperatively for an operator of n rows and ELL width w, the
-// widths of triangle meshes as compile-time constants, others at run time.
-#define FVM_TRB_LAUNCH(kernel, w, n, args, st)                                                           \
-  ([&]() -> hipError_t {                                                                                \
-    const void* f_ = nullptr;                                                                           \
-    switch (w) {                                                                                        \
-      case 4: f_ = (const void*)kernel<4, kRows>; break;                                                \
-      case 5: f_ = (const void*)kernel<5, kRows>; break;                                                \
-      case 6: f_ = (const void*)kernel<6, kRows>; break;                                                \
-      case 7: f_ = (const void*)kernel<7, kRows>; break;                                                \
-      case 8: f_ = (const void*)kernel<8, kRows>; break;                                                \
-      case 9: f_ = (const void*)kernel<9, kRows>; break;                                                \
-      case 10: f_ = (const void*)kernel<10, kRows>; break;                                              \
-      default: f_ = (const void*)kernel<0, kRows>;                                                      \
-    }                                                                                                   \
-    void* p_[] = {&(args)};                                                                             \
-    return hipLaunchCooperativeKernel(f_, dim3((unsigned)(((n) + kRows - 1) / kRows)), dim3(kRows), p_, 0, (st)); \
-  }())
+// kernel<W, kRows> for an operator of ELL width w: the widths of triangle meshes as
+// compile-time constants, others at run time.
+#define FVM_TRB_KERNEL(kernel, w)                            \
+  ((w) == 4    ? (const void*)kernel<4, kRows>               \
+   : (w) == 5  ? (const void*)kernel<5, kRows>               \
+   : (w) == 6  ? (const void*)kernel<6, kRows>               \
+   : (w) == 7  ? (const void*)kernel<7, kRows>               \
+   : (w) == 8  ? (const void*)kernel<8, kRows>               \
+   : (w) == 9  ? (const void*)kernel<9, kRows>               \
+   : (w) == 10 ? (const void*)kernel<10, kRows>              \
+               : (const void*)kernel<0, kRows>)
+
+int64_t workgroups(int64_t n) { return (n + kRows - 1) / kRows; }
+
+// FVM_ERR_STATE where the device does not hold the kernel's workgroups for n rows at once
+int check_fits(const void* kernel, int64_t n, const char* who) {
+  bool fits;
+  FVM_HIP(fvm::grid_fits(kernel, kRows, workgroups(n), &fits));
+  if (fits) return FVM_OK;
+  fvm::set_error(std::string(who) + ": the device does not hold a workgroup per 256 unknowns at once");
+  return FVM_ERR_STATE;
+}
+
+template <class Args>
+hipError_t launch(const void* kernel, int64_t n, Args& a, hipStream_t s) {
+  void* p[] = {&a};
+  return hipLaunchCooperativeKernel(kernel, dim3((unsigned)workgroups(n)), dim3(kRows), p, 0, s);
+}
 
 int check_op(const fvm_affine_op* op, const char* who) {
   FVM_CHECK(op->n > 0 && op->n <= kMaxN, std::string(who) + ": 1 <= n <= 65536");
@@ -531,6 +541,8 @@ int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts* o, double*
             "fvm_trbdf2_affine: bad options");
   FVM_CHECK(o->n_save >= 0 && (o->n_save == 0 || (o->save_t && o->d_saves)), "fvm_trbdf2_affine: save times");
   const int64_t n = op->n;
+  const void* const kernel = FVM_TRB_KERNEL(trbdf2_affine_kernel, op->width);
+  if ((rc = check_fits(kernel, n, "fvm_trbdf2_affine"))) return rc;
   Trb a;
   a.J = ell_of(op);
   a.c = op->d_c;
@@ -563,7 +575,7 @@ int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts* o, double*
   hipError_t e = hipMemsetAsync(base, 0, sizeof(double) * words, st_);
   if (e == hipSuccess && o->n_save > 0)
     e = hipMemcpyAsync(tail, o->save_t, sizeof(double) * (size_t)o->n_save, hipMemcpyHostToDevice, st_);
-  if (e == hipSuccess) e = FVM_TRB_LAUNCH(trbdf2_affine_kernel, a.J.W, n, a, st_);
+  if (e == hipSuccess) e = launch(kernel, n, a, st_);
   if (e == hipSuccess) e = hipMemcpyAsync(r, a.stats, sizeof r, hipMemcpyDeviceToHost, st_);
   if (e == hipSuccess) e = hipStreamSynchronize(st_);
   (void)fvm::dev_free(base);
@@ -594,6 +606,8 @@ int fvm_gmres_ell(const fvm_affine_op* op, double a, double b, int32_t jacobi, c
   if (rc) return rc;
   FVM_CHECK(restart >= 1 && restart <= kMaxRestart, "fvm_gmres_ell: restart 1..30");
   FVM_CHECK(rtol > 0 && maxiter > 0, "fvm_gmres_ell: rtol and maxiter must be positive");
+  const void* const kernel = FVM_TRB_KERNEL(gmres_kernel, op->width);
+  if ((rc = check_fits(kernel, op->n, "fvm_gmres_ell"))) return rc;
   Gm g;
   g.J = ell_of(op);
   g.a = a;
@@ -605,7 +619,21 @@ int fvm_gmres_ell(const fvm_affine_op* op, double a, double b, int32_t jacobi, c
   g.restart = restart;
   g.maxiter = maxiter;
   g.grid = (uint64_t*)d_work;
-  FVM_HIP(FVM_TRB_LAUNCH(gmres_kernel, g.J.W, g.J.n, g, (hipStream_t)s));
+  FVM_HIP(launch(kernel, g.J.n, g, (hipStream_t)s));
+  return FVM_OK;
+}
+
+int fvm_ell_resident(int64_t n, int32_t* fits) {
+  FVM_CHECK(fits, "fvm_ell_resident: null output");
+  *fits = 0;
+  if (n <= 0 || n > kMaxN) return FVM_OK;
+  for (int w : {0, 4, 5, 6, 7, 8, 9, 10}) {
+    bool a, b;
+    FVM_HIP(fvm::grid_fits(FVM_TRB_KERNEL(trbdf2_affine_kernel, w), kRows, workgroups(n), &a));
+    FVM_HIP(fvm::grid_fits(FVM_TRB_KERNEL(gmres_kernel, w), kRows, workgroups(n), &b));
+    if (!a || !b) return FVM_OK;
+  }
+  *fits = 1;
   return FVM_OK;
 }
 

@@ -49,6 +49,10 @@ int hip_fail(hipError_t e, const char* what);
 hipError_t dev_malloc(void** p, size_t bytes);
 hipError_t dev_alloc(void** p, size_t bytes);
 hipError_t dev_free(void* p);
+// Whether wgs workgroups of the kernel fit on the current device at once, as the kernels whose
+// workgroups wait for each other need (fvm_grid.hpp; fewer CUs than the whole chip's may be
+// visible).  Decided before the launch, so that a caller can keep another path.
+hipError_t grid_fits(const void* kernel, int threads, int64_t wgs, bool* fits);
 // fvm_mesh_create with the triangles of each tri_group kept contiguous (NULL: one group)
 int mesh_create_grouped(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh** out);
 // One forward-Euler step of fvm_eqs! in place, fused into the RHS kernels:

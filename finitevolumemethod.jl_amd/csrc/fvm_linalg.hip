@@ -2006,8 +2006,9 @@ int fvm_template_solve(fvm_template* t, const fvm_solve_opts* o, double* d_x, fv
 namespace fvm {
 
 // The Tsit5 loop of fvm_ode_solve on the template's ELL copy of A in one launch
-// (fvm_tsit5.hip); FVM_ERR_STATE when the template has no ELL copy or n exceeds
-// kTsit5GridMax, so that the caller keeps the multi-kernel loop.
+// (fvm_tsit5.hip); FVM_ERR_STATE when the template has no ELL copy, n exceeds
+// kTsit5GridMax or the device does not hold the grid at once, so that the caller keeps
+// the multi-kernel loop.
 int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const Tsit5Loop& start, fvm_ode_stats* st,
                          hipStream_t s) {
   // (an assembled ODE template: its pattern is symmetric, as the grid form requires)
@@ -2015,6 +2016,11 @@ int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const Tsi
   // one workgroup while its registers hold the rows: 11 us a step at 2,500 rows, where
   // the grid takes 14
   const bool local = o->n <= tsit5_rows_local_max(t->ellW);
+  if (!local) {
+    bool fits;
+    FVM_HIP(tsit5_rows_fits(o->n, t->ellW, &fits));
+    if (!fits) return FVM_ERR_STATE;
+  }
   SmallTsit5 a;
   static_cast<Tsit5Loop&>(a) = start;
   a.W = t->ellW;

@@ -2,8 +2,10 @@
 #include <cstdio>
 #include <cstring>
 #include <exception>
+#include <map>
 #include <mutex>
 #include <unordered_map>
+#include <utility>
 #include <vector>
 
 #include "fvm_internal.hpp"
@@ -150,6 +152,40 @@ hipError_t dev_free(void* p) {
   });
   return hipSuccess;
 }
+
+namespace {
+thread_local int64_t g_resident_limit = 0;  // fvm_test_resident_limit
+std::mutex g_occupancy;
+std::map<std::pair<const void*, int>, int64_t>* const g_resident = new std::map<std::pair<const void*, int>, int64_t>;
+}  // namespace
+
+hipError_t grid_fits(const void* kernel, int threads, int64_t wgs, bool* fits) {
+  *fits = false;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  int64_t most = -1;
+  {
+    std::lock_guard<std::mutex> lock(g_occupancy);
+    const auto it = g_resident->find({kernel, dev});
+    if (it != g_resident->end()) most = it->second;
+  }
+  if (most < 0) {
+    int per = 0, cus = 0;
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return e;
+    most = (int64_t)per * cus;
+    std::lock_guard<std::mutex> lock(g_occupancy);
+    try {
+      (*g_resident)[{kernel, dev}] = most;
+    } catch (const std::exception&) {  // no host memory: asked again the next time
+    }
+  }
+  if (g_resident_limit > 0 && g_resident_limit < most) most = g_resident_limit;
+  *fits = wgs <= most;
+  return hipSuccess;
+}
 }  // namespace fvm
 
 extern "C" {
@@ -160,6 +196,10 @@ void fvm_test_fail_allocations(int64_t after, int64_t count) {
   fvm::g_fail_after = after;
   fvm::g_fail_count = count;
 }
+
+// And: the device holds at most wgs workgroups of the kernels that need to be resident, for the
+// calling thread (0: what it does hold).
+void fvm_test_resident_limit(int64_t wgs) { fvm::g_resident_limit = wgs; }
 
 int fvm_last_error(char* buf, size_t n) {
   if (!buf || n == 0) return FVM_ERR_ARG;

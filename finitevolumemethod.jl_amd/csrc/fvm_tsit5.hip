@@ -190,17 +190,16 @@ hipError_t run_local(SmallTsit5& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int W, int T>
-hipError_t run_grid(SmallTsit5& a, hipStream_t s) {
-  void* args[] = {&a};
-  return hipLaunchCooperativeKernel((const void*)tsit5_rows_kernel<W, T, 1, false>, dim3((unsigned)((a.n + T - 1) / T)),
-                                    dim3(T), args, 0, s);
+const void* grid_kernel(int W) {
+  if (W <= 6) return (const void*)tsit5_rows_kernel<6, kGridT, 1, false>;
+  if (W <= 8) return (const void*)tsit5_rows_kernel<8, kGridT, 1, false>;
+  return (const void*)tsit5_rows_kernel<10, kGridT, 1, false>;
 }
+int64_t grid_wgs(int64_t n) { return (n + kGridT - 1) / kGridT; }
 
 // rows per thread of the one-workgroup form, at most: what its registers hold
 template <int W>
-hipError_t run(SmallTsit5& a, bool local, hipStream_t s) {
-  if (!local) return run_grid<W, kGridT>(a, s);
+hipError_t run(SmallTsit5& a, hipStream_t s) {
   const int rows = (int)((a.n + kLocalT - 1) / kLocalT);
   if (rows <= 2) return run_local<W, 2>(a, s);
   return rows <= 4 ? run_local<W, 4>(a, s) : run_local<W, W <= 6 ? 5 : 4>(a, s);
@@ -232,10 +231,15 @@ int tsit5_run(Tsit5Loop& a, size_t words, uint64_t** grid, const fvm_ode_opts* o
   if (e == hipSuccess && o->n_save > 0)
     e = hipMemcpyAsync(dev + words, o->save_t, sizeof(double) * (size_t)o->n_save, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = launch();
+  const bool refused = e == hipErrorCooperativeLaunchTooLarge;
   double r[6] = {0, 0, 0, 0, 0, 0};
   if (e == hipSuccess) e = hipMemcpyAsync(r, a.stats, sizeof r, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   (void)dev_free(dev);
+  if (refused) {  // fewer resident workgroups than grid_fits was told: the multi-kernel loop
+    (void)hipGetLastError();
+    return FVM_ERR_STATE;
+  }
   if (e != hipSuccess) return hip_fail(e, "fvm_ode_solve (one-launch Tsit5)");
   if (r[5] < 0) {
     set_error("fvm_ode_solve: the grid's exchange timed out");
@@ -252,10 +256,18 @@ int tsit5_run(Tsit5Loop& a, size_t words, uint64_t** grid, const fvm_ode_opts* o
 
 size_t tsit5_rows_grid_words(int64_t n) { return grid_words(n); }
 
+hipError_t tsit5_rows_fits(int64_t n, int W, bool* fits) {
+  return grid_fits(grid_kernel(W), kGridT, grid_wgs(n), fits);
+}
+
 hipError_t tsit5_rows(SmallTsit5& a, bool local, hipStream_t s) {
-  if (a.W <= 6) return run<6>(a, local, s);
-  if (a.W <= 8) return run<8>(a, local, s);
-  return run<10>(a, local, s);
+  if (!local) {
+    void* args[] = {&a};
+    return hipLaunchCooperativeKernel(grid_kernel(a.W), dim3((unsigned)grid_wgs(a.n)), dim3(kGridT), args, 0, s);
+  }
+  if (a.W <= 6) return run<6>(a, s);
+  if (a.W <= 8) return run<8>(a, s);
+  return run<10>(a, s);
 }
 
 }  // namespace fvm

@@ -24,7 +24,8 @@ struct Tsit5Loop {
 };
 
 // The options' part of a, its device memory (words of exchange memory, zeroed, to *grid
-// before launch()), the launch and the results to st.
+// before launch()), the launch and the results to st; FVM_ERR_STATE, nothing done, when the
+// runtime refuses the grid.
 int tsit5_run(Tsit5Loop& a, size_t words, uint64_t** grid, const fvm_ode_opts* o, const std::function<hipError_t()>& launch,
               fvm_ode_stats* st, hipStream_t s);
 
@@ -48,6 +49,8 @@ constexpr int64_t kTsit5GridMax = 65536;  // rows of the grid form (256 workgrou
 int64_t tsit5_rows_local_max(int W);
 // 8-byte words of exchange memory of the grid form
 size_t tsit5_rows_grid_words(int64_t n);
+// whether the device holds the grid form's workgroups at once
+hipError_t tsit5_rows_fits(int64_t n, int W, bool* fits);
 hipError_t tsit5_rows(SmallTsit5& a, bool local, hipStream_t s);
 
 }  // namespace fvm

@@ -211,14 +211,14 @@ __global__ __launch_bounds__(kT) void tsit5_mesh_kernel(MeshTsit5 a) {
   tsit5_loop<1, true>(a, k, un, u_of, row, apply, norm_sum, dirichlet, up);
 }
 
-template <int FK>
-hipError_t run(MeshTsit5& a, hipStream_t s) {
-  if (a.m.n == 1) {
-    hipLaunchKernelGGL(tsit5_mesh_kernel<FK>, dim3(1), dim3(kT), 0, s, a);
-    return hipGetLastError();
+const void* kernel_of(int flux_kind) {
+  switch (flux_kind) {
+    case FVM_FLUX_D_POLY_U: return (const void*)tsit5_mesh_kernel<FVM_FLUX_D_POLY_U>;
+    case FVM_FLUX_D_NODAL: return (const void*)tsit5_mesh_kernel<FVM_FLUX_D_NODAL>;
+    case FVM_FLUX_LINEAR: return (const void*)tsit5_mesh_kernel<FVM_FLUX_LINEAR>;
+    case FVM_FLUX_D_POWER: return (const void*)tsit5_mesh_kernel<FVM_FLUX_D_POWER>;
+    default: return (const void*)tsit5_mesh_kernel<FVM_FLUX_D_EDGE>;
   }
-  void* args[] = {&a};
-  return hipLaunchCooperativeKernel((const void*)tsit5_mesh_kernel<FK>, dim3((unsigned)a.m.n), dim3(kT), args, 0, s);
 }
 
 }  // namespace
@@ -229,19 +229,19 @@ int problem_tsit5_small(const fvm_ctx* c, const fvm_ode_opts* o, const Tsit5Loop
                         hipStream_t s) {
   const MeshBlocks& m = c->m->blocks;
   if (m.n == 0 || o->n != c->m->N || c->flux_kind == FVM_FLUX_JIT) return FVM_ERR_STATE;
+  const void* const kernel = kernel_of(c->flux_kind);
+  bool fits;
+  FVM_HIP(grid_fits(kernel, kT, m.n, &fits));
+  if (!fits) return FVM_ERR_STATE;
   MeshTsit5 a;
   static_cast<Tsit5Loop&>(a) = start;
   a.p = make_args(c);
   a.m = m;
   const size_t words = grid_words(2 * (int64_t)m.n * NB);
   auto launch = [&] {
-    switch (c->flux_kind) {
-      case FVM_FLUX_D_POLY_U: return run<FVM_FLUX_D_POLY_U>(a, s);
-      case FVM_FLUX_D_NODAL: return run<FVM_FLUX_D_NODAL>(a, s);
-      case FVM_FLUX_LINEAR: return run<FVM_FLUX_LINEAR>(a, s);
-      case FVM_FLUX_D_POWER: return run<FVM_FLUX_D_POWER>(a, s);
-      default: return run<FVM_FLUX_D_EDGE>(a, s);
-    }
+    void* args[] = {&a};
+    if (m.n == 1) return hipLaunchKernel(kernel, dim3(1), dim3(kT), args, 0, s);
+    return hipLaunchCooperativeKernel(kernel, dim3((unsigned)m.n), dim3(kT), args, 0, s);
   };
   return tsit5_run(a, words, &a.grid, o, launch, st, s);
 }

@@ -239,6 +239,7 @@ HIP_API = {
     "fvm_gmres_work_bytes": [ctypes.c_int64],
     "fvm_gmres_ell": [_vp, ctypes.c_double, ctypes.c_double, ctypes.c_int32, _vp, _vp, ctypes.c_double,
                       ctypes.c_int32, ctypes.c_int64, _vp, _vp],
+    "fvm_ell_resident": [ctypes.c_int64, _i32p],
     "fvm_gmres_iterations": [_vp, _i64p, _vp],
     "fvm_jacobian_ell": [_vp, ctypes.c_int32, ctypes.POINTER(_vp), _vp, ctypes.c_int32, _vp, ctypes.c_double, _vp,
                          _vp, _vp, _vp],

@@ -8,9 +8,9 @@ J on its jacobian_sparsity pattern (solve.jl:50-77, 167-183).  Here J is extract
 once per problem from fvm_jvp probes over a distance-2 colouring of that pattern (one
 probe per colour, about a dozen on a triangle mesh; exact for an affine f), stored in
 ELL form, and fvm_trbdf2_affine integrates the whole problem in one launch of resident
-workgroups (no host round trip per Krylov iteration).  Problems above 65,536 unknowns, with a user
-callback, without save times or outside the affine forms keep the host-driven
-integrator (solve.py).
+workgroups (no host round trip per Krylov iteration).  Problems above 65,536 unknowns (or
+what the visible part of the chip holds at once), with a user callback, without save times
+or outside the affine forms keep the host-driven integrator (solve.py).
 """
 import ctypes
 
@@ -187,7 +187,7 @@ class FrozenJacobian:
         """A FrozenJacobian for prob, or None where the pattern is not one for it."""
         from .problem import FVMProblem
 
-        if not isinstance(prob, FVMProblem) or prob.mesh.triangulation.num_points() > MAX_N:
+        if not isinstance(prob, FVMProblem) or not resident(prob.mesh.triangulation.num_points()):
             return None
         plan = getattr(prob, "_jacobian_plan", None)
         if plan is None:
@@ -242,12 +242,20 @@ def affine_operator(prob):
     return op
 
 
+def resident(n):
+    """Whether the device holds the one-launch solvers' workgroups for n unknowns at once
+    (65,536 on a whole MI355X; fewer where fewer CUs are visible)."""
+    fits = ctypes.c_int32()
+    _lib.check(_lib.hip_lib().fvm_ell_resident(n, ctypes.byref(fits)), "fvm_ell_resident")
+    return bool(fits.value)
+
+
 def eligible(prob, alg, saveat, user_callback):
     from .problem import FVMProblem
 
     return (isinstance(prob, FVMProblem) and getattr(alg, "device_loop", True) and user_callback is None
             and saveat is not None and len(prob.initial_condition) <= MAX_N and 1 <= alg.krylov_restart <= 30
-            and is_affine(prob))
+            and resident(len(prob.initial_condition)) and is_affine(prob))
 
 
 def trbdf2_affine(prob, alg, saveat, abstol, reltol, dt, maxiters, save_start):

@@ -530,11 +530,15 @@ int fvm_trbdf2_affine(const fvm_affine_op* op, const fvm_trbdf2_opts* o, double*
  * launch; does not wait.  d_work: fvm_gmres_work_bytes(n) bytes, zeroed before its first
  * use, for one call at a time.  A call that fails on the device (its workgroups' exchange
  * timed out) and every later one on that d_work set x to NaN.
+ * fvm_ell_resident: whether the current device holds the workgroups of fvm_trbdf2_affine and
+ * fvm_gmres_ell for n unknowns at once (one per 256), as both need; they return FVM_ERR_STATE,
+ * nothing done, where it does not.
  * fvm_gmres_iterations: the iterations of all calls on d_work so far; waits, and fails
  * if one of them did. */
 size_t fvm_gmres_work_bytes(int64_t n);
 int fvm_gmres_ell(const fvm_affine_op* J, double a, double b, int32_t jacobi, const double* d_rhs, double* d_x,
                   double rtol, int32_t restart, int64_t maxiter, void* d_work, fvm_stream s);
+int fvm_ell_resident(int64_t n, int32_t* fits);
 int fvm_gmres_iterations(const void* d_work, int64_t* iterations, fvm_stream s);
 int fvm_jacobian_ell(fvm_ctx* ctx, int32_t n_colours, const double* const* d_probes, const uint8_t* d_colour,
                      int32_t width, const double* d_u, double t, double* d_products, double* d_val,

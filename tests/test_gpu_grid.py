@@ -7,6 +7,9 @@ stopped at 1e-7 and GMRES at 1e-9 of their scales: the two then take the same st
 differ by the Newton tolerance times the error norm's scale (abstol + reltol |u|, 1e-3
 |u| here) per solve, two solves a step: at most 2e-10 |u| per step, 1e-8 |u| over the
 fifty steps allowed here, and 1e-7 with the step controller's own amplification."""
+import contextlib
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -140,3 +143,57 @@ def test_one_launch_tsit5_is_the_host_loop_bit_for_bit(gpu, shape):
     assert a.retcode == b.retcode == "Success" and a.stats == b.stats and a.stats["naccept"] > 3, (a.stats, b.stats)
     for x, y in zip(a.u, b.u):
         assert np.array_equal(x[:-1], y)
+
+
+@contextlib.contextmanager
+def _resident(wgs):
+    from finitevolumemethod import _lib
+
+    f = _lib.hip_lib().fvm_test_resident_limit
+    f.argtypes, f.restype = [ctypes.c_int64], None
+    f(wgs)
+    try:
+        yield
+    finally:
+        f(0)
+
+
+def test_a_device_that_does_not_hold_the_grid_keeps_the_other_loops(gpu):
+    """Fewer resident workgroups than a launch needs (as where fewer CUs are visible; a limit
+    of the library's own here): Tsit5 runs the multi-kernel loop to the same bits, TR-BDF2 the
+    host integrator, and the C entry points return FVM_ERR_STATE with nothing done."""
+    from finitevolumemethod import _lib, implicit
+
+    prob, J = _frozen(61, 47)  # 12 workgroups
+    n = J.n
+    u = FVM.DeviceArray.from_host(prob.initial_condition)
+    J.take(u, 0.0)
+    b, x = FVM.DeviceArray.from_host(np.ones(n)), FVM.DeviceArray.from_host(np.full(n, 3.0))
+    tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 67, 61, single_boundary=True)
+    mesh = FVM.FVMGeometry(tri)
+    u0 = np.random.default_rng(2).random(tri.num_points())
+    ode = FVM.DiffusionEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.0 * x, FVM.Neumann),
+                                diffusion_function=lambda x, y, p: 0.5 + x, initial_condition=u0, final_time=0.005)
+    affine = _problem(FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 61, 47, single_boundary=False))
+    opts, ts = dict(newton_kappa=1e-7, krylov_rtol=1e-9), [0.005, 0.01]
+    cases = [lambda: FVM.solve(ode, FVM.Tsit5(), saveat=[0.0025, 0.005]), lambda: FVM.solve(prob, FVM.Tsit5(), saveat=ts),
+             lambda: FVM.solve(prob, FVM.TRBDF2(**opts), saveat=ts), lambda: FVM.solve(affine, FVM.TRBDF2(**opts), saveat=ts)]
+    whole = [c() for c in cases]
+    assert whole[3].stats.get("device_loop") and implicit.resident(n)
+    A, o, st = implicit.affine_operator(affine).op(), implicit.TrbOpts(), implicit.TrbStats()
+    o.tf, o.dt, o.abstol, o.reltol, o.maxiters = 0.05, 1e-3, 1e-6, 1e-3, 1000
+    o.newton_kappa, o.max_newton, o.krylov_restart, o.krylov_rtol = 1e-2, 10, 20, 1e-3
+    L = _lib.hip_lib()
+    with _resident(11):
+        assert not implicit.resident(n) and implicit.resident(11 * 256) and implicit.FrozenJacobian.of(prob) is None
+        with pytest.raises(_lib.FVMError, match="at once"):
+            J.solve(1.0, -1e-4, b, x, 1e-3, 20, 400, True)
+        assert L.fvm_trbdf2_affine(ctypes.byref(A), ctypes.byref(o), x.ptr, ctypes.byref(st), None) == -4
+        assert np.all(x.to_host() == 3.0)
+        part = [c() for c in cases]
+    assert "device_loop" not in part[3].stats
+    for k, (w, p) in enumerate(zip(whole, part)):
+        assert w.retcode == p.retcode == "Success" and w.stats["naccept"] == p.stats["naccept"]
+        assert k < 2 or w.stats["naccept"] <= 50
+        for a, b in zip(w.u, p.u):
+            assert np.array_equal(a, b) if k < 2 else np.max(np.abs(a - b)) <= 1e-7 * np.max(np.abs(b)), k
