@@ -176,7 +176,7 @@ def test_a_device_that_does_not_hold_the_grid_keeps_the_other_loops(gpu):
                                 diffusion_function=lambda x, y, p: 0.5 + x, initial_condition=u0, final_time=0.005)
     affine = _problem(FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 61, 47, single_boundary=False))
     opts, ts = dict(newton_kappa=1e-7, krylov_rtol=1e-9), [0.005, 0.01]
-    cases = [lambda: FVM.solve(ode, FVM.Tsit5(), saveat=[0.0025, 0.005]), lambda: FVM.solve(prob, FVM.Tsit5(), saveat=ts),
+    cases = [lambda: FVM.solve(ode, FVM.Tsit5(), saveat=[0.0025, 0.005]), lambda: FVM.solve(prob, FVM.Tsit5(), saveat=ts, dt=1e-6),
              lambda: FVM.solve(prob, FVM.TRBDF2(**opts), saveat=ts), lambda: FVM.solve(affine, FVM.TRBDF2(**opts), saveat=ts)]
     whole = [c() for c in cases]
     assert whole[3].stats.get("device_loop") and implicit.resident(n)
