@@ -399,8 +399,56 @@ __global__ __launch_bounds__(kB) void transpose_fill_kernel(int64_t n, const uin
   key[qtp[c] + atomicAdd(count + c, -1) - 1] = (uint32_t)i << 4 | (uint32_t)k;
 }
 
+// Lists of more than kListWave entries (the columns of a hub's aggregate) in ascending order: a
+// workgroup looks at 1024 lists and sorts those it finds one after the other, by Batcher's
+// bitonic network with every comparator ascending (the first step of a merge mirrored), so that
+// places beyond the end act as infinities; in LDS up to kListLds entries.  m log^2 m steps by
+// 1024 threads: a list in memory of 10^5 entries takes about 15,000 rounds, where one lane's
+// insertion sort of a list that arrives in descending order takes 5 10^9 dependent steps.
+constexpr int kListWave = 128, kListLds = 8192;
+__global__ __launch_bounds__(1024) void transpose_sort_long_kernel(int64_t nc, const int32_t* __restrict__ qtp,
+                                                                   uint32_t* __restrict__ key) {
+  __shared__ uint32_t sh[kListLds];
+  __shared__ int found[1024], n_found;
+  const int tid = threadIdx.x;
+  if (tid == 0) n_found = 0;
+  __syncthreads();
+  const int64_t c = gid();
+  if (c < nc && qtp[c + 1] - qtp[c] > kListWave) found[atomicAdd(&n_found, 1)] = (int)c;
+  __syncthreads();
+  for (int f = 0; f < n_found; ++f) {
+    const int k0 = qtp[found[f]], m = qtp[found[f] + 1] - k0;
+    const bool lds = m <= kListLds;
+    uint32_t* const a = lds ? sh : key + k0;
+    if (lds)
+      for (int i = tid; i < m; i += 1024) a[i] = key[k0 + i];
+    __syncthreads();
+    auto order = [&](int64_t i, int64_t j) {
+      if (j >= m) return;
+      const uint32_t x = a[i], y = a[j];
+      if (x > y) {
+        a[i] = y;
+        a[j] = x;
+      }
+    };
+    for (int64_t size = 2; size < 2 * (int64_t)m; size <<= 1) {
+      const int64_t half = size >> 1;
+      // pairs t of blocks of `size`; the last block's may lie beyond the end
+      for (int64_t t = tid; t / half * size < m; t += 1024) order(t / half * size + t % half, t / half * size + size - 1 - t % half);
+      __syncthreads();
+      for (int64_t step = half >> 1; step > 0; step >>= 1) {
+        for (int64_t t = tid; t / step * 2 * step < m; t += 1024) order(t / step * 2 * step + t % step, t / step * 2 * step + t % step + step);
+        __syncthreads();
+      }
+    }
+    if (lds)
+      for (int i = tid; i < m; i += 1024) key[k0 + i] = a[i];
+    __syncthreads();
+  }
+}
+
 // each list in ascending order, and its values: a wave per list, two entries per lane up
-// to 128 (a bitonic network over e = lane + 64 r), in memory by one lane beyond
+// to kListWave (a bitonic network over e = lane + 64 r); longer ones are in order already
 __global__ __launch_bounds__(kB) void transpose_sort_kernel(int64_t nc, const int32_t* __restrict__ qtp,
                                                             uint32_t* __restrict__ key, const float* __restrict__ qv,
                                                             int64_t qi, int64_t qk, int32_t* __restrict__ qti,
@@ -409,17 +457,7 @@ __global__ __launch_bounds__(kB) void transpose_sort_kernel(int64_t nc, const in
   const int lane = threadIdx.x & 63;
   if (c >= nc) return;
   const int k0 = qtp[c], m = qtp[c + 1] - k0;
-  if (m > 128) {
-    if (lane == 0)
-      for (int k = k0 + 1; k < k0 + m; ++k) {
-        const uint32_t x = key[k];
-        int j = k;
-        for (; j > k0 && key[j - 1] > x; --j) key[j] = key[j - 1];
-        key[j] = x;
-      }
-    __threadfence_block();
-    __builtin_amdgcn_wave_barrier();
-  } else {
+  if (m <= kListWave) {
     uint32_t x[2];
 #pragma unroll
     for (int r = 0; r < 2; ++r) x[r] = lane + 64 * r < m ? key[k0 + lane + 64 * r] : 0xffffffffu;
@@ -862,6 +900,8 @@ int amg_build(int64_t n0, const int32_t* rp, const int32_t* col, const double* v
                        L.qtp);
     FVM_HIP(hipMemcpyAsync(L.qtp + nc, sums + nbc, sizeof nq, hipMemcpyDeviceToDevice, st));
     hipLaunchKernelGGL(transpose_fill_kernel, grid1(n * kG), dim3(kB), 0, st, n, L.qcnt, tcol, L.qtp, count, key);
+    hipLaunchKernelGGL(transpose_sort_long_kernel, dim3((unsigned)((nc + 1023) / 1024)), dim3(1024), 0, st, (int64_t)nc,
+                       L.qtp, key);
     hipLaunchKernelGGL(transpose_sort_kernel, grid1((int64_t)nc * 64), dim3(kB), 0, st, (int64_t)nc, L.qtp, key, L.qv,
                        L.qi, L.qk, L.qti, L.qtv);
     hipLaunchKernelGGL(coarse_kernel, dim3((unsigned)(((int64_t)nc * kG + 63) / 64)), dim3(64), 0, st, (int64_t)nc,

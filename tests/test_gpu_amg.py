@@ -6,9 +6,11 @@ Both stop at |b - A x| <= 1e-10 |b|; the solutions then differ by at most
 the factorisation), and the same call twice gives the same bits."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 import scipy.sparse.linalg as spla
 
 import finitevolumemethod as FVM
+from finitevolumemethod import CG
 
 pytestmark = pytest.mark.gpu
 
@@ -69,14 +71,45 @@ def test_default_steady_solve_matches_a_direct_solution(gpu, kind, D):
     assert np.array_equal(FVM.solve(prob).u, a.u)
 
 
+@pytest.mark.parametrize("k", [127, 129, 4000, 8190, 8192, 20000])
+def test_a_row_with_many_entries(gpu, k):
+    """A node joined to k others across the mesh: its aggregate's column is in the transposed
+    lists of k rows and more, sorted by a wave up to 128 entries, by a workgroup in LDS up to
+    8,192 and in memory beyond."""
+    from finitevolumemethod.templates import DeviceTemplate
+
+    tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 150, 140, single_boundary=True)
+    mesh = FVM.FVMGeometry(tri)
+    n = tri.num_points()
+    edges = np.unique(np.sort(np.concatenate([tri.triangles[:, [0, 1]], tri.triangles[:, [1, 2]], tri.triangles[:, [2, 0]]]), axis=1), axis=0)
+    hub, others = 75 + 150 * 70, np.random.default_rng(k).permutation(n)[:k]
+    i = np.concatenate([edges[:, 0], np.full(k, hub)])
+    j = np.concatenate([edges[:, 1], others])
+    w = np.concatenate([np.ones(len(edges)), np.full(k, 0.1)]) * (i != j)
+    L = sp.coo_matrix((np.concatenate([w, w]), (np.concatenate([i, j]), np.concatenate([j, i]))), shape=(n, n)).tocsr()
+    L = sp.diags(np.asarray(L.sum(1)).ravel() + 1e-3) - L
+    A = (sp.diags(-1.0 / mesh.cv_volumes) @ L).tocsr()
+    A.sort_indices()
+    b = np.random.default_rng(1).standard_normal(n) / mesh.cv_volumes
+    make = lambda: DeviceTemplate.from_csr(mesh, A.indptr, A.indices, A.data, b, np.zeros(n, bool))  # noqa: E731
+    T = make()
+    x, st = T.solve(maxiter=200)
+    # sorted lists: the same hierarchy bit for bit, though they arrive in the order of atomics
+    assert np.array_equal(make().solve(maxiter=200)[0].to_host(), x.to_host())
+    assert st["converged"] and st["residual"] <= 1e-10, st
+    assert not T.solve(CG(), maxiter=2 * st["iterations"])[1]["converged"]
+    ref = spla.spsolve(A.tocsc(), b)
+    # |A^-1 r| <= |L^-1| |V r| <= 1e3 max(V) 1e-10 |b|
+    bound = 1e3 * mesh.cv_volumes.max() * 1e-10 * np.linalg.norm(b)
+    assert np.linalg.norm(x.to_host() - ref) <= bound + 1e-12 * np.linalg.norm(ref)
+
+
 def test_a_singular_system_ends_as_it_does_with_jacobi(gpu):
     """Zero flux everywhere and a source that does not sum to zero: no solution."""
     tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 30, 30, single_boundary=True)
     mesh = FVM.FVMGeometry(tri)
     prob = FVM.PoissonsEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.0 * x, FVM.Neumann),
                                 source_function=lambda x, y, p: 1.0 + 0.0 * x)
-    from finitevolumemethod import CG
-
     a, b = FVM.solve(prob, maxiter=500), FVM.solve(prob, CG(), maxiter=500)
     assert a.retcode == b.retcode == "MaxIters" and np.all(np.isfinite(a.u))
 
@@ -84,8 +117,6 @@ def test_a_singular_system_ends_as_it_does_with_jacobi(gpu):
 def test_a_source_of_one_mode_needs_no_cycle(gpu):
     """sin(pi x) sin(pi y) on a uniform grid is an eigenvector of the scaled operator: the
     Jacobi-preconditioned steps before the cycle meet the target, as CG() does."""
-    from finitevolumemethod import CG
-
     tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, 70, 70, single_boundary=True)
     mesh = FVM.FVMGeometry(tri)
     prob = FVM.PoissonsEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.0 * x, FVM.Dirichlet),
