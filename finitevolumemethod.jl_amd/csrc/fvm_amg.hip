@@ -776,7 +776,7 @@ Amg::~Amg() {
 
 int amg_build(int64_t n0, const int32_t* rp, const int32_t* col, const double* val, Amg** out, hipStream_t st) {
   *out = nullptr;
-  if (n0 >= (1 << 28)) return FVM_OK;  // the transposed lists' keys hold 28 bits of row
+  if (n0 > kAmgMaxRows) return FVM_OK;
   const auto t0 = std::chrono::steady_clock::now();
   struct Guard {
     Amg* a;

@@ -10,6 +10,9 @@ namespace fvm {
 // A sparse matrix by rows: CSR (rp given), or kAmgRow places per row, cnt of them used.
 constexpr int kAmgRow = 48;  // entries per row of a coarse operator, at most
 constexpr int kAmgQ = 16;    // entries per row of Q, at most (the transposed lists' keys hold 4 bits of it)
+// Rows of an operator, at most: the transposed lists' starts are int32, their keys row << 4 | slot.
+constexpr int64_t kAmgMaxRows = INT32_MAX / kAmgQ;
+static_assert(kAmgMaxRows * kAmgQ <= INT32_MAX && kAmgMaxRows < ((int64_t)1 << 28) && kAmgQ <= 16, "int32 lists");
 
 struct AmgMat {
   int64_t n = 0;
