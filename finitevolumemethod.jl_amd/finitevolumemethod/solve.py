@@ -513,6 +513,7 @@ def _integrate_trbdf2(rhs, jvp, u0, t0, tf, alg, *, saveat, abstol, reltol, dt, 
         if jacobian is not None:
             if frozen["t"] != tbase:
                 jacobian.take(ubase, tbase)
+                stats["njvp"] += jacobian.n_colours  # a product per colour; none in the Krylov steps
                 frozen["t"] = tbase
             jacobian.solve(1.0, -_TRB_D * h, b, x, alg.krylov_rtol, alg.krylov_restart, 20 * alg.krylov_restart,
                            alg.precond == "jacobi")
@@ -626,7 +627,6 @@ def _integrate_trbdf2(rhs, jvp, u0, t0, tf, alg, *, saveat, abstol, reltol, dt, 
         sol.retcode = "Success" if t >= tf else "MaxIters"
     if jacobian is not None:
         stats["nkrylov"] = jacobian.iterations()
-        stats["njvp"] = stats["nkrylov"]
     sol.stats = stats
     sol.final_device = u
     return sol

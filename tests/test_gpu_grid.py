@@ -52,7 +52,7 @@ def test_affine_trbdf2_matches_the_host_integrator(gpu, shape):
 
 
 @pytest.mark.parametrize("shape", [(5, 4), (16, 16), (61, 47), (131, 127), "wheel"], ids=str)
-def test_nonlinear_trbdf2_with_a_frozen_jacobian_matches_the_matrix_free_loop(gpu, shape):
+def test_nonlinear_trbdf2_with_a_frozen_jacobian_matches_the_matrix_free_loop(gpu, shape, monkeypatch):
     """The same loop with each linear system solved in one launch on the extracted J
     (fvm_jacobian_ell, fvm_gmres_ell) or matrix-free: a hub's wide rows keep the latter.
     Tolerances as above."""
@@ -67,7 +67,11 @@ def test_nonlinear_trbdf2_with_a_frozen_jacobian_matches_the_matrix_free_loop(gp
                           source_function=lambda x, y, t, u, p: u * (1 - u), initial_condition=u0, final_time=0.02)
     assert (implicit.FrozenJacobian.of(prob) is None) == wheel
     opts = dict(newton_kappa=1e-7, krylov_rtol=1e-9)
+    colours, take = [], implicit.FrozenJacobian.take
+    monkeypatch.setattr(implicit.FrozenJacobian, "take", lambda J, u, t: (colours.append(J.n_colours), take(J, u, t)))
     a = FVM.solve(prob, FVM.TRBDF2(**opts), saveat=[0.01, 0.02])
+    if not wheel:  # the products made: those that J is extracted from, once per step's start
+        assert a.stats["njvp"] == sum(colours) > 0 and len(colours) == a.stats["naccept"], (a.stats, colours)
     b = FVM.solve(prob, FVM.TRBDF2(device_loop=False, **opts), saveat=[0.01, 0.02])
     assert a.retcode == b.retcode == "Success"
     assert a.stats["naccept"] == b.stats["naccept"] <= 50 and a.stats["nnewton"] > 0, (a.stats, b.stats)
