@@ -60,6 +60,8 @@ int mesh_create_grouped(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_me
 // callback at t + dt.  Exclusive nodes are read and written by one tile only, and
 // shared nodes only by the fix-up after every tile has read them.
 int euler_step(fvm_ctx* c, double* d_u, const double* tile_dt, const double* dtv, double t, hipStream_t s);
+// fvm_eqs! by the tile kernels, on small meshes too (to time a tile size)
+int rhs_tiles(fvm_ctx* c, const double* d_u, double* d_du, double t, hipStream_t s);
 
 #define FVM_HIP(call)                                        \
   do {                                                       \

@@ -127,7 +127,7 @@ void launch_fix(const KArgs& a, hipStream_t s) {
 }
 
 template <int FK, int MODE>
-int launch_fk(const fvm_mesh* m, const KArgs& a, hipStream_t s) {
+int launch_fk(const fvm_mesh* m, const KArgs& a, hipStream_t s, bool by_nodes) {
   if constexpr (MODE != M_EULER) {
     // One launch by nodes up to the size where its threefold fluxes cost more than the
     // second launch.  Measured, us, node against tile kernels (RHS of a quadratic D(u)):
@@ -136,7 +136,7 @@ int launch_fk(const fvm_mesh* m, const KArgs& a, hipStream_t s) {
     // per triangle 7.5 / 8.9 at 28,900 and 9.9 / 8.9 at 40,000; with pow in every edge's
     // flux 8.4 / 11.1 at 14,400 and 11.9 / 11.2 at 28,900.
     constexpr int64_t kMost = FK == FVM_FLUX_D_POWER ? 20000 : (FK == FVM_FLUX_LINEAR ? 32000 : kNodeMeshMax);
-    if (m->node_ent && m->N <= kMost) {
+    if (by_nodes && m->node_ent && m->N <= kMost) {
       const NodeArgs nodes = {m->N, m->node_ent, m->node_next, m->node_bed};
       hipLaunchKernelGGL((node_kernel<FK, MODE>), dim3((unsigned)((m->N * kNodeLanes + 255) / 256)), dim3(256), 0, s, a,
                          nodes);
@@ -160,15 +160,16 @@ int launch_jit(const fvm_ctx* c, const KArgs& a, int mode, hipStream_t s) {
   return rc;
 }
 
+// by_nodes: a small mesh may take node_kernel
 template <int MODE>
-int launch(const fvm_ctx* c, const KArgs& a, hipStream_t s) {
+int launch(const fvm_ctx* c, const KArgs& a, hipStream_t s, bool by_nodes = true) {
   switch (c->flux_kind) {
     case FVM_FLUX_JIT: return launch_jit(c, a, MODE, s);
-    case FVM_FLUX_D_POLY_U: return launch_fk<FVM_FLUX_D_POLY_U, MODE>(c->m, a, s);
-    case FVM_FLUX_D_NODAL: return launch_fk<FVM_FLUX_D_NODAL, MODE>(c->m, a, s);
-    case FVM_FLUX_LINEAR: return launch_fk<FVM_FLUX_LINEAR, MODE>(c->m, a, s);
-    case FVM_FLUX_D_POWER: return launch_fk<FVM_FLUX_D_POWER, MODE>(c->m, a, s);
-    default: return launch_fk<FVM_FLUX_D_EDGE, MODE>(c->m, a, s);
+    case FVM_FLUX_D_POLY_U: return launch_fk<FVM_FLUX_D_POLY_U, MODE>(c->m, a, s, by_nodes);
+    case FVM_FLUX_D_NODAL: return launch_fk<FVM_FLUX_D_NODAL, MODE>(c->m, a, s, by_nodes);
+    case FVM_FLUX_LINEAR: return launch_fk<FVM_FLUX_LINEAR, MODE>(c->m, a, s, by_nodes);
+    case FVM_FLUX_D_POWER: return launch_fk<FVM_FLUX_D_POWER, MODE>(c->m, a, s, by_nodes);
+    default: return launch_fk<FVM_FLUX_D_EDGE, MODE>(c->m, a, s, by_nodes);
   }
 }
 
@@ -405,6 +406,14 @@ int euler_step(fvm_ctx* c, double* d_u, const double* tile_dt, const double* dtv
   a.tile_dt = tile_dt;
   a.dtv = dtv;
   return launch<M_EULER>(c, a, s);
+}
+
+int rhs_tiles(fvm_ctx* c, const double* d_u, double* d_du, double t, hipStream_t s) {
+  KArgs a = make_args(c);
+  a.u = d_u;
+  a.out = d_du;
+  a.t = t;
+  return launch<M_RHS>(c, a, s, false);
 }
 
 }  // namespace fvm

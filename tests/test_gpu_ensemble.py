@@ -3,6 +3,7 @@ and explicit Euler steps (graph-replayed or not) match stepping each member
 alone through the single-problem path."""
 import numpy as np
 import pytest
+import torch
 
 import finitevolumemethod as FVM
 from finitevolumemethod import ensemble as EN
@@ -110,6 +111,24 @@ def test_autotuner_reports_candidates(gpu):
     ms = list(info.candidate_ms)[:3]
     assert all(m > 0 for m in ms)
     assert info.tile_triangles == tiles[int(np.argmin(ms))]
+
+
+def test_autotuner_times_the_kernels_of_the_steps(gpu):
+    """The Euler steps run the tile kernels (two launches) at every size; a small ensemble's
+    right-hand side is one launch by nodes, which knows no tile size: 4 us against 7.5."""
+    b = EN.DeviceBatch(members(P=3, seed=2), autotune=True)
+    assert b.n <= 20000
+    u, du = FVM.DeviceArray.from_host(np.random.default_rng(0).random(b.n)), FVM.DeviceArray(b.n)
+    e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    best = np.inf
+    for _ in range(10):
+        e[0].record()
+        for _ in range(50):
+            b.rhs(u, du)
+        e[1].record()
+        e[1].synchronize()
+        best = min(best, e[0].elapsed_time(e[1]) / 50)
+    assert min(list(b.info.candidate_ms)[:3]) > 1.3 * best, (list(b.info.candidate_ms), best)
 
 
 def test_ensemble_solve_and_errors(gpu):
