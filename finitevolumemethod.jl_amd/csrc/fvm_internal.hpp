@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -121,6 +122,41 @@ __device__ __forceinline__ int32_t find_directed_edge(const int32_t* __restrict_
 }
 
 
+}  // namespace fvm
+
+// Nodes of the meshes that keep node_kernel's lists, at most (see launch_fk).
+constexpr int64_t kNodeMeshMax = 40000;
+
+// A mesh of up to 65,536 nodes cut into blocks of kBlockNodes nodes, one per workgroup
+// of the one-launch Tsit5 loop (fvm_tsit5_mesh.hip), with every triangle of a block's
+// nodes.  Lists in one device array, made by the first such solve (fvm_mesh_lists.hip).
+constexpr int kBlockNodes = 256;
+constexpr int kBlockTris = 512;    // triangles per list: inner ones, and those with nodes of other blocks
+constexpr int kBlockHalo = 512;    // nodes of other blocks, at most
+constexpr int kBlockItems = 256;   // boundary items, at most
+constexpr int kBlockFlux = 2 * kBlockTris + 1;  // row length of the block's fluxes
+struct MeshBlocks {
+  int32_t n = 0;                   // blocks, 0: no lists
+  const int32_t* node = nullptr;   // [n][256] node, -1: none (the last block's end)
+  const int32_t* bitem = nullptr;  // [n][256] its boundary items in the block: first << 8 | count
+  const int32_t* deg = nullptr;    // [n][256] its triangles
+  const int32_t* more = nullptr;   // [n][256] where those past the eighth stand in rest
+  const uint16_t* inc = nullptr;   // [n][256][8] slot kBlockFlux + local triangle, | 0x8000: first of another tile
+  const uint16_t* rest = nullptr;  // such entries
+  const int32_t* tri = nullptr;    // [n][1024] sorted triangle (-1: none), inner ones in the first half
+  const int32_t* loc = nullptr;    // [n][1024] its vertices' local ids a | b << 10 | c << 20 (256 +: halo)
+  const int32_t* halo = nullptr;   // [n][512] position 256 block + local id, -1: none
+  const int32_t* item = nullptr;   // [n][256] boundary edge << 1 | endpoint, -1: none
+  const int32_t* iloc = nullptr;   // [n][256] its triangle's vertices, as loc
+};
+
+namespace fvm {
+
+// Lists of a mesh (fvm_mesh_lists.hip): node_kernel's, queued on the null stream; the blocks of
+// the one-launch Tsit5, made by the first call for a mesh (waits for s), n = 0 for none.
+int make_node_lists(fvm_mesh* m);
+int mesh_blocks(const fvm_mesh* m, MeshBlocks* out, hipStream_t s);
+
 struct Tsit5Loop;
 // fvm_ode_solve's Tsit5 loop for a small ODE template or mesh in one launch
 // (fvm_linalg.hip, fvm_tsit5_mesh.hip), from start's time, step, state and k0 (its
@@ -136,32 +172,6 @@ int problem_tsit5_small(const fvm_ctx* c, const fvm_ode_opts* o, const Tsit5Loop
 int cgs2_norm(int64_t n, int k, const double* const* xs, double* w, double* h_host, hipStream_t s);
 
 }  // namespace fvm
-
-// Nodes of the meshes that keep node_kernel's lists, at most (see launch_fk).
-constexpr int64_t kNodeMeshMax = 40000;
-
-// A mesh of up to 65,536 nodes cut into blocks of kBlockNodes nodes, one per workgroup
-// of the one-launch Tsit5 loop (fvm_tsit5_mesh.hip), with every triangle of a block's
-// nodes.  Lists in one device array, made by mesh_blocks (fvm_mesh.hip).
-constexpr int kBlockNodes = 256;
-constexpr int kBlockTris = 512;    // triangles per list: inner ones, and those with nodes of other blocks
-constexpr int kBlockHalo = 512;    // nodes of other blocks, at most
-constexpr int kBlockItems = 256;   // boundary items, at most
-constexpr int kBlockFlux = 2 * kBlockTris + 1;  // row length of the block's fluxes
-struct MeshBlocks {
-  int32_t n = 0;                   // blocks, 0: no lists
-  const int32_t* node = nullptr;   // [n][256] node, -1: none (the last block's end)
-  const int32_t* bitem = nullptr;  // [n][256] its boundary items in the block: first << 8 | count
-  const int32_t* deg = nullptr;    // [n][256] its triangles
-  const int32_t* more = nullptr;   // [n][256] where those past the eighth stand in rest
-  const uint16_t* inc = nullptr;   // [n][256][8] slot kBlockFlux + local triangle, | 0x8000: first of another tile
-  const int32_t* rest = nullptr;   // such entries
-  const int32_t* tri = nullptr;    // [n][1024] sorted triangle (-1: none), inner ones in the first half
-  const int32_t* loc = nullptr;    // [n][1024] its vertices' local ids a | b << 10 | c << 20 (256 +: halo)
-  const int32_t* halo = nullptr;   // [n][512] position 256 block + local id, -1: none
-  const int32_t* item = nullptr;   // [n][256] boundary edge << 1 | endpoint, -1: none
-  const int32_t* iloc = nullptr;   // [n][256] its triangle's vertices, as loc
-};
 
 // Device-resident mesh: geometry SoA in tile (sorted) triangle order plus the
 // tile / fix-up structures from fvmh_tiles_build.
@@ -190,8 +200,12 @@ struct fvm_mesh {
                                     // first of another tile << 2 | slot (-1: padding)
   int32_t* node_next = nullptr;     // [blocks] the node's next block, -1: none (behind node_ent)
   int32_t* node_bed = nullptr;      // [N] boundary items: first << 8 | count (behind node_next)
-  int32_t* block_mem = nullptr;     // the lists of blocks
-  MeshBlocks blocks;
+  bool grouped = false;             // packed from several meshes (an ensemble)
+  // the lists of blocks (mesh_blocks), null and n = 0 when they are not made or do not fit
+  mutable std::mutex blocks_mutex;
+  mutable bool blocks_made = false;
+  mutable void* block_mem = nullptr;
+  mutable MeshBlocks blocks;
   int32_t* qflag = nullptr;         // device flag of the pointwise queries (run_flagged)
   bool convex = false;              // one boundary loop that turns left (or goes straight) at
                                     // every vertex: a point outside a boundary edge is outside

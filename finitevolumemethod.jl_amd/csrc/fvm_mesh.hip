@@ -6,11 +6,8 @@
 // FMA contraction off (the library is built with -ffp-contract=off): the
 // shape-function determinant cancels badly on small triangles far from the
 // origin, so any other evaluation order changes s1..s9 well above 1e-12.
-#include <algorithm>
-#include <array>
 #include <cstring>
 #include <exception>
-#include <future>
 #include <vector>
 
 #include "fvm_internal.hpp"
@@ -181,168 +178,6 @@ bool convex_domain(const fvm_mesh_desc* d) {
   return (3 * T + B) % 2 == 0 && nv - E + T == 1;
 }
 
-// The per-node incidences of node_kernel: blocks of eight in ascending triangle order, a
-// node's first block its own index, further ones after all nodes'.
-struct NodeLists {
-  std::vector<int4> ent;
-  std::vector<int32_t> next, bed;  // empty: no lists
-};
-NodeLists node_lists(const fvmh_tiles* tl) {
-  const int64_t N = tl->n_points, T = tl->n_tri;
-  constexpr int L = 8;
-  std::vector<int32_t> tile_of(T), next(N, -1), bed(N, 0);
-  for (int32_t k = 0; k < tl->n_tiles; ++k)
-    for (int32_t s = tl->tile_tri_start[k]; s < tl->tile_tri_start[k + 1]; ++s) tile_of[s] = k;
-  std::vector<int4> ent((size_t)N * L);
-  for (int64_t g = 0; g < N; ++g) {
-    for (int k = 0; k < L; ++k) ent[(size_t)g * L + k] = make_int4((int)g, (int)g, (int)g, -1);
-    int64_t blk = g;
-    const int32_t k0 = tl->node_tri_start[g], k1 = tl->node_tri_start[g + 1];
-    for (int32_t k = k0; k < k1; ++k) {
-      if (k > k0 && (k - k0) % L == 0) {
-        next[blk] = (int32_t)next.size();
-        blk = (int64_t)next.size();
-        next.push_back(-1);
-        ent.resize(ent.size() + L, make_int4((int)g, (int)g, (int)g, -1));
-      }
-      const int32_t s = tl->node_tri[k] >> 2;
-      const bool fresh = k > k0 && tile_of[s] != tile_of[tl->node_tri[k - 1] >> 2];
-      int4& e = ent[(size_t)blk * L + (k - k0) % L];
-      e.x = tl->tri_sorted[s];
-      e.y = tl->tri_sorted[T + s];
-      e.z = tl->tri_sorted[2 * T + s];
-      e.w = s << 3 | (int)fresh << 2 | (tl->node_tri[k] & 3);
-    }
-  }
-  for (int32_t f = 0; f < tl->n_fix; ++f) {
-    const int32_t b0 = tl->fix_bedge_start[f], nb = tl->fix_bedge_start[f + 1] - b0;
-    if (nb > 255 || b0 >= 1 << 23) return {};  // the tile kernels
-    bed[tl->fix_nodes[f]] = b0 << 8 | nb;
-  }
-  return {std::move(ent), std::move(next), std::move(bed)};
-}
-
-// The lists of MeshBlocks; none (n = 0) when a block would not fit its bounds.
-// Blocks are runs of the nodes in the order in which the triangles, sorted along a
-// space-filling curve, first reach them: compact patches, whatever the numbering.
-struct BlockLists {
-  int64_t n = 0;
-  std::vector<int32_t> all;   // inc, node, bitem, deg, more, tri, loc, halo, item, iloc, rest
-  std::array<int64_t, 11> at;  // where each begins
-};
-BlockLists mesh_blocks(const fvmh_tiles* tl) {
-  constexpr int NB = kBlockNodes, NT = 2 * kBlockTris, NH = kBlockHalo, NI = kBlockItems;
-  const int64_t N = tl->n_points, T = tl->n_tri;
-  const int32_t* tri = tl->tri_sorted;
-  std::vector<int32_t> pos(N, -1), order;
-  order.reserve(N);
-  for (int64_t s = 0; s < T; ++s)
-    for (int v = 0; v < 3; ++v) {
-      const int32_t g = tri[v * T + s];
-      if (pos[g] < 0) pos[g] = (int32_t)order.size(), order.push_back(g);
-    }
-  for (int64_t g = 0; g < N; ++g)
-    if (pos[g] < 0) pos[g] = (int32_t)order.size(), order.push_back((int32_t)g);
-  std::vector<int32_t> tile_of(T), fix_of(N, -1);
-  for (int32_t k = 0; k < tl->n_tiles; ++k)
-    for (int32_t s = tl->tile_tri_start[k]; s < tl->tile_tri_start[k + 1]; ++s) tile_of[s] = k;
-  for (int32_t f = 0; f < tl->n_fix; ++f) fix_of[tl->fix_nodes[f]] = f;
-
-  BlockLists out;
-  const int64_t n = (N + NB - 1) / NB;
-  const int64_t per[] = {NB * 4, NB, NB, NB, NB, NT, NT, NH, NI, NI};
-  auto& at = out.at;
-  at[0] = 0;
-  for (int k = 0; k < 10; ++k) at[k + 1] = at[k] + n * per[k];
-  std::vector<int32_t>& all = out.all;
-  all.assign(at[10], 0);
-  uint16_t* inc = (uint16_t*)all.data();
-  int32_t *node = &all[at[1]], *bitem = &all[at[2]], *deg = &all[at[3]], *more = &all[at[4]], *btri = &all[at[5]],
-          *loc = &all[at[6]], *halo = &all[at[7]], *item = &all[at[8]], *iloc = &all[at[9]];
-  for (int32_t* p : {node, btri, halo, item}) {
-    const int64_t* k = std::find(at.data(), at.data() + 10, p - all.data());
-    std::fill(p, p + (k[1] - k[0]), -1);
-  }
-  std::vector<int32_t> rest;
-  std::vector<int32_t> tri_at(T, -1), tri_in(T, -1), halo_at(N, -1), halo_in(N, -1);  // local id, of which block
-  for (int64_t b = 0; b < n; ++b) {
-    const int64_t p0 = b * NB, p1 = std::min(N, p0 + NB);
-    int n_in = 0, n_out = 0, n_halo = 0, n_item = 0;
-    auto local = [&](int32_t g) {
-      return pos[g] >= p0 && pos[g] < p1 ? pos[g] - (int32_t)p0 : (halo_in[g] == b ? NB + halo_at[g] : -1);
-    };
-    auto vertices = [&](int32_t s) {
-      return local(tri[s]) | local(tri[T + s]) << 10 | local(tri[2 * T + s]) << 20;
-    };
-    for (int64_t p = p0; p < p1; ++p) {
-      const int32_t g = order[p];
-      node[p] = g;
-      const int32_t k0 = tl->node_tri_start[g], k1 = tl->node_tri_start[g + 1];
-      deg[p] = k1 - k0;
-      more[p] = (int32_t)rest.size();
-      for (int32_t k = k0; k < k1; ++k) {
-        const int32_t s = tl->node_tri[k] >> 2;
-        if (tri_in[s] != b) {
-          bool inner = true;
-          for (int v = 0; v < 3; ++v) {
-            const int32_t h = tri[v * T + s];
-            if (local(h) >= 0 && local(h) < NB) continue;
-            inner = false;
-            if (local(h) >= 0) continue;
-            if (n_halo == NH) return {};
-            halo_in[h] = (int32_t)b;
-            halo_at[h] = n_halo;
-            halo[b * NH + n_halo++] = pos[h];
-          }
-          if (inner && n_in == kBlockTris) inner = false;
-          if (!inner && n_out == kBlockTris) return {};
-          tri_in[s] = (int32_t)b;
-          tri_at[s] = inner ? n_in++ : kBlockTris + n_out++;
-          btri[b * NT + tri_at[s]] = s;
-          loc[b * NT + tri_at[s]] = vertices(s);
-        }
-        const bool fresh = k > k0 && tile_of[s] != tile_of[tl->node_tri[k - 1] >> 2];
-        const int e = (tl->node_tri[k] & 3) * kBlockFlux + tri_at[s] + (fresh ? 0x8000 : 0);
-        if (k - k0 < 8) inc[(size_t)p * 8 + (k - k0)] = (uint16_t)e;
-        else rest.push_back(e);
-      }
-      if (fix_of[g] < 0) continue;
-      const int32_t b0 = tl->fix_bedge_start[fix_of[g]], b1 = tl->fix_bedge_start[fix_of[g] + 1];
-      if (n_item + (b1 - b0) > NI || b1 - b0 > 255) return {};
-      bitem[p] = n_item << 8 | (b1 - b0);
-      for (int32_t q = b0; q < b1; ++q, ++n_item) {
-        item[b * NI + n_item] = tl->fix_bedge[q];
-        iloc[b * NI + n_item] = vertices(tl->badj_sorted[tl->fix_bedge[q] >> 1]);
-        if (iloc[b * NI + n_item] < 0) return {};  // a boundary edge beside a triangle without its node
-      }
-    }
-  }
-  all.insert(all.end(), rest.begin(), rest.end());
-  out.n = n;
-  return out;
-}
-
-int upload_blocks(const BlockLists& b, fvm_mesh* m) {
-  if (b.n == 0) return FVM_OK;
-  const int rc = upload(&m->block_mem, b.all.data(), (int64_t)b.all.size());
-  if (rc != FVM_OK) return rc;
-  MeshBlocks& B = m->blocks;
-  const auto& at = b.at;
-  B.n = (int32_t)b.n;
-  B.inc = (const uint16_t*)m->block_mem;
-  B.node = m->block_mem + at[1];
-  B.bitem = m->block_mem + at[2];
-  B.deg = m->block_mem + at[3];
-  B.more = m->block_mem + at[4];
-  B.tri = m->block_mem + at[5];
-  B.loc = m->block_mem + at[6];
-  B.halo = m->block_mem + at[7];
-  B.item = m->block_mem + at[8];
-  B.iloc = m->block_mem + at[9];
-  B.rest = m->block_mem + at[10];
-  return FVM_OK;
-}
-
 int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
   // Tiles of up to 512 triangles run on 256-thread workgroups with room for 512
   // local nodes; tiles of up to 1024 triangles on 512-thread workgroups with 1024.
@@ -378,11 +213,7 @@ int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
             "fvm_mesh_create: mesh too large (the node and tile-node arrays must stay below 4 GiB: "
             "at most 536,870,911 points and tile-node slots)");
   int rc;
-  // made beside the uploads and the geometry kernels
-  std::future<NodeLists> nodes;
-  std::future<BlockLists> blocks;
-  if (N <= kNodeMeshMax) nodes = std::async(node_lists, (const fvmh_tiles*)tl);
-  if (N <= 65536 && !tri_group) blocks = std::async(mesh_blocks, (const fvmh_tiles*)tl);
+  m->grouped = tri_group != nullptr;
 #define UP(dst, src, n) \
   if ((rc = upload(&(dst), src, n)) != FVM_OK) return rc
   UP(m->x, d->x, N);
@@ -439,23 +270,12 @@ int build(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_mesh* m) {
   if (m->n_local > 0)
     hipLaunchKernelGGL(local_cv_kernel, dim3((unsigned)((m->n_local + 255) / 256)), dim3(256), 0, 0,
                        m->n_local, m->tile_nodes, m->cv, m->lcv);
+  rc = N <= kNodeMeshMax ? make_node_lists(m) : FVM_OK;
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipDeviceSynchronize();
   (void)hipFree(sub);
+  if (rc != FVM_OK) return rc;
   if (e != hipSuccess) return hip_fail(e, "fvm_mesh_create: geometry kernels");
-  if (nodes.valid()) {
-    const NodeLists L = nodes.get();
-    if (!L.bed.empty()) {  // in one array
-      std::vector<int32_t> all(4 * L.ent.size());
-      memcpy(all.data(), L.ent.data(), sizeof(int4) * L.ent.size());
-      all.insert(all.end(), L.next.begin(), L.next.end());
-      all.insert(all.end(), L.bed.begin(), L.bed.end());
-      if ((rc = upload((int32_t**)&m->node_ent, all.data(), (int64_t)all.size())) != FVM_OK) return rc;
-      m->node_next = (int32_t*)(m->node_ent + L.ent.size());
-      m->node_bed = m->node_next + L.next.size();
-    }
-  }
-  if (blocks.valid() && (rc = upload_blocks(blocks.get(), m)) != FVM_OK) return rc;
   return FVM_OK;
 }
 
@@ -475,7 +295,7 @@ int mesh_create_grouped(const fvm_mesh_desc* d, const int32_t* tri_group, fvm_me
   int rc;
   try {
     rc = build(d, tri_group, m);
-  } catch (const std::exception& e) {  // of the lists: no host memory
+  } catch (const std::exception& e) {  // no host memory
     set_error(std::string("fvm_mesh_create: ") + e.what());
     rc = FVM_ERR_ALLOC;
   }

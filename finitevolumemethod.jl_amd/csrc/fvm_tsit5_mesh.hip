@@ -17,6 +17,8 @@
 // Every element's arithmetic is the multi-kernel path's (tri_fluxes, boundary_flux,
 // NodeSum, finish_pre; the error norm in the order of the nodes' numbers, handed over
 // once a step): the same states bit for bit.
+#include <exception>
+
 #include "fvm_internal.hpp"
 #include "fvm_rhs_kernels.hpp"
 #include "fvm_tsit5_loop.hpp"
@@ -227,12 +229,21 @@ namespace fvm {
 
 int problem_tsit5_small(const fvm_ctx* c, const fvm_ode_opts* o, const Tsit5Loop& start, fvm_ode_stats* st,
                         hipStream_t s) {
-  const MeshBlocks& m = c->m->blocks;
-  if (m.n == 0 || o->n != c->m->N || c->flux_kind == FVM_FLUX_JIT) return FVM_ERR_STATE;
+  const int64_t wgs = (c->m->N + NB - 1) / NB;
+  if (wgs > kGridMaxWgs || o->n != c->m->N || c->flux_kind == FVM_FLUX_JIT) return FVM_ERR_STATE;
   const void* const kernel = kernel_of(c->flux_kind);
   bool fits;
-  FVM_HIP(grid_fits(kernel, kT, m.n, &fits));
+  FVM_HIP(grid_fits(kernel, kT, wgs, &fits));
   if (!fits) return FVM_ERR_STATE;
+  MeshBlocks m;
+  int rc;
+  try {
+    rc = mesh_blocks(c->m, &m, s);
+  } catch (const std::exception&) {  // no host memory
+    rc = FVM_ERR_ALLOC;
+  }
+  if (rc == FVM_ERR_ALLOC || (rc == FVM_OK && m.n == 0)) return FVM_ERR_STATE;  // no (room for) lists
+  if (rc != FVM_OK) return rc;
   MeshTsit5 a;
   static_cast<Tsit5Loop&>(a) = start;
   a.p = make_args(c);

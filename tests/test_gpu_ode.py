@@ -138,6 +138,25 @@ def test_tsit5_on_resident_blocks_matches_host_loop(gpu, build):
     assert_same(a, b)
 
 
+@pytest.mark.parametrize("build,blocks", [
+    (lambda: nonlinear_problem(4, 3)[0], 1), (lambda: nonlinear_problem(16, 16)[0], 1),
+    (lambda: nonlinear_problem(255, 257)[0], 256), (lambda: nonlinear_problem(257, 256)[0], 0),
+    (lambda: fan_problem(40, True), 1), (lambda: fan_problem(600, True), 0), (lambda: fan_problem(5000, True), 0),
+    (shuffled_problem, 4)], ids=["tiny", "one_block", "most_blocks", "over_them", "hub", "wide_hub", "wider_hub", "shuffled"])
+def test_blocks_are_made_by_the_first_solve_that_uses_them(gpu, build, blocks):
+    """Not with the mesh or a right-hand side; none where a block does not fit (what the lists
+    hold is held by the solves above, bit for bit)."""
+    L = _lib.hip_lib()
+    L.fvm_test_mesh_blocks.argtypes, L.fvm_test_mesh_blocks.restype = [ctypes.c_void_p], ctypes.c_int64
+    prob = build()
+    made = lambda: L.fvm_test_mesh_blocks(prob.mesh.handle)  # noqa: E731
+    u = np.asarray(prob.initial_condition)
+    FVM.fvm_eqs(np.zeros_like(u), u, prob, 0.0)
+    assert made() == -1
+    FVM.solve(prob, FVM.Tsit5(), saveat=[prob.initial_time], maxiters=1)
+    assert made() == (blocks if blocks else -1 if len(u) > 65536 else 0)
+
+
 def test_system_matches_host_loop(gpu):
     tri = FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, 20, 18, jitter=0.2, seed=2, single_boundary=False)
     sys = brusselator_system(tri, final_time=0.5)
