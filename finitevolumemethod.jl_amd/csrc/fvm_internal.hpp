@@ -195,7 +195,7 @@ struct fvm_mesh {
   uint8_t* is_vertex = nullptr;
   double* lcv = nullptr;            // [n_local] control volume of each local-node entry
   // per-node incidences of the one-launch RHS of small meshes (node_kernel), null on
-  // meshes above kNodeMeshMax
+  // meshes above kNodeMeshMax and with hubs
   int4* node_ent = nullptr;         // [blocks][8]: the triangle's vertices, sorted triangle << 3 |
                                     // first of another tile << 2 | slot (-1: padding)
   int32_t* node_next = nullptr;     // [blocks] the node's next block, -1: none (behind node_ent)

@@ -289,6 +289,13 @@ struct Pieces {
   }
 };
 
+int64_t max_degree(const fvm_mesh* m) {
+  int64_t most = 0;
+  for (int64_t g = 0; g < m->N; ++g) most = std::max<int64_t>(most, m->h_node_tri_start[g + 1] - m->h_node_tri_start[g]);
+  return most;
+}
+constexpr int64_t kNodeDegree = 40;
+
 // extra[g]: units(degree) summed over the nodes before g; empty when no node has any
 template <class F>
 std::vector<int32_t> running(const fvm_mesh* m, F units, int64_t* total) {
@@ -312,6 +319,11 @@ namespace fvm {
 
 // Queues the kernels on the null stream, as the mesh's geometry kernels.
 int make_node_lists(fvm_mesh* m) {
+  // one group of lanes adds a node's incidences, eight a round of about 1 us: with a hub the
+  // tile kernels, which share its triangles among their workgroups, are faster (RHS, us, node
+  // against tile kernels: 6.1 / 7.5 at a degree of 28, 7.0 / 6.9 at 40, 15 / 10 at 100, 126 / 16 at
+  // 1,000, 525 / 25 at 4,000)
+  if (max_degree(m) > kNodeDegree) return FVM_OK;
   for (int32_t f = 0; f < m->n_fix; ++f) {
     const int32_t b0 = m->h_fix_bedge_start[f];
     if (m->h_fix_bedge_start[f + 1] - b0 > 255 || b0 >= 1 << 23) return FVM_OK;  // the tile kernels
@@ -349,8 +361,8 @@ int mesh_blocks(const fvm_mesh* m, MeshBlocks* out, hipStream_t s) {
   if (!m->blocks_made) {
     const int64_t N = m->N, T = m->T, n = (N + kBlockNodes - 1) / kBlockNodes;
     // each triangle is in a block's list, each incidence in a node's
-    int64_t n_rest, most = 0;
-    for (int64_t g = 0; g < N; ++g) most = std::max<int64_t>(most, m->h_node_tri_start[g + 1] - m->h_node_tri_start[g]);
+    int64_t n_rest;
+    const int64_t most = max_degree(m);
     if (N > 65536 || m->grouped || T > n * 2 * kBlockTris || most > 3 * 2 * kBlockTris) {
       m->blocks_made = true;
       *out = m->blocks;

@@ -6,10 +6,14 @@ ulp, control volumes within 1e-14 (different summation order); du within
 1e-12 of the oracle in the max norm and per node relative to
 sum_sigma |Q_sigma| / V_i + |S_i| (the reference's own threaded and serial forms
 differ by rounding of the same size)."""
+import ctypes
+import time
+
 import numpy as np
 import pytest
 
 import finitevolumemethod as FVM
+from finitevolumemethod import _lib
 from oracle import geometry as oracle_geometry
 from problems import (annulus_problem, diffusion_problem, dxy_problem, heat_convection_problem,
                       mixed_problem, nodal_problem, nonlinear_problem, oracle_for)
@@ -256,11 +260,12 @@ def _fan(d, closed):
     return FVM.Triangulation(x, y, tris, edges, seg)
 
 
-@pytest.mark.parametrize("closed,d", [(True, 3), (True, 8), (True, 9), (True, 17), (True, 64), (False, 1),
-                                      (False, 2), (False, 8), (False, 9), (False, 25)])
+@pytest.mark.parametrize("closed,d", [(True, 3), (True, 8), (True, 9), (True, 17), (True, 40), (True, 41), (True, 64),
+                                      (False, 1), (False, 2), (False, 8), (False, 9), (False, 25)])
 def test_nodes_of_any_degree(gpu, closed, d):
-    """The hub's sum runs over one, a full and several blocks of eight incidences, with and
-    without boundary edges; the tangent too (bars of the RHS and JVP tests)."""
+    """The hub's sum runs over one, a full and several blocks of eight incidences (up to 40, by
+    tiles beyond), with and without boundary edges; the tangent too (bars of the RHS and JVP
+    tests)."""
     tri = _fan(d, closed)
     mesh = FVM.FVMGeometry(tri)
     BCs = FVM.BoundaryConditions(mesh, (lambda x, y, t, u, p: 0.3 + 0.0 * u, lambda x, y, t, u, p: 0.5 * u),
@@ -278,3 +283,26 @@ def test_nodes_of_any_degree(gpu, closed, d):
     prob.device_context().jvp(FVM.DeviceArray.from_host(u), FVM.DeviceArray.from_host(v), jv, 0.0)
     ref = orc.rhs_cs(u + 1e-30j * v, None, 0.0).imag / 1e-30
     assert np.max(np.abs(jv.to_host() - ref)) <= 1e-11 * np.max(np.abs(ref))
+
+
+def test_a_hub_does_not_hold_up_the_right_hand_side(gpu):
+    """A node of 1,000 triangles: the tile kernels (16 us and less), not the one launch by nodes,
+    where one group of lanes adds them (126 us)."""
+    tri = _fan(1000, True)
+    mesh = FVM.FVMGeometry(tri)
+    zero = lambda x, y, t, u, p: 0.0 * u  # noqa: E731
+    prob = FVM.FVMProblem(mesh, FVM.BoundaryConditions(mesh, (zero, zero), (FVM.Neumann, FVM.Dirichlet)),
+                          diffusion_function=lambda x, y, t, u, p: 0.1 + u ** 2, initial_condition=tri.x, final_time=1.0)
+    ctx, u, du = prob.device_context(), FVM.DeviceArray.from_host(tri.x), FVM.DeviceArray(len(tri.x))
+    ms = [[ctypes.c_float(), ctypes.c_float()] for _ in range(20)]
+    for a, b in ms:
+        _lib.check(_lib.hip_lib().fvm_rhs_timed(ctx.handle, u.ptr, du.ptr, 0.0, None, ctypes.byref(a), ctypes.byref(b)))
+    best = np.inf
+    for _ in range(20):
+        _lib.synchronize()
+        t = time.perf_counter()
+        for _ in range(50):
+            ctx.rhs(u, du, 0.0)
+        _lib.synchronize()
+        best = min(best, (time.perf_counter() - t) / 50)
+    assert best <= 2e-3 * min(a.value + b.value for a, b in ms), (best, ms)
