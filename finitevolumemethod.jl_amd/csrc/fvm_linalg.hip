@@ -56,6 +56,7 @@ constexpr int kRowsPerBlock = kRT / kLPR;
 constexpr int kRPG = FVM_SPMV_ROWS;      // rows per lane group per step of the SpMV loops
 constexpr int kEllMin = 4, kEllMax = 10; // unrolled slots of the sliced ELL form: the longest row's, in 4..10
 constexpr int kSlice = 64;               // rows per slice of the sliced ELL form: one wave
+static_assert(kEllMax == kTsit5MaxW, "build_ell leaves rows longer than ellW only where ellW is kEllMax");
 // Unknowns up to which FVM_SOLVE_AUTO first runs Jacobi-preconditioned CG in one
 // workgroup (cg_small), and the iterations it gives that.  Measured, ms, against the
 // cycle: 0.31 / 0.75 at 930 unknowns, 0.44 / 0.95 at 1,640, 0.65 / 1.06 at 2,813 (254
@@ -2018,12 +2019,13 @@ int template_tsit5_small(const fvm_template* t, const fvm_ode_opts* o, const Tsi
   const bool local = o->n <= tsit5_rows_local_max(t->ellW);
   if (!local) {
     bool fits;
-    FVM_HIP(tsit5_rows_fits(o->n, t->ellW, &fits));
+    FVM_HIP(tsit5_rows_fits(o->n, t->ellW, t->ell_overflow > 0, &fits));
     if (!fits) return FVM_ERR_STATE;
   }
   SmallTsit5 a;
   static_cast<Tsit5Loop&>(a) = start;
   a.W = t->ellW;
+  a.long_rows = t->ell_overflow > 0;
   a.off = t->sl_off;
   a.perm = t->sl_perm;
   a.rem_ptr = t->sl_rem_ptr;

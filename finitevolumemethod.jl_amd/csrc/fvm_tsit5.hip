@@ -48,7 +48,9 @@ struct Lds {
   GridShared<T> grid;
 };
 
-template <int W, int T, int RPT, bool kLocal>
+// kLong: there are rows longer than the operator's W slots (hubs); a form of its own, for its
+// registers (the others need 6 to 40 fewer without it, and spill none).
+template <int W, int T, int RPT, bool kLocal, bool kLong>
 __global__ __launch_bounds__(T) void tsit5_rows_kernel(SmallTsit5 a) {
   static_assert(W % 2 == 0 && (kLocal || RPT == 1) && T * RPT <= 8192, "layout");
   __shared__ Lds<T, RPT, kLocal> S;
@@ -68,7 +70,7 @@ __global__ __launch_bounds__(T) void tsit5_rows_kernel(SmallTsit5 a) {
   Rows<W, RPT, kLocal> R;
   double u0 = 0.0, b0 = 0.0;   // one row per thread: the state and b in registers
   double k[7][RPT], un[RPT];
-  uint32_t longer = 0;         // slices with rows longer than the operator's W slots, bit r
+  uint32_t longer = 0;         // kLong: slices with such rows, bit r
 #pragma unroll
   for (int r = 0; r < RPT; ++r) {
     const int64_t i = i0 + (int64_t)r * T, b = i / kSlice;
@@ -89,7 +91,7 @@ __global__ __launch_bounds__(T) void tsit5_rows_kernel(SmallTsit5 a) {
     k[0][r] = in ? a.k0[i] : 0.0;
     (kLocal ? S.u[tid + r * T] : u0) = in ? a.u[i] : 0.0;
     (kLocal ? S.b[tid + r * T] : b0) = in ? a.b[i] : 0.0;
-    if (__any(in && a.rem_ptr[b + 1] > a.rem_ptr[b])) longer |= 1u << r;
+    if (kLong && __any(in && a.rem_ptr[b + 1] > a.rem_ptr[b])) longer |= 1u << r;
   }
   auto u_of = [&](int r) -> double& { return kLocal ? S.u[tid + r * T] : u0; };
 
@@ -121,18 +123,47 @@ __global__ __launch_bounds__(T) void tsit5_rows_kernel(SmallTsit5 a) {
       double acc = 0.0;
 #pragma unroll
       for (int s = 0; s < W; ++s) acc += R.v[r][s] * xc[s];
-      if (longer & (1u << r)) {
+      if (kLong && longer & (1u << r)) {
         const int64_t i = i0 + (int64_t)r * T, b = i / kSlice;
         const int pos = slot_of(i);
         if (i < n) {
+          // eight entries' loads in flight (absent ones load entry 0), added in their order:
+          // 20 steps with a hub of 300 on 661 rows 7.6 -> 2.5 ms (one by one against eight), on
+          // 3,661 rows (the grid) 13.0 -> 4.8 ms; the multi-kernel loop takes 7.5
+          constexpr int K = 8;
           int st = a.off[(a.W + 1) * b + a.W];
-          for (int q = a.rem_ptr[b]; q < a.rem_ptr[b + 1]; ++q) {
-            const int e = st + pos;
-            if (e < a.rem_off[q]) {
-              const int c = a.eoff ? (int)i + (int)a.eoff[e] : a.ecol[e];
-              acc += a.eval[e] * (kLocal ? X[c] : G.fetch1(c));
+          const int q1 = a.rem_ptr[b + 1];
+          for (int q = a.rem_ptr[b]; q < q1; q += K) {
+            int e[K], c[K];
+            double v[K], xc[K];
+            uint32_t on = 0, o[K];
+#pragma unroll
+            for (int s = 0; s < K; ++s) {
+              const int end = a.rem_off[q + s < q1 ? q + s : q1 - 1];
+              const bool here = q + s < q1 && st + pos < end;
+              on |= (uint32_t)here << s;
+              e[s] = here ? st + pos : 0;
+              st = end;
             }
-            st = a.rem_off[q];
+            if (a.eoff) {
+#pragma unroll
+              for (int s = 0; s < K; ++s) c[s] = (int)i + (int)a.eoff[e[s]];
+            } else {
+#pragma unroll
+              for (int s = 0; s < K; ++s) c[s] = a.ecol[e[s]];
+            }
+#pragma unroll
+            for (int s = 0; s < K; ++s) v[s] = a.eval[e[s]];
+#pragma unroll
+            for (int s = 0; s < K; ++s) {
+              if (!(on >> s & 1)) c[s] = (int)i;
+              if (kLocal) xc[s] = X[c[s]];
+              else o[s] = grid_offset(c[s]);
+            }
+            if constexpr (!kLocal) G.fetch(o, xc, true);
+#pragma unroll
+            for (int s = 0; s < K; ++s)
+              if (on >> s & 1) acc += v[s] * xc[s];
           }
         }
       }
@@ -184,25 +215,27 @@ __global__ __launch_bounds__(T) void tsit5_rows_kernel(SmallTsit5 a) {
 
 constexpr int kLocalT = 512, kGridT = 256;
 
-template <int W, int RPT>
+template <int W, int RPT, bool kLong>
 hipError_t run_local(SmallTsit5& a, hipStream_t s) {
-  hipLaunchKernelGGL((tsit5_rows_kernel<W, kLocalT, RPT, true>), dim3(1), dim3(kLocalT), 0, s, a);
+  hipLaunchKernelGGL((tsit5_rows_kernel<W, kLocalT, RPT, true, kLong>), dim3(1), dim3(kLocalT), 0, s, a);
   return hipGetLastError();
 }
 
-const void* grid_kernel(int W) {
-  if (W <= 6) return (const void*)tsit5_rows_kernel<6, kGridT, 1, false>;
-  if (W <= 8) return (const void*)tsit5_rows_kernel<8, kGridT, 1, false>;
-  return (const void*)tsit5_rows_kernel<10, kGridT, 1, false>;
+// (rows are longer than W slots only where W is the operators' most, kTsit5MaxW)
+const void* grid_kernel(int W, bool long_rows) {
+  if (W <= 6) return (const void*)tsit5_rows_kernel<6, kGridT, 1, false, false>;
+  if (W <= 8) return (const void*)tsit5_rows_kernel<8, kGridT, 1, false, false>;
+  if (!long_rows) return (const void*)tsit5_rows_kernel<kTsit5MaxW, kGridT, 1, false, false>;
+  return (const void*)tsit5_rows_kernel<kTsit5MaxW, kGridT, 1, false, true>;
 }
 int64_t grid_wgs(int64_t n) { return (n + kGridT - 1) / kGridT; }
 
 // rows per thread of the one-workgroup form, at most: what its registers hold
-template <int W>
+template <int W, bool kLong>
 hipError_t run(SmallTsit5& a, hipStream_t s) {
   const int rows = (int)((a.n + kLocalT - 1) / kLocalT);
-  if (rows <= 2) return run_local<W, 2>(a, s);
-  return rows <= 4 ? run_local<W, 4>(a, s) : run_local<W, W <= 6 ? 5 : 4>(a, s);
+  if (rows <= 2) return run_local<W, 2, kLong>(a, s);
+  return rows <= 4 ? run_local<W, 4, kLong>(a, s) : run_local<W, W <= 6 ? 5 : 4, kLong>(a, s);
 }
 
 }  // namespace
@@ -256,18 +289,18 @@ int tsit5_run(Tsit5Loop& a, size_t words, uint64_t** grid, const fvm_ode_opts* o
 
 size_t tsit5_rows_grid_words(int64_t n) { return grid_words(n); }
 
-hipError_t tsit5_rows_fits(int64_t n, int W, bool* fits) {
-  return grid_fits(grid_kernel(W), kGridT, grid_wgs(n), fits);
+hipError_t tsit5_rows_fits(int64_t n, int W, bool long_rows, bool* fits) {
+  return grid_fits(grid_kernel(W, long_rows), kGridT, grid_wgs(n), fits);
 }
 
 hipError_t tsit5_rows(SmallTsit5& a, bool local, hipStream_t s) {
   if (!local) {
     void* args[] = {&a};
-    return hipLaunchCooperativeKernel(grid_kernel(a.W), dim3((unsigned)grid_wgs(a.n)), dim3(kGridT), args, 0, s);
+    return hipLaunchCooperativeKernel(grid_kernel(a.W, a.long_rows), dim3((unsigned)grid_wgs(a.n)), dim3(kGridT), args, 0, s);
   }
-  if (a.W <= 6) return run<6>(a, s);
-  if (a.W <= 8) return run<8>(a, s);
-  return run<10>(a, s);
+  if (a.W <= 6) return run<6, false>(a, s);
+  if (a.W <= 8) return run<8, false>(a, s);
+  return a.long_rows ? run<kTsit5MaxW, true>(a, s) : run<kTsit5MaxW, false>(a, s);
 }
 
 }  // namespace fvm

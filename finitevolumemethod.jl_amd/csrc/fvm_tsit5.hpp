@@ -41,16 +41,18 @@ struct SmallTsit5 : Tsit5Loop {
   const double* eval;
   const double* diag;
   const double* b;
+  bool long_rows;    // some rows have more than W entries off the diagonal
   uint64_t* grid;    // the grid form's exchange memory, zeroed
 };
 
+constexpr int kTsit5MaxW = 10;            // unrolled slots of the operators, at most
 constexpr int64_t kTsit5GridMax = 65536;  // rows of the grid form (256 workgroups of 256)
 // rows of the one-workgroup form for an ELL width, at most
 int64_t tsit5_rows_local_max(int W);
 // 8-byte words of exchange memory of the grid form
 size_t tsit5_rows_grid_words(int64_t n);
 // whether the device holds the grid form's workgroups at once
-hipError_t tsit5_rows_fits(int64_t n, int W, bool* fits);
+hipError_t tsit5_rows_fits(int64_t n, int W, bool long_rows, bool* fits);
 hipError_t tsit5_rows(SmallTsit5& a, bool local, hipStream_t s);
 
 }  // namespace fvm

@@ -115,17 +115,22 @@ def test_a_failed_gmres_leaves_no_stale_solution(gpu, shape):
 
 
 @pytest.mark.parametrize("shape", [(3, 3), (16, 16), (32, 32), (64, 40), (13, 197), (45, 46, 0.25), (64, 32, 0.25),
-                                   (90, 80, 0.25), (256, 256), (200, 190, "permuted"), "wheel"], ids=str)
+                                   (90, 80, 0.25), (256, 256), (200, 190, "permuted"), "wheel", ("hub", 11, 3),
+                                   ("hub", 18, 40), ("hub", 19, 140), ("hub", 300, 2), ("hub", 300, 12)], ids=str)
 def test_one_launch_tsit5_is_the_host_loop_bit_for_bit(gpu, shape):
     """A small ODE template's whole Tsit5 loop in one launch: one workgroup up to the rows
     its registers hold (2,560 with up to 6 off-diagonals a row, 2,048 with more), a resident
-    grid up to 65,536, 16- and 32-bit columns, a hub's row of 40: every saved state, time
-    and counter equals the multi-kernel arithmetic of the host loop."""
+    grid up to 65,536, 16- and 32-bit columns, a hub's row of 11 to 300 (one, eight, nine and
+    many entries beyond the ten slots) in either: every saved state, time and counter equals
+    the multi-kernel arithmetic of the host loop."""
     from finitevolumemethod.solve import integrate
+    from test_gpu_amg import _hub
     from test_gpu_templates import _permuted
 
     if shape == "wheel":
         tri = wheel_triangulation()
+    elif shape[0] == "hub":
+        tri = _hub(*shape[1:])
     elif len(shape) == 2:
         tri = FVM.triangulate_rectangle(0.0, 1.0, 0.0, 1.0, *shape, single_boundary=True)
     else:
