@@ -164,9 +164,17 @@ __global__ __launch_bounds__(kT) void tsit5_mesh_kernel(MeshTsit5 a) {
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) sum.add(j < deg, e2[j / 2] >> (16 * (j & 1)) & 0x8000, qa[j], qb[j]);
-    for (int j = 8; j < deg; ++j) {
-      const int e = a.m.rest[rest + j - 8];
-      sum.add(true, e & 0x8000, S.q[e & 0x7fff], S.q[(e & 0x7fff) + kRow]);
+    for (int j0 = 8; j0 < deg; j0 += 8) {  // a hub's others, eight loads in flight
+      int e[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) e[j] = j0 + j < deg ? a.m.rest[rest + j0 + j - 8] : 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        qa[j] = S.q[e[j] & 0x7fff];
+        qb[j] = S.q[(e[j] & 0x7fff) + kRow];
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sum.add(j0 + j < deg, e[j] & 0x8000, qa[j], qb[j]);
     }
     double acc = sum.value();
     for (int j = 0; j < (bit & 255); ++j) acc = acc - S.b[(bit >> 8) + j];

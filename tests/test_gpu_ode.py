@@ -13,6 +13,7 @@ from finitevolumemethod import _lib
 from finitevolumemethod.solve import fsal_ok, integrate
 from problems import (annulus_problem, brusselator_system, dxy_problem, heat_convection_problem, mixed_problem,
                       nodal_problem, nonlinear_problem)
+from test_gpu_amg import _hub
 from test_gpu_linear_flux import CASES as LINEAR_CASES, problem as linear_problem
 from test_gpu_power_law import power_problem
 from test_gpu_rhs import _fan
@@ -109,6 +110,15 @@ def shuffled_problem():
                           final_time=1.0)
 
 
+def hub_problem(d):
+    """A hub of d triangles inside two rings of d nodes (several blocks)."""
+    tri = _hub(d, 2)
+    mesh = FVM.FVMGeometry(tri)
+    return FVM.FVMProblem(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.3 + 0.0 * u, FVM.Neumann),
+                          diffusion_function=lambda x, y, t, u, p: 0.1 + u ** 2,
+                          initial_condition=np.random.default_rng(d).random(len(tri.x)), final_time=d ** -3.0)
+
+
 def fan_problem(d, closed):
     mesh = FVM.FVMGeometry(_fan(d, closed))
     BCs = FVM.BoundaryConditions(mesh, (lambda x, y, t, u, p: 0.3 + 0.0 * u, lambda x, y, t, u, p: 0.5 * u),
@@ -123,12 +133,13 @@ def fan_problem(d, closed):
     lambda: nonlinear_problem(255, 257)[0], lambda: nonlinear_problem(257, 256)[0], lambda: nodal_problem(33, 31)[0],
     lambda: dxy_problem(30)[0], lambda: linear_problem(*LINEAR_CASES["anisotropic"])[0],
     lambda: power_problem()[0], lambda: heat_convection_problem(40)[0], lambda: fan_problem(40, True),
-    lambda: fan_problem(9, False), lambda: fan_problem(600, True), shuffled_problem],
+    lambda: fan_problem(9, False), lambda: fan_problem(17, True), lambda: hub_problem(200),
+    lambda: fan_problem(600, True), shuffled_problem],
     ids=["tiny", "one_block", "strip", "most_blocks", "over_them", "nodal", "edge", "linear", "power", "neumann", "hub",
-         "boundary_hub", "wide_hub", "shuffled"])
+         "boundary_hub", "hub_17", "widest_hub", "wide_hub", "shuffled"])
 def test_tsit5_on_resident_blocks_matches_host_loop(gpu, build):
     """One block of 256 nodes, several, the most, and meshes that keep the multi-kernel
-    loop (more nodes, a hub beyond a block's triangles); every flux kind."""
+    loop (more nodes, a hub of more than 200 triangles); every flux kind."""
     prob = build()
     cv = prob.mesh.cv_volumes
     t0, h2 = prob.initial_time, cv[cv > 0].min()
@@ -141,8 +152,8 @@ def test_tsit5_on_resident_blocks_matches_host_loop(gpu, build):
 @pytest.mark.parametrize("build,blocks", [
     (lambda: nonlinear_problem(4, 3)[0], 1), (lambda: nonlinear_problem(16, 16)[0], 1),
     (lambda: nonlinear_problem(255, 257)[0], 256), (lambda: nonlinear_problem(257, 256)[0], 0),
-    (lambda: fan_problem(40, True), 1), (lambda: fan_problem(600, True), 0), (lambda: fan_problem(5000, True), 0),
-    (shuffled_problem, 4)], ids=["tiny", "one_block", "most_blocks", "over_them", "hub", "wide_hub", "wider_hub", "shuffled"])
+    (lambda: hub_problem(200), 2), (lambda: hub_problem(201), 0), (lambda: fan_problem(129, True), 0), (lambda: fan_problem(5000, True), 0),
+    (shuffled_problem, 4)], ids=["tiny", "one_block", "most_blocks", "over_them", "widest_hub", "wide_hub", "items", "wider_hub", "shuffled"])
 def test_blocks_are_made_by_the_first_solve_that_uses_them(gpu, build, blocks):
     """Not with the mesh or a right-hand side; none where a block does not fit (what the lists
     hold is held by the solves above, bit for bit)."""
