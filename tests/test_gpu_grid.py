@@ -1,6 +1,6 @@
 """The kernels whose workgroups exchange data without leaving the kernel (fvm_grid.hpp),
 at the sizes where their layout changes: one workgroup, whole and ragged last
-workgroups, 256- and 512-row workgroups, rows wider than the unrolled widths.
+workgroups, rows wider than the unrolled widths.
 
 fvm_trbdf2_affine against the host integrator on the same problem, both with Newton
 stopped at 1e-7 and GMRES at 1e-9 of their scales: the two then take the same steps and
@@ -79,6 +79,47 @@ def test_nonlinear_trbdf2_with_a_frozen_jacobian_matches_the_matrix_free_loop(gp
         assert np.max(np.abs(x - y)) <= 1e-7 * np.max(np.abs(y))
 
 
+@pytest.mark.parametrize("case", ["outside", "callback", "dirichlet"])
+def test_frozen_jacobian_over_free_points_and_callbacks(gpu, case):
+    """Points that are no vertices (rows of the diagonal alone), a user callback that changes u
+    after every step, Dirichlet values that depend on t: J is taken where the step starts."""
+    from finitevolumemethod import implicit
+
+    base = FVM.jittered_rectangle(0.0, 1.0, 0.0, 1.0, 23, 19, jitter=0.2, seed=3, single_boundary=False)
+    x, y, tri = base.x, base.y, base
+    if case == "outside":
+        new = np.random.default_rng(8).permutation(len(x) + 3)
+        x, y = np.full(len(new), 0.5), np.full(len(new), 0.5)
+        x[new[:-3]], y[new[:-3]] = base.x, base.y
+        tri = FVM.Triangulation(x, y, new[base.triangles], new[base.boundary_edges], base.boundary_segments)
+    mesh = FVM.FVMGeometry(tri)
+    hold = FVM.Dirichlet if case == "dirichlet" else FVM.Neumann
+    prob = FVM.FVMProblem(mesh, FVM.BoundaryConditions(mesh, (lambda x, y, t, u, p: 0.5 + 0.3 * t + 0.0 * u,) * 4,
+                                                       (hold, FVM.Neumann) * 2),
+                          diffusion_function=lambda x, y, t, u, p: 0.1 + u ** 2,
+                          source_function=lambda x, y, t, u, p: u * (1 - u),
+                          initial_condition=0.5 + 0.4 * np.sin(5 * x) * np.cos(4 * y), final_time=0.02)
+    J = implicit.FrozenJacobian.of(prob)
+    assert J is not None and (J.op.width > 0)
+    calls = []
+
+    def callback(u, t):
+        calls.append(t)
+        u.upload(0.97 * u.to_host())
+
+    kw = dict(saveat=[0.01, 0.02], callback=callback if case == "callback" else None)
+    opts = dict(newton_kappa=1e-7, krylov_rtol=1e-9)
+    a = FVM.solve(prob, FVM.TRBDF2(**opts), **kw)
+    seen, calls[:] = list(calls), []
+    b = FVM.solve(prob, FVM.TRBDF2(device_loop=False, **opts), **kw)
+    assert a.retcode == b.retcode == "Success" and a.stats["naccept"] == b.stats["naccept"] <= 50
+    # times of steps agree to the controller's amplification of the states' differences
+    assert len(seen) == len(calls) == (a.stats["naccept"] if case == "callback" else 0)
+    np.testing.assert_allclose(seen, calls, rtol=1e-5)
+    for p, q in zip(a.u, b.u):
+        assert np.max(np.abs(p - q)) <= 1e-7 * np.max(np.abs(q))
+
+
 def _frozen(nx, ny):
     from finitevolumemethod import implicit
 
@@ -114,15 +155,18 @@ def test_a_failed_gmres_leaves_no_stale_solution(gpu, shape):
         J.iterations()
 
 
+@pytest.mark.parametrize("sides", ["neumann", "dirichlet"])
 @pytest.mark.parametrize("shape", [(3, 3), (16, 16), (32, 32), (64, 40), (13, 197), (45, 46, 0.25), (64, 32, 0.25),
                                    (90, 80, 0.25), (256, 256), (200, 190, "permuted"), "wheel", ("hub", 11, 3),
                                    ("hub", 18, 40), ("hub", 19, 140), ("hub", 300, 2), ("hub", 300, 12)], ids=str)
-def test_one_launch_tsit5_is_the_host_loop_bit_for_bit(gpu, shape):
+def test_one_launch_tsit5_is_the_host_loop_bit_for_bit(gpu, shape, sides):
     """A small ODE template's whole Tsit5 loop in one launch: one workgroup up to the rows
     its registers hold (2,560 with up to 6 off-diagonals a row, 2,048 with more), a resident
     grid up to 65,536, 16- and 32-bit columns, a hub's row of 11 to 300 (one, eight, nine and
     many entries beyond the ten slots) in either: every saved state, time and counter equals
-    the multi-kernel arithmetic of the host loop."""
+    the multi-kernel arithmetic of the host loop.  Dirichlet rows have no flux but keep their
+    neighbours as entries of zero: the grid form needs a symmetric pattern, or waves of such
+    rows alone (a side of a large rectangle) could run ahead of the others' reads."""
     from finitevolumemethod.solve import integrate
     from test_gpu_amg import _hub
     from test_gpu_templates import _permuted
@@ -140,9 +184,14 @@ def test_one_launch_tsit5_is_the_host_loop_bit_for_bit(gpu, shape):
     mesh = FVM.FVMGeometry(tri)
     n = tri.num_points()
     u0 = np.random.default_rng(n).random(n)
-    prob = FVM.DiffusionEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 1.5, FVM.Neumann),
+    bc = FVM.Neumann if sides == "neumann" else FVM.Dirichlet
+    prob = FVM.DiffusionEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 1.5, bc),
                                  diffusion_function=lambda x, y, p: 0.5 + x, initial_condition=u0,
                                  final_time=25.0 / n)
+    if sides == "dirichlet":  # the property itself, of the assembled operator
+        A = prob.A.copy()
+        A.data[:] = 1.0
+        assert np.all(np.diff(A.indptr) > 1) and (A != A.T).nnz == 0
     ts = [0.0, 7.0 / n, 25.0 / n]
     a = FVM.solve(prob, FVM.Tsit5(), saveat=ts)
     p = prob.problem
