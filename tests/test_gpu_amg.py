@@ -128,3 +128,17 @@ def test_a_source_of_one_mode_needs_no_cycle(gpu):
     assert a.retcode == "Success" and a.resid <= 1e-10 and a.iters <= 3
     # both residuals are below 1e-10 |b| and |A^-1| <= 1 / (2 pi^2) here, up to the grid's error
     assert np.linalg.norm(a.u - b.u) <= 2e-10 * np.linalg.norm(prob.b) / 19.0 + 1e-12 * np.linalg.norm(b.u)
+
+
+@pytest.mark.parametrize("nx,ny,cycle", [(1100, 3, False), (1100, 6, False), (1100, 7, True), (30000, 4, False)])
+def test_strips_within_two_edges_of_fixed_rows_need_no_cycle(gpu, nx, ny, cycle):
+    """Some twenty Jacobi-preconditioned iterations an edge of distance: CG() bit for bit,
+    without setting up the multigrid hierarchy."""
+    tri = FVM.jittered_rectangle(0.0, nx - 1.0, 0.0, ny - 1.0, nx, ny, jitter=0.25, seed=5, single_boundary=True)
+    mesh = FVM.FVMGeometry(tri)
+    prob = FVM.PoissonsEquation(mesh, FVM.BoundaryConditions(mesh, lambda x, y, t, u, p: 0.0 * x, FVM.Dirichlet),
+                                diffusion_function=lambda x, y, p: 1.0 + 0.0 * x, source_function=lambda x, y, p: p,
+                                source_parameters=np.random.default_rng(1).random(tri.num_points()))
+    a, b = FVM.solve(prob), FVM.solve(prob, CG())
+    assert a.retcode == b.retcode == "Success" and a.resid <= 1e-10
+    assert (a.iters < b.iters) == cycle and np.array_equal(a.u, b.u) != cycle, (a.stats, b.stats)
