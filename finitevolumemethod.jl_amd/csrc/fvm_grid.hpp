@@ -141,6 +141,9 @@ struct Grid {
   uint32_t vtag, rtag;
   GridShared<T>* sh;
 
+  // kAgain: memory that earlier kernels have used.  A fault of one of them stands: its exchange
+  // numbers are unknown, so every workgroup gives up after its first sum.
+  template <bool kAgain = false>
   __device__ __forceinline__ void open(uint64_t* m, int64_t n_, GridShared<T>* s) {
     mem = m;
     view = grid_view(m, grid_words(n_));
@@ -149,9 +152,7 @@ struct Grid {
     sh = s;
     vtag = __builtin_amdgcn_readfirstlane((uint32_t)m[kGridVec]);
     rtag = __builtin_amdgcn_readfirstlane((uint32_t)m[kGridSum]);
-    // a fault of an earlier kernel on this memory stands: its exchange numbers are unknown,
-    // so every workgroup gives up after its first sum
-    if (threadIdx.x == 0) s->fault = grid_fault(m) != 0;
+    if (threadIdx.x == 0) s->fault = kAgain ? grid_fault(m) != 0 : 0;
     __syncthreads();
   }
   // the numbers the next kernel on this memory starts from (every workgroup has read

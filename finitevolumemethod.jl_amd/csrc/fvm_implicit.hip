@@ -445,7 +445,7 @@ __global__ __launch_bounds__(T) void gmres_kernel(Gm p) {
   const int64_t i = (int64_t)blockIdx.x * T + threadIdx.x;
   const bool active = i < p.J.n;
   Grid<T> G;
-  G.open(p.grid, p.J.n, &S.grid);
+  G.template open<true>(p.grid, p.J.n, &S.grid);
   Row<W> R;
   R.load(p.J, i, active);
   const double di = p.a + p.bj * R.diag;  // the row's diagonal entry
