@@ -2,11 +2,10 @@
 // template operators, set up and applied on the device.
 //
 // Jacobi-preconditioned CG needs a number of iterations that grows like the side of the
-// mesh (254 on the 2,813-node exit time mesh, 3,800 on 1000 x 1000 jittered nodes); with
-// this preconditioner 21 and 44.  On 1000 x 1000 a solve takes 9.2 ms instead of 158, the
-// first one of a template 14.5 with the set-up (5 ms: half of it sorting and summing the
-// first level's lists, bound by the latency of its gathers); on the exit time mesh 1.05 ms
-// instead of 3.18, the first 1.6.
+// mesh: 3,800 on 1000 x 1000 jittered nodes, with this preconditioner 44 (and the three
+// Jacobi steps before it).  A solve there takes 9.2 ms instead of 158, the first one of a
+// template 14.5 with the set-up (5 ms: half of it sorting and summing the first level's
+// lists, bound by the latency of its gathers).
 //
 // Set-up, per level:
 //   weights   s_i = 1.8 / sum_j |a_ij|: Jacobi with 0.9 of the inverse diagonal on an
@@ -25,8 +24,9 @@
 // is, for symmetric A, x = S (2 b - A S b) + Q A_c^-1 Q^T b: one pass over Q^T on the way
 // down and one over A and Q on the way up, instead of two products with A, a restriction
 // and a prolongation.  Of an iteration's 200 us on 1000 x 1000, the first level's passes
-// take 100 (up 40, the product p.M p 30, down 19, update 12: 3 to 4 TB/s), the levels
-// below 60, the gaps between the 11 launches the rest.  Levels of at most kTailRows rows and the coarsest one's dense
+// take 100 (up 40, the product p.M p 30, down 19, update 12; by their counters 148, 94, 47
+// and 51 MB of HBM traffic: 3.7, 3.2, 2.4 and 4.5 TB/s), the levels below 65, the gaps
+// between the 11 launches the rest.  Levels of at most kTailRows rows and the coarsest one's dense
 // inverse run in one workgroup, in one launch: smaller launches cost 3 to 4 us each and
 // hold next to no work.
 #include "fvm_amg.hpp"
@@ -54,6 +54,7 @@ __device__ __forceinline__ int wave_max(int x) {
 inline dim3 grid1(int64_t n) { return dim3((unsigned)((n + kB - 1) / kB)); }
 __device__ __forceinline__ int64_t gid() { return (int64_t)blockIdx.x * blockDim.x + threadIdx.x; }
 
+// the integer mixer lowbias32 (C. Wellons, hash-prospector, 2018)
 __device__ __forceinline__ uint32_t hash32(uint32_t x) {
   x ^= x >> 16;
   x *= 0x7feb352du;
