@@ -91,31 +91,29 @@ class _EllSlots:
     off-diagonals of each row in CSR order, slot-major [W][n], the diagonal apart."""
 
     def __init__(self, rp, col, n):
-        rows = np.repeat(np.arange(n), np.diff(rp))
-        on = col == rows
-        if not np.all(np.bincount(rows[on], minlength=n) == 1):
+        self.n, self.col = n, col
+        self.off = col != np.repeat(np.arange(n, dtype=col.dtype), np.diff(rp))
+        deg = np.diff(rp) - 1
+        if len(col) - np.count_nonzero(self.off) != n or not np.array_equal(col[~self.off], np.arange(n)):
             raise ValueError("the pattern must hold every diagonal entry")
-        slot = np.arange(len(col)) - rp[rows]  # position in the row, diagonal included
-        dpos = np.zeros(n, np.int64)
-        dpos[rows[on]] = slot[on]
-        self.n, self.on, self.off = n, on, ~on
-        self.row = rows[self.off]
-        self.slot = (slot - (slot > dpos[rows]))[self.off]  # minus 1 after the diagonal
-        self.col = col[self.off]
-        self.W = int(np.bincount(self.row, minlength=n).max()) if n else 0
+        self.W = int(deg.max()) if n else 0
+        # entry k of the off-diagonals: slot k - (those of the rows before), at [slot n + row]
+        first = rp[:-1] - np.arange(n)
+        self.at = np.arange(len(col) - n) * n + np.repeat(np.arange(n) - first * n, deg)
 
     def diagonal(self, v):
-        return v[self.on].copy()
+        return v[~self.off]
 
     def columns(self):
         """The columns, padded with the row's own."""
-        ecol = np.repeat(np.arange(self.n, dtype=np.int32)[None, :], self.W, axis=0)
-        ecol[self.slot, self.row] = self.col
-        return ecol
+        e = np.tile(np.arange(self.n, dtype=np.int32), self.W)
+        e[self.at] = self.col[self.off]
+        return e
 
     def spread(self, v, pad):
-        e = np.full((self.W, self.n), pad, np.asarray(v).dtype)
-        e[self.slot, self.row] = v[self.off]
+        v = np.asarray(v)
+        e = np.full(self.W * self.n, pad, v.dtype)
+        e[self.at] = v[self.off]
         return e
 
 
@@ -147,8 +145,8 @@ class AffineOperator:
         slots = _EllSlots(rp, col, n)
         diag, ecol, eval_ = slots.diagonal(val), slots.columns(), slots.spread(val, 0.0)
         self.W = slots.W
-        self.d_col = _lib.DeviceArray.from_host(ecol.ravel(), np.int32)
-        self.d_val = _lib.DeviceArray.from_host(eval_.ravel())
+        self.d_col = _lib.DeviceArray.from_host(ecol, np.int32)
+        self.d_val = _lib.DeviceArray.from_host(eval_)
         self.d_diag = _lib.DeviceArray.from_host(diag)
         self.d_orp = _lib.DeviceArray.from_host(np.zeros(n + 1, np.int32), np.int32)
         self.d_c = f0
@@ -198,9 +196,9 @@ class FrozenJacobian:
             nc = int(colour.max()) + 1
             plan = prob._jacobian_plan = (nc, slots.W, None) if nc > cls.MAX_COLOURS or slots.W > cls.MAX_WIDTH else (
                 nc, slots.W, [_lib.DeviceArray.from_host((colour == c).astype(np.float64)) for c in range(nc)],
-                _lib.DeviceArray.from_host(np.concatenate([slots.spread(colour[col].astype(np.uint8), 255),
-                                                           colour.astype(np.uint8)[None, :]]).ravel(), np.uint8),
-                _lib.DeviceArray.from_host(slots.columns().ravel(), np.int32),
+                _lib.DeviceArray.from_host(np.concatenate([slots.spread(colour.astype(np.uint8)[col], 255),
+                                                           colour.astype(np.uint8)]), np.uint8),
+                _lib.DeviceArray.from_host(slots.columns(), np.int32),
                 _lib.DeviceArray.from_host(np.zeros(n + 1, np.int32), np.int32))
         return cls(prob, plan) if plan[2] is not None else None
 

@@ -380,3 +380,31 @@ def test_distance_two_colouring_separates_columns_of_every_row():
             assert len(np.unique(cs)) == len(cs), i
     with pytest.raises(ValueError):
         _colouring(np.array([0, 2, 3]), np.array([0, 5, 1], np.int32), 2)
+
+
+@pytest.mark.parametrize("case", ["single", "diagonal", "first", "random"])
+def test_ell_slots_are_the_rows_off_diagonals_in_order(case):
+    """Against a loop over the rows: one row, rows of the diagonal alone, the diagonal first or
+    last in its row, rows of 1 to n entries; a missing diagonal raises."""
+    from finitevolumemethod.implicit import _EllSlots
+
+    rng = np.random.default_rng(4)
+    n = 1 if case == "single" else 9
+    keep = {"single": np.ones((1, 1)), "diagonal": np.eye(n), "first": np.eye(n) + np.triu(rng.random((n, n)) < 0.5, 1),
+            "random": np.eye(n) + (rng.random((n, n)) < 0.4)}[case] > 0
+    keep[0] = True  # a full row
+    col = np.concatenate([np.flatnonzero(r) for r in keep]).astype(np.int32)
+    rp = np.concatenate([[0], np.cumsum(keep.sum(1))]).astype(np.int64)
+    s = _EllSlots(rp, col, n)
+    v = rng.random(len(col))
+    W = max(keep.sum(1)) - 1
+    cols, vals = np.tile(np.arange(n), (W, 1)), np.full((W, n), -7.0)
+    for i in range(n):
+        off = [k for k in range(rp[i], rp[i + 1]) if col[k] != i]
+        cols[:len(off), i], vals[:len(off), i] = col[off], v[off]
+    assert s.W == W and np.array_equal(s.columns(), cols.ravel()) and s.columns().dtype == np.int32
+    assert np.array_equal(s.spread(v, -7.0), vals.ravel())
+    assert np.array_equal(s.diagonal(v), [v[rp[i] + list(col[rp[i]:rp[i + 1]]).index(i)] for i in range(n)])
+    if n > 1:
+        with pytest.raises(ValueError, match="diagonal"):
+            _EllSlots(np.array([0, 2, 3]), np.array([0, 1, 0], np.int32), 2)
