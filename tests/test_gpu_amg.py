@@ -70,6 +70,8 @@ def test_default_steady_solve_matches_a_direct_solution(gpu, kind, D):
     assert np.linalg.norm(a.u - x) <= bound + 1e-12 * np.linalg.norm(x)
     if len(b) > 3072:  # the cycle met the target, not the Jacobi-preconditioned CG behind it
         assert FVM.solve(prob, CG(), maxiter=2 * a.iters).retcode == "MaxIters", a.stats
+    if kind == (200, 170):
+        assert a.iters <= 60, a.stats  # Jacobi-preconditioned CG takes hundreds
     assert np.array_equal(FVM.solve(prob, maxiter=1000).u, a.u)
 
 
